@@ -180,6 +180,21 @@ int gpic_fp8_swiglu_bwd_t(const uint16_t *z, const uint16_t *da, int64_t M, int6
                           void *stream);
 
 /*
+ * The SwiGLU backward without a cast: dz [M, 2H] bf16 (contiguous) from z [M, 2H] (row stride sz) and da [M, H] (row
+ * stride sda), the values gpic_fp8_swiglu_bwd writes. For a caller whose backward GEMMs are bf16: the elementwise
+ * torch expressions of _SwiGLUw3.backward (fp8_native.py:226-231) as one pass. H % 8 == 0, sz, sda % 8 == 0, 16-byte
+ * aligned pointers.
+ */
+int gpic_fp8_swiglu_dz(const uint16_t *z, const uint16_t *da, int64_t M, int64_t H, int64_t sz, int64_t sda,
+                       uint16_t *dz, void *stream);
+
+/*
+ * y = bf16(fp32(q) * s), n e4m3 bytes: (aq.to(float32) * sa).to(bfloat16), the bf16 wgrad's operand
+ * (fp8_native.py:225, 265), as one pass. s: device fp32 scalar; q and y 16-byte aligned.
+ */
+int gpic_fp8_dequant(const uint8_t *q, const float *s, int64_t n, uint16_t *y, void *stream);
+
+/*
  * The norm sites' producer with the cast of its output folded in. Replaces gpic::res_mod_rmsnorm_fwd
  * (baselines/PixelGen/src/models/layers/fused_norm.py:150-175, kernel :64-91) followed by the FP8 linear's tcast of
  * its output h (fp8_native.py:114-122), as one producer (the reference keeps them apart, fp8_native.py:3-6):

@@ -684,6 +684,89 @@ __global__ __launch_bounds__(kCastThreads) void swiglu_bwd_cast_kernel(const uin
     }
 }
 
+// ------------------------------------------------------------------------------------------- bf16 backward
+//
+// The elementwise work of the recipes whose backward GEMMs are bf16 ("native", "native2"): dz without a cast and the
+// dequantized SwiGLU product, each in one pass. Both are bound by HBM: for H = 3072 and 32768 rows dz takes 171 us
+// (960 MiB, 5.9 TB/s) and the product 54 us (288 MiB, 5.6 TB/s). As separate torch operations the dz expression's passes
+// over fp32 intermediates took 2.5 ms and the product's three 0.36 ms; the d10 MLP's step went from 4.38 to 1.76 ms.
+
+// dz [M, 2H] (contiguous) = dz_words of z and da. Unit i (8 columns of each half of row i / (H / 8)) to thread i %
+// 512 of a group of 512 units, workgroup b taking groups b, b + G, ...; kDzBatch units' loads in flight per thread.
+// 24 KiB of LDS (the sigmoid table) and 512 threads: 4 workgroups a CU, each building its table once.
+constexpr int kDzThreads = 512, kDzBatch = 2;
+constexpr int kDzBlocks = 1024;
+__global__ __launch_bounds__(kDzThreads) void swiglu_dz_kernel(const uint16_t *__restrict__ z,
+                                                               const uint16_t *__restrict__ da, int64_t nu, int64_t H,
+                                                               int64_t sz, int64_t sda, uint16_t *__restrict__ dz) {
+  __shared__ float lut[kLutLds];
+  lut_build(lut);
+  const int64_t units = H / 8, step = (int64_t)gridDim.x * kDzThreads;
+  const int64_t dq = step / units, dr = step % units;
+  int64_t i = (int64_t)blockIdx.x * kDzThreads + threadIdx.x, r = i / units, u = i % units;
+  auto ld = [](const uint16_t *p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p)); };
+  for (; i < nu; i += kDzBatch * step) {
+    u32x4 Z1[kDzBatch], Z2[kDzBatch], D[kDzBatch];
+    uint16_t *o[kDzBatch];
+#pragma unroll
+    for (int k = 0; k < kDzBatch; k++) {
+      const bool ok = i + k * step < nu;   // (a unit past the end reads unit 0 and is not stored)
+      const uint16_t *zr = ok ? z + r * sz + 8 * u : z;
+      Z1[k] = ld(zr);
+      Z2[k] = ld(zr + H);
+      D[k] = ld(ok ? da + r * sda + 8 * u : da);
+      o[k] = ok ? dz + r * 2 * H + 8 * u : nullptr;
+      r += dq;
+      u += dr;
+      if (u >= units) {
+        u -= units;
+        r++;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kDzBatch; k++) {
+      u32x4 h1, h2;
+      dz_words(lut, Z1[k], Z2[k], D[k], h1, h2);
+      if (o[k]) {
+        *reinterpret_cast<u32x4 *>(o[k]) = h1;
+        *reinterpret_cast<u32x4 *>(o[k] + H) = h2;
+      }
+    }
+  }
+}
+
+// y = bf16(fp32(q) * s) for n e4m3 bytes: 16 bytes a thread and step, kUnroll steps' loads in flight; the n % 16 tail
+// by the first threads of workgroup 0.
+__device__ __forceinline__ u32x2 dequant4(uint32_t w, float s) {
+  const f32x2_t a = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, false), b = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, true);
+  return u32x2{pack_bf16(a.x * s, a.y * s), pack_bf16(b.x * s, b.y * s)};
+}
+__global__ __launch_bounds__(kCastThreads) void dequant_kernel(const uint8_t *__restrict__ q, const float *__restrict__ sp,
+                                                               int64_t n, uint16_t *__restrict__ y) {
+  const float s = sp[0];
+  const int64_t units = n / 16, stride = (int64_t)gridDim.x * blockDim.x;
+  const u32x4 *qv = reinterpret_cast<const u32x4 *>(q);
+  u32x4 *yv = reinterpret_cast<u32x4 *>(y);
+  auto emit = [&](int64_t u, u32x4 w) {
+    const u32x2 a = dequant4(w.x, s), b = dequant4(w.y, s), c = dequant4(w.z, s), d = dequant4(w.w, s);
+    yv[2 * u] = u32x4{a.x, a.y, b.x, b.y};
+    yv[2 * u + 1] = u32x4{c.x, c.y, d.x, d.y};
+  };
+  int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  for (; u + (kUnroll - 1) * stride < units; u += kUnroll * stride) {
+    u32x4 w[kUnroll];
+#pragma unroll
+    for (int k = 0; k < kUnroll; k++) w[k] = __builtin_nontemporal_load(qv + u + k * stride);
+#pragma unroll
+    for (int k = 0; k < kUnroll; k++) emit(u + k * stride, w[k]);
+  }
+  for (; u < units; u += stride) emit(u, __builtin_nontemporal_load(qv + u));
+  if (blockIdx.x == 0 && threadIdx.x < (n & 15)) {
+    const int64_t i = units * 16 + threadIdx.x;
+    y[i] = (uint16_t)dequant4(q[i], s).x;
+  }
+}
+
 // ------------------------------------------------------------------------------------------- host side
 
 static inline int grid_for(int64_t units, int cap) {
@@ -2093,6 +2176,29 @@ int gpic_fp8_swiglu_bwd_t(const uint16_t *z, const uint16_t *da, int64_t M, int6
       !aligned16(ws))
     return GPIC_EALIGN;
   return swiglu_bwd_common(z, da, M, H, sz, sda, dz, dzq, dzqt, ldt, dequant, ws, (hipStream_t)stream);
+}
+
+int gpic_fp8_swiglu_dz(const uint16_t *z, const uint16_t *da, int64_t M, int64_t H, int64_t sz, int64_t sda,
+                       uint16_t *dz, void *stream) {
+  status_scope();
+  if (M < 0 || H < 0 || (M > 0 && H > 0 && (!z || !da || !dz))) return GPIC_EINVAL;
+  if (H % 8 != 0 || sz % 8 != 0 || sda % 8 != 0 || sz < 2 * H || sda < H) return GPIC_ESHAPE;
+  if (!aligned16(z) || !aligned16(da) || !aligned16(dz)) return GPIC_EALIGN;
+  if (M == 0 || H == 0) return GPIC_OK;
+  const int64_t nu = M * (H / 8);
+  const int grid = (int)std::min<int64_t>((nu + kDzThreads - 1) / kDzThreads, kDzBlocks);
+  swiglu_dz_kernel<<<grid, kDzThreads, 0, (hipStream_t)stream>>>(z, da, nu, H, sz, sda, dz);
+  return (int)hipGetLastError();
+}
+
+int gpic_fp8_dequant(const uint8_t *q, const float *s, int64_t n, uint16_t *y, void *stream) {
+  status_scope();
+  if (n < 0 || !s || (n > 0 && (!q || !y))) return GPIC_EINVAL;
+  if (!aligned16(q) || !aligned16(y)) return GPIC_EALIGN;
+  if (n == 0) return GPIC_OK;
+  const int grid = grid_for((n / 16 + kUnroll - 1) / kUnroll, kMaxCastBlocks);
+  dequant_kernel<<<grid, kCastThreads, 0, (hipStream_t)stream>>>(q, s, n, y);
+  return (int)hipGetLastError();
 }
 
 }  // extern "C"

@@ -345,6 +345,41 @@ def _(z, da, want_dz=True):
             z.new_empty(1, dtype=torch.float32))
 
 
+@L.custom_op("gpic::fp8_swiglu_dz")
+def swiglu_dz(z: torch.Tensor, da: torch.Tensor) -> torch.Tensor:
+    """z [M, 2H] bf16, da [M, H] bf16 -> dz [M, 2H] bf16, swiglu_bwd's dz without its cast: the SwiGLU backward of the
+    bf16 recipes (fp8_native.py:226-231) in one pass."""
+    zc, dac = _bwd_prep(z, da)
+    M, H2 = zc.shape
+    dz = torch.empty(M, H2, dtype=torch.bfloat16, device=z.device)
+    with L.on_device(z.device):
+        L.check(L.lib().gpic_fp8_swiglu_dz(zc.data_ptr(), dac.data_ptr(), M, H2 // 2, zc.stride(0), dac.stride(0),
+                                           dz.data_ptr(), L.stream_ptr(z.device)), "gpic_fp8_swiglu_dz")
+    return dz
+
+
+@swiglu_dz.register_fake
+def _(z, da):
+    return z.new_empty(z.shape)
+
+
+@L.custom_op("gpic::fp8_dequant")
+def dequant(q: torch.Tensor, s: torch.Tensor) -> torch.Tensor:
+    """(q.to(float32) * s).to(bfloat16) for e4m3 q and its scale s [1] fp32, in one pass."""
+    L.require_gpu(q, s)
+    qc = L.aligned(q.contiguous())
+    y = torch.empty(q.shape, dtype=torch.bfloat16, device=q.device)
+    with L.on_device(q.device):
+        L.check(L.lib().gpic_fp8_dequant(qc.data_ptr(), s.data_ptr(), qc.numel(), y.data_ptr(),
+                                         L.stream_ptr(q.device)), "gpic_fp8_dequant")
+    return y
+
+
+@dequant.register_fake
+def _(q, s):
+    return q.new_empty(q.shape, dtype=torch.bfloat16)
+
+
 # ------------------------------------------------------------------------------------------------ GEMM
 
 def _gemm_operand(t, name):
@@ -555,7 +590,10 @@ class _SwiGLUw3(torch.autograd.Function):
         z, aq, sa, w3 = ctx.saved_tensors
         dy2 = dy.reshape(-1, dy.shape[-1]).to(torch.bfloat16)
         da = dy2 @ w3.to(torch.bfloat16)
-        dw3 = (dy2.t() @ (aq.to(torch.float32) * sa).to(torch.bfloat16)).to(ctx.wdt)
+        dw3 = (dy2.t() @ L.call(dequant, aq, sa)).to(ctx.wdt)
+        if not torch.is_grad_enabled() or torch.compiler.is_compiling():
+            return L.call(swiglu_dz, z, da).view(ctx.shape), dw3
+        # a backward that is itself recorded (create_graph): the same expression as torch operations
         z1, z2 = z.chunk(2, dim=-1)
         z1f = z1.float()
         sg = torch.sigmoid(z1f)
@@ -594,7 +632,7 @@ class _Fp8MLP(torch.autograd.Function):
         _, w12tq, s12t = L.call(tcast_t, w12, False)               # [C, 2H]
         dx = _mm(dzq, sdz, w12tq, s12t, fast=False)        # [M, C]
         dw12 = (dz.t() @ x2).to(ctx.dt[0])
-        dw3 = (dy2.t() @ (aq.to(torch.float32) * sa).to(torch.bfloat16)).to(ctx.dt[1])
+        dw3 = (dy2.t() @ L.call(dequant, aq, sa)).to(ctx.dt[1])
         return dx.view(ctx.shape), dw12, dw3
 
 
