@@ -73,16 +73,22 @@ def check(status, what):
         raise RuntimeError(f"{what} failed: {msg} (status {status})")
 
 
-_IMPL = {}   # custom op -> the function it was made from
+_IMPL = {}   # custom op -> the function it was made from: the package's public ops
+_STEP = {}   # the same for ops that only the path's own autograd Functions call
 
 
-def custom_op(name):
+def custom_op(name, impl=_IMPL):
     """torch.library.custom_op(name, mutates_args=()) that also keeps the function it wraps, for call()."""
     def deco(fn):
         op = torch.library.custom_op(name, mutates_args=())(fn)
-        _IMPL[op] = fn
+        impl[op] = fn
         return op
     return deco
+
+
+def step_op(name):
+    """custom_op for an op that only the path's own autograd Functions call."""
+    return custom_op(name, _STEP)
 
 
 def call(op, *args):
@@ -90,7 +96,7 @@ def call(op, *args):
     tracing the op's function runs directly, skipping the dispatcher (~10 us of host time per call, which bounds
     blocks of short kernels); under tracing the op itself, so a compiled graph holds the opaque custom op. Any other
     callable (a stand-in put in an op's place) is called as it is."""
-    fn = None if torch.compiler.is_compiling() else _IMPL.get(op)
+    fn = None if torch.compiler.is_compiling() else _IMPL.get(op) or _STEP.get(op)
     return fn(*args) if fn is not None else op(*args)
 
 

@@ -345,7 +345,7 @@ def _(z, da, want_dz=True):
             z.new_empty(1, dtype=torch.float32))
 
 
-@L.custom_op("gpic::fp8_swiglu_dz")
+@L.step_op("gpic::fp8_swiglu_dz")
 def swiglu_dz(z: torch.Tensor, da: torch.Tensor) -> torch.Tensor:
     """z [M, 2H] bf16, da [M, H] bf16 -> dz [M, 2H] bf16, swiglu_bwd's dz without its cast: the SwiGLU backward of the
     bf16 recipes (fp8_native.py:226-231) in one pass."""
@@ -363,7 +363,7 @@ def _(z, da):
     return z.new_empty(z.shape)
 
 
-@L.custom_op("gpic::fp8_dequant")
+@L.step_op("gpic::fp8_dequant")
 def dequant(q: torch.Tensor, s: torch.Tensor) -> torch.Tensor:
     """(q.to(float32) * s).to(bfloat16) for e4m3 q and its scale s [1] fp32, in one pass."""
     L.require_gpu(q, s)
