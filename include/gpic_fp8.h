@@ -270,6 +270,25 @@ int gpic_fp8_gemm_mn(const uint8_t *A, int64_t lda, const float *sa, const uint8
                      const uint16_t *bias, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K, void *ws,
                      size_t ws_bytes, void *stream);
 
+/*
+ * gpic_fp8_gemm_mn whose C is fp32 and holds the bf16-rounded results: the gradient of an fp32 weight, `.to(wdt)` of
+ * fp8_native.py:202, without a conversion pass. The same values as gpic_fp8_gemm_mn's, no bias; also ldc < 2^21.
+ */
+int gpic_fp8_gemm_mn_f32(const uint8_t *A, int64_t lda, const float *sa, const uint8_t *B, int64_t ldb,
+                         const float *sb, float *C, int64_t ldc, int64_t M, int64_t N, int64_t K, void *ws,
+                         size_t ws_bytes, void *stream);
+
+/*
+ * The bf16 weight gradient of the recipes "native" and "native2" (the reference's `dy.t() @ x`, fp8_native.py:202, 225,
+ * 264-265), fp32 accumulation, one bf16 rounding, deterministic:
+ *   C[m, n] = bf16(sum_k A[k, m] * B[k, n]);  A [K, M], B [K, N] bf16; C bf16, or fp32 with the bf16-rounded values
+ *   (c_dtype GPIC_DTYPE_*)
+ *   M, N % 16 == 0, any K; lda, ldb, ldc % 8 == 0; 2 K lda, 2 K ldb < 2^31; ldc < 2^22 (fp32: 2^21)
+ *   ws: gpic_fp8_gemm_workspace_bytes(M, N, 2 K) bytes.
+ */
+int gpic_fp8_bf16_gemm_mn(const uint16_t *A, int64_t lda, const uint16_t *B, int64_t ldb, void *C, int c_dtype,
+                          int64_t ldc, int64_t M, int64_t N, int64_t K, void *ws, size_t ws_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

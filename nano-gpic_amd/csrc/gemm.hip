@@ -35,6 +35,7 @@
 //  * Split-K (for the small-output wgrad shapes): each split writes fp32 partials; a second kernel sums them in
 //    split order (deterministic) and applies scale, bias and the bf16 rounding.
 #include <algorithm>
+#include <type_traits>
 
 #include "gpic_device.h"
 #include "gpic_launch.h"
@@ -42,8 +43,10 @@
 namespace gpic {
 
 typedef int v8i __attribute__((ext_vector_type(8)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
+typedef short v4s __attribute__((ext_vector_type(4)));
 // Types for the C staging block in LDS and the bf16 stores: may_alias, since LDS holding fragments of A and B as
 // one type is reused for C as another, and type-based alias analysis must not separate the two.
 typedef float f4a_t __attribute__((ext_vector_type(4), __may_alias__));
@@ -82,6 +85,10 @@ __device__ __forceinline__ int mn_swz(int r) { return ((r & 7) << 1) | ((r >> 5)
 // the 4 rows of each parity XOR the chunk with 4 different even masks, and the two groups 32 rows apart differ in
 // the lowest bit.
 __device__ __forceinline__ int mn_swz_n(int r) { return (((r >> 1) & 3) << 1) | ((r >> 5) & 1); }
+// bf16 MN-major K tiles (rows of 512 bytes, the narrow B's of 256): 16-byte chunk c of K row r lives in slot
+// c ^ mn_swz16(r). A half-wave of a transposing read takes the same two chunks of 4 consecutive rows and of 4 more
+// 8 rows on; the even masks send those 8 chunk pairs to 8 different 32-byte bank groups.
+__device__ __forceinline__ int mn_swz16(int r) { return ((r & 3) << 1) | (((r >> 3) & 1) << 3); }
 
 // The column of C that MFMA output row i of a pair of 16 x 16 tiles (i = 0..31: tile i / 16, row i % 16) stands for.
 // Lane l holds output rows 4 (l / 16) + v, v = 0..3, of each tile; through this map those of tiles 2p and 2p + 1 are
@@ -133,6 +140,11 @@ __device__ __forceinline__ int opaque_v(int v) {
   return v;
 }
 
+// Half h of a 32-byte fragment as a bf16 MFMA operand.
+__device__ __forceinline__ v8bf frag16(const v8i &f, int h) {
+  return __builtin_bit_cast(v8bf, v4i{f[4 * h], f[4 * h + 1], f[4 * h + 2], f[4 * h + 3]});
+}
+
 // Logical tile id for workgroup `bid` out of G: XCD x (= bid % 8) gets the contiguous range of ids
 // [start_x, start_x + count_x).
 __device__ __forceinline__ int xcd_remap(int bid, int G) {
@@ -146,14 +158,27 @@ __device__ __forceinline__ int xcd_remap(int bid, int G) {
 // the transposing ds_read_b64_tr_b8.
 // kBNt: the tile's width, 256 or 128 -- the narrow tile class for shapes whose 256 x 256 tiles leave CUs idle or end
 // on a partial round: each wave then owns 64 x 64 of C, a B K tile is 16 KiB (MN-major: 128 K rows x 128 bytes).
-template <bool kTail, bool kMN, int kBNt>
+// kEl: bytes of an operand element, 1 (e4m3) or 2 (bf16, kMN only: the bf16 wgrad of the recipes "native" and
+// "native2"). A bf16 K tile holds the same bytes, 64 K rows x 512 bytes, so loads, stages and phases are the e4m3 ones; it
+// is read with ds_read_b64_tr_b16, and a fragment's 32 bytes are the operands of two v_mfma_f32_16x16x32_bf16, half the
+// flops of the e4m3 instruction in the same cycles. lda and ldb are in bytes. No scales. Against the library's bf16
+// GEMM (dy^T @ x): [32768 tokens, 6144 x 768] 288-312 us against 418-428, [32768, 768 x 3072] 144 / 300, [32768,
+// 3072 x 1024] 176 / 303, [13303, 7168 x 896] 183-190 / 200, [13303, 896 x 3584] 101 / 138, [6592, 8192 x 1024] 102 / 102,
+// [512, 1024 x 1024] 15 / 18: never slower, so every wgrad takes it. (A bf16 dgrad with this kernel, its B read
+// MN-major, was not kept: 6-20% faster on some shapes, 14-25% slower on others, with no rule on sizes between them.)
+// kC32: C is fp32 and holds the bf16-rounded results: the gradient of an fp32 weight, without a separate conversion.
+template <bool kTail, bool kMN, int kBNt, int kEl = 1, bool kC32 = false, typename CT = std::conditional_t<kC32, float, uint16_t>>
 __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__restrict__ A, int lda,
                                                             const uint8_t *__restrict__ B, int ldb,
                                                             const float *__restrict__ sa, const float *__restrict__ sb,
-                                                            const uint16_t *__restrict__ bias, uint16_t *__restrict__ C,
+                                                            const uint16_t *__restrict__ bias, CT *__restrict__ C,
                                                             int64_t ldc, float *__restrict__ P, int M, int N, int K,
                                                             int ksplit, int tiles_m, int tiles_n, int splits) {
   static_assert(kBNt == 256 || kBNt == 128, "tile widths: 256 or 128");
+  static_assert(kMN || (kEl == 1 && !kC32), "bf16 operands and fp32 outputs: MN-major only");
+  constexpr int kKT = kBK / kEl;                  // K positions per K tile
+  constexpr int kRowA = kBM * kEl;                // MN-major: bytes of a K row of A's K tile
+  constexpr int kRowBK = kBNt * kEl;              // and of B's
   constexpr int kWTNt = kBNt / 2;                 // wave tile columns
   constexpr int kTNt = kWTNt / 16;                // 16-column MFMA tiles per wave: 8 or 4
   constexpr int kHalfB = kBNt * kBK;              // one B K tile: 32 or 16 KiB
@@ -179,19 +204,24 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
   // MN-major: instruction i of a wave fills K rows [R0, R0 + 4), R0 = (i * 4 + wave % 4) * 4 = 16 i + mrow - lane / 16;
   // lane j writes 16-byte slot j & 15 of row 16 i + mrow, i.e. MN chunk (j & 15) ^ mn_swz(row), and mn_swz depends on
   // row & 7 = mrow & 7 only.
-  const int mrow = (wave & 3) * 4 + (lane >> 4);
-  const int mchunk = (lane & 15) ^ mn_swz(mrow);   // for K rows with bit 5 clear (i & 2 == 0); else mchunk ^ 1
+  // bf16: rows of 512 bytes, an instruction fills rows [R0, R0 + 2), R0 = 2 (4 i + wave % 4) = 8 i + mrow - lane / 32;
+  // slot lane & 31, and mn_swz16 depends on mrow & 3 and on bit 3 of the row, i & 1.
+  const int mrow = kEl == 1 ? (wave & 3) * 4 + (lane >> 4) : (wave & 3) * 2 + (lane >> 5);
+  const int mchunk = kEl == 1 ? (lane & 15) ^ mn_swz(mrow)   // for K rows with bit 5 clear (i & 2 == 0); else mchunk ^ 1
+                              : (lane & 31) ^ mn_swz16(mrow);   // bit 3 clear (i & 1 == 0); else mchunk ^ 8
+  constexpr int kMFlip = kEl == 1 ? 1 : 8;
   // MN-major B of the narrow tile: instruction i fills K rows [R0, R0 + 8), R0 = (i * 4 + wave % 4) * 8 =
   // 32 i + mrowB - lane / 8; lane j writes slot j & 7 of row 32 i + mrowB, i.e. MN chunk (j & 7) ^ mn_swz_n(row), and
   // mn_swz_n depends on (row / 2) & 3 = (mrowB / 2) & 3 and on bit 5 of the row, i & 1.
-  const int mrowB = kBNt == 256 ? mrow : (wave & 3) * 8 + (lane >> 3);
-  const int mchunkB = kBNt == 256 ? mchunk : (lane & 7) ^ mn_swz_n(mrowB);
+  // bf16: rows of 256 bytes, R0 = 4 (4 i + wave % 4) = 16 i + mrowB - lane / 16: the swizzle does not depend on i.
+  const int mrowB = kBNt == 256 ? mrow : kEl == 1 ? (wave & 3) * 8 + (lane >> 3) : (wave & 3) * 4 + (lane >> 4);
+  const int mchunkB = kBNt == 256 ? mchunk : kEl == 1 ? (lane & 7) ^ mn_swz_n(mrowB) : (lane & 15) ^ mn_swz16(mrowB);
   const int baseA = kMN ? mrow * lda + 16 * mchunk : lrow * lda + kchunk;
   const int baseB = kMN ? mrowB * ldb + 16 * mchunkB : col_of(lrow) * ldb + kchunk;
   // MN-major: the same loads for K rows with bit 5 set, whose chunks are swizzled with one more bit
-  const int baseA1 = mrow * lda + 16 * (mchunk ^ 1);
-  const int baseB1 = mrowB * ldb + 16 * (mchunkB ^ 1);
-  const float s = sa[0] * sb[0];
+  const int baseA1 = mrow * lda + 16 * (mchunk ^ kMFlip);
+  const int baseB1 = mrowB * ldb + 16 * (mchunkB ^ kMFlip);
+  const float s = kEl == 1 ? sa[0] * sb[0] : 1.0f;
 
   // ---- persistent: work item `it` (a tile and a K split) goes to workgroup it % gridDim.x. The grid is a multiple
   // of 8 (or covers every item in one pass), so it & 7 is the XCD the workgroup runs on and xcd_remap gives each
@@ -216,14 +246,15 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
     w.n0 = ((tile % per_group) / gsz) * kBNt;
     w.kbeg = w.split * ksplit;
     w.kend = min(K, w.kbeg + ksplit);
-    w.nk = (w.kend - w.kbeg + kBK - 1) / kBK;
+    w.nk = (w.kend - w.kbeg + kKT - 1) / kKT;
     if constexpr (kMN) {   // descriptors from the item's first column to the end of the matrix (K x ld bytes)
-      w.rA = buffer_rsrc(A + w.m0, K * lda - w.m0);
-      w.rB = buffer_rsrc(B + w.n0, K * ldb - w.n0);
-      w.voA = w.m0 + 16 * mchunk < M ? baseA : kOOB;
-      w.voB = w.n0 + 16 * mchunkB < N ? baseB : kOOB;
-      w.voA1 = w.m0 + 16 * (mchunk ^ 1) < M ? baseA1 : kOOB;
-      w.voB1 = w.n0 + 16 * (mchunkB ^ 1) < N ? baseB1 : kOOB;
+      const int ma = w.m0 * kEl, nb = w.n0 * kEl;
+      w.rA = buffer_rsrc(A + ma, K * lda - ma);
+      w.rB = buffer_rsrc(B + nb, K * ldb - nb);
+      w.voA = ma + 16 * mchunk < M * kEl ? baseA : kOOB;
+      w.voB = nb + 16 * mchunkB < N * kEl ? baseB : kOOB;
+      w.voA1 = ma + 16 * (mchunk ^ kMFlip) < M * kEl ? baseA1 : kOOB;
+      w.voB1 = nb + 16 * (mchunkB ^ kMFlip) < N * kEl ? baseB1 : kOOB;
     } else {
       w.rA = buffer_rsrc(A + (int64_t)w.m0 * lda, min(M - w.m0, kBM) * lda);
       w.rB = buffer_rsrc(B + (int64_t)w.n0 * ldb, min(N - w.n0, kBNt) * ldb);
@@ -238,25 +269,29 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
   // kend read zeros.
   auto load = [&](const Item &w, bool isA, int dst, int k0, int i) {
     if constexpr (kMN && kBNt == 128) {
-      if (!isA) {   // the narrow B K tile: K rows k0 + 32 i + mrowB, 128 bytes each
-        const int R0 = (i * kLoaders + (wave & 3)) * 8;
-        const int vo = ((i & 1) ? w.voB1 : w.voB) + i * opaque(32 * ldb);   // (K row bit 5 = i & 1)
-        const uint32_t to = lds_addr(smem) + dst + R0 * 128;
-        if (!kTail || k0 + kBK <= w.kend) lds_dma16(w.rB, vo, k0 * ldb, to);
-        else lds_dma16(w.rB, k0 + 32 * i + mrowB < w.kend ? vo + k0 * ldb : kOOB, 0, to);
+      if (!isA) {   // the narrow B K tile: K rows k0 + 32 i + mrowB, 128 bytes each (bf16: 16 i, 256 bytes)
+        constexpr int kStep = kKT / kLoadsB;
+        const int R0 = (i * kLoaders + (wave & 3)) * (kStep / kLoaders);
+        const int vo = (kEl == 1 && (i & 1) ? w.voB1 : w.voB) + i * opaque(kStep * ldb);   // (K row bit 5 = i & 1)
+        const uint32_t to = lds_addr(smem) + dst + R0 * kRowBK;
+        if (!kTail || k0 + kKT <= w.kend) lds_dma16(w.rB, vo, k0 * ldb, to);
+        else lds_dma16(w.rB, k0 + kStep * i + mrowB < w.kend ? vo + k0 * ldb : kOOB, 0, to);
         return;
       }
     }
     if constexpr (kMN) {
       // K rows k0 + 16 i + mrow; the K position goes to the scalar offset (k0 * ld), the row within the tile and the
       // chunk to the lane's; lanes whose chunk lies past M / N start from kOOB
+      // (bf16: K rows k0 + 8 i + mrow of 512 bytes)
+      constexpr int kStep = kKT / kLoads;
       const int ld = isA ? lda : ldb;
-      const int R0 = (i * kLoaders + (wave & 3)) * 4;
+      const int R0 = (i * kLoaders + (wave & 3)) * (kStep / kLoaders);
+      const bool flip = kEl == 1 ? i & 2 : i & 1;   // the swizzle's row bit (5, bf16: 3)
       // (kOOB + these offsets stays in [2^31, 2^32): still past the range, which is below 2^31)
-      const int vo = ((i & 2) ? (isA ? w.voA1 : w.voB1) : (isA ? w.voA : w.voB)) + i * opaque(16 * ld);   // (bit 5 = i & 2)
-      const uint32_t to = lds_addr(smem) + dst + R0 * 256;
-      if (!kTail || k0 + kBK <= w.kend) lds_dma16(isA ? w.rA : w.rB, vo, k0 * ld, to);
-      else lds_dma16(isA ? w.rA : w.rB, k0 + 16 * i + mrow < w.kend ? vo + k0 * ld : kOOB, 0, to);
+      const int vo = (flip ? (isA ? w.voA1 : w.voB1) : (isA ? w.voA : w.voB)) + i * opaque(kStep * ld);
+      const uint32_t to = lds_addr(smem) + dst + R0 * kRowA;
+      if (!kTail || k0 + kKT <= w.kend) lds_dma16(isA ? w.rA : w.rB, vo, k0 * ld, to);
+      else lds_dma16(isA ? w.rA : w.rB, k0 + kStep * i + mrow < w.kend ? vo + k0 * ld : kOOB, 0, to);
     } else {
       const int R0 = (i * kLoaders + (wave & 3)) * 8;
       const int vo = isA ? baseA + i * opaque(32 * lda) : baseB + i * opaque(32 * ldb);
@@ -277,7 +312,7 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
     }
     if (w.nk > 1) {
 #pragma unroll
-      for (int i = 0; i < kLoads; i++) load(w, true, a_half(1), w.kbeg + kBK, i);
+      for (int i = 0; i < kLoads; i++) load(w, true, a_half(1), w.kbeg + kKT, i);
     }
   };
 
@@ -293,25 +328,35 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
   // index mnb + (l & 15) and K 32 (l / 16) + 8 q + [0, 8) in bytes 8 q .. 8 q + 7 of its operand -- the layout of the
   // K-major fragment. The chunk mnb / 16 of K row 32 g + 8 q + s / 2 sits in slot (mnb / 16) ^ mn_swz(row), and
   // mn_swz of those rows does not depend on q.
+  // bf16: ds_read_b64_tr_b16 takes 4 K rows x 16 columns per 16-lane group: source lane s reads 8 bytes of K row s / 4,
+  // columns 4 (s % 4) + [0, 4), and output lane j gets column j of the 4 rows. Read q = 0..3 of a fragment takes K rows
+  // 32 (q / 2) + 8 g + 4 (q % 2) + s / 4: lane l gets K 8 (l / 16) + [0, 8) of each half of the K tile, the operands
+  // of its two MFMAs. mn_swz16 of those rows does not depend on q.
   const int tr_g = lane >> 4, tr_s = lane & 15;
-  const int tr_row = 32 * tr_g + (tr_s >> 1);
-  const int tr_off = tr_row * 256 + 8 * (tr_s & 1);
-  const int tr_x = 16 * mn_swz(tr_row);
-  // (the narrow tile's B: rows of 128 bytes, chunk (mnb / 16) ^ mn_swz_n(row))
-  const int tr_offB = kBNt == 256 ? tr_off : tr_row * 128 + 8 * (tr_s & 1);
-  const int tr_xB = kBNt == 256 ? tr_x : 16 * mn_swz_n(tr_row);
+  const int tr_row = kEl == 1 ? 32 * tr_g + (tr_s >> 1) : 8 * tr_g + (tr_s >> 2);
+  const int tr_col = kEl == 1 ? 8 * (tr_s & 1) : 8 * (tr_s & 3);
+  const int tr_off = tr_row * kRowA + tr_col;
+  const int tr_x = 16 * (kEl == 1 ? mn_swz(tr_row) : mn_swz16(tr_row));
+  // (the narrow tile's B: rows of 128 bytes, chunk (mnb / 16) ^ mn_swz_n(row); bf16: of 256 bytes, the same swizzle)
+  const int tr_offB = kBNt == 256 ? tr_off : tr_row * kRowBK + tr_col;
+  const int tr_xB = kBNt == 256 || kEl == 2 ? tr_x : 16 * mn_swz_n(tr_row);
   auto read_frag = [&](int ast, int bst, int j) {
     const int f = j;
     if constexpr (kMN) {
-      const int mnb = f < kTM ? wm * kWTM + f * 16 : wn * kWTNt + (f - kTM) * 16;
-      const int rowb = f < kTM ? 256 : kBNt;   // bytes per K row of the operand's K tile
+      const int mnb = (f < kTM ? wm * kWTM + f * 16 : wn * kWTNt + (f - kTM) * 16) * kEl;   // (bytes)
+      const int rowb = f < kTM ? kRowA : kRowBK;   // bytes per K row of the operand's K tile
       const GPIC_LDS uint8_t *p =
           kBNt == 256 ? (const GPIC_LDS uint8_t *)smem + (f < kTM ? a_half(ast) : b_half(bst)) + tr_off + (mnb ^ tr_x)
                       : (const GPIC_LDS uint8_t *)smem +
                             (f < kTM ? a_half(ast) + tr_off + (mnb ^ tr_x) : b_half(bst) + tr_offB + (mnb ^ tr_xB));
       v2i r[4];
 #pragma unroll
-      for (int q = 0; q < 4; q++) r[q] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((GPIC_LDS v2i *)(p + q * 8 * rowb));
+      for (int q = 0; q < 4; q++) {
+        if constexpr (kEl == 1) r[q] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((GPIC_LDS v2i *)(p + q * 8 * rowb));
+        else
+          r[q] = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                             (GPIC_LDS v4s *)(p + (32 * (q >> 1) + 4 * (q & 1)) * rowb)));
+      }
       const v8i v{r[0].x, r[0].y, r[1].x, r[1].y, r[2].x, r[2].y, r[3].x, r[3].y};
       if (f < kTM) fa[f] = v;
       else fb[f - kTM] = v;
@@ -389,7 +434,8 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
       else asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
     }
   };
-  constexpr int kStoresBF16 = (kTM / 2) * (32 * kRowB / 1024);   // bf16 epilogue: 16 (narrow: 8) buffer stores per wave, always issued
+  // epilogue stores per wave, always issued: bf16 16 (narrow: 8), fp32 twice as many
+  constexpr int kStoresBF16 = (kTM / 2) * (32 * kRowB / 1024) * (kC32 ? 2 : 1);
   constexpr int kStoresF32 = kTNt * kTM;                         // split-K partials: 32 (narrow: 16)
 
   int it = blockIdx.x;
@@ -421,10 +467,10 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
       const int bst = kt & 1;
       // memory phase
       if (group == 0) {
-        mem_phase(cur, ast, bst, kt + 1 < cur.nk, false, b_half(bst ^ 1), cur.kbeg + (kt + 1) * kBK);
+        mem_phase(cur, ast, bst, kt + 1 < cur.nk, false, b_half(bst ^ 1), cur.kbeg + (kt + 1) * kKT);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // done reading the stages before anyone overwrites them
       } else {
-        mem_phase(cur, ast, bst, kt + 2 < cur.nk, true, a_half(ast == 0 ? 2 : ast - 1), cur.kbeg + (kt + 2) * kBK);
+        mem_phase(cur, ast, bst, kt + 2 < cur.nk, true, a_half(ast == 0 ? 2 : ast - 1), cur.kbeg + (kt + 2) * kKT);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (opaque(kt) > 0) {   // A(kt + 1) has landed (A(1) is group 0's, waited for by group 0); opaque: no peeled copy of the first iteration
           if (kt + 2 < cur.nk) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
@@ -436,8 +482,14 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
 #pragma unroll
       for (int ni = 0; ni < kTNt; ni++)
 #pragma unroll
-        for (int mi = 0; mi < kTM; mi++)
-          acc[ni][mi] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[ni], fa[mi], acc[ni][mi], 0, 0, 0, 0, 0, 0);
+        for (int mi = 0; mi < kTM; mi++) {
+          if constexpr (kEl == 1) {
+            acc[ni][mi] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[ni], fa[mi], acc[ni][mi], 0, 0, 0, 0, 0, 0);
+          } else {
+            acc[ni][mi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag16(fb[ni], 0), frag16(fa[mi], 0), acc[ni][mi], 0, 0, 0);
+            acc[ni][mi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag16(fb[ni], 1), frag16(fa[mi], 1), acc[ni][mi], 0, 0, 0);
+          }
+        }
       if (group == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // B(kt + 1) (and A(1)) have landed
       phase_barrier();
       ast = ast == 2 ? 0 : ast + 1;
@@ -484,13 +536,16 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
       GPIC_LDS uint8_t *cst =
           (GPIC_LDS uint8_t *)smem + (group == 0 ? a_half(2) : b_half(1)) + (wave & 3) * kCStage;
       const __amdgpu_buffer_rsrc_t rC =
-          __builtin_amdgcn_make_buffer_rsrc((void *)(C + (int64_t)cur.m0 * ldc), 0, rows_c * (int)ldc * 2, kBufferFlags);
-      constexpr int kLPR = kRowB / 16, kRPI = 64 / kLPR;   // read-back: lanes per row, rows per instruction
+          __builtin_amdgcn_make_buffer_rsrc((void *)(C + (int64_t)cur.m0 * ldc), 0, rows_c * (int)ldc * (int)sizeof(CT),
+                                            kBufferFlags);
+      constexpr int kCol = 16 / (int)sizeof(CT);               // columns of a 16-byte store: 8 (fp32: 4)
+      constexpr int kLPR = kWTNt / kCol, kRPI = 64 / kLPR;     // read-back: lanes per row, rows per instruction
+      typedef std::conditional_t<kC32, st8_t, st16_t> back_t;  // the bf16 of one store
       auto slot = [](int c, int r) { return kBNt == 256 ? c ^ (r & 15) : c ^ ((r >> 1) & 7); };
       const int rr = (unsigned)el / kLPR, rc = (unsigned)el % kLPR;   // read-back: rows kRPI j + rr, chunk rc
-      const int n = cur.n0 + wn * kWTNt + 8 * rc;   // the read-back lane's 8 columns
+      const int n = cur.n0 + wn * kWTNt + kCol * rc;   // the read-back lane's columns
       uint32_t b[4] = {0, 0, 0, 0};
-      if (bias && n < N) {
+      if (!kC32 && bias && n < N) {
         const u32x2 b0 = *reinterpret_cast<const u32x2 *>(bias + n), b1 = *reinterpret_cast<const u32x2 *>(bias + n + 4);
         b[0] = b0.x, b[1] = b0.y, b[2] = b1.x, b[3] = b1.y;
       }
@@ -521,26 +576,33 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the block is complete before any lane reads it back
         // all 8 rows read back first (their latencies overlap; a store between them would order them), then stored
-        constexpr int kNI = 32 / kRPI;   // read-back instructions per block: 8 (narrow: 4)
-        st16_t wv[kNI];
+        constexpr int kNI = 32 / kRPI;   // read-back instructions per block: 8 (narrow: 4; fp32: twice as many)
+        back_t wv[kNI];
 #pragma unroll
         for (int j = 0; j < kNI; j++) {
           const int r = kRPI * j + rr;
-          wv[j] = *(const GPIC_LDS st16_t *)(cst + r * kRowB + 16 * slot(rc, r));
+          if constexpr (kC32) wv[j] = *(const GPIC_LDS st8_t *)(cst + r * kRowB + 16 * slot(rc >> 1, r) + 8 * (rc & 1));
+          else wv[j] = *(const GPIC_LDS st16_t *)(cst + r * kRowB + 16 * slot(rc, r));
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // read back before the next block overwrites it
         const int rl0 = wm * kWTM + mq * 32 + rr;   // row within the tile of j = 0; row j is rl0 + kRPI j
-        int off = (rl0 * (int)ldc + n) * 2;
+        int off = (rl0 * (int)ldc + n) * (int)sizeof(CT);
 #pragma unroll
         for (int j = 0; j < kNI; j++) {
-          st16_t w = wv[j];
-          if (bias) {   // bf16(bf16(acc * s) + bias)
+          u32x4 o;
+          if constexpr (kC32) {
+            o = u32x4{wv[j].x << 16, wv[j].x & 0xffff0000u, wv[j].y << 16, wv[j].y & 0xffff0000u};
+          } else {
+            st16_t w = wv[j];
+            if (bias) {   // bf16(bf16(acc * s) + bias)
 #pragma unroll
-            for (int e = 0; e < 4; e++) w[e] = pack_bf16(bf16_lo(w[e]) + bf16_lo(b[e]), bf16_hi(w[e]) + bf16_hi(b[e]));
+              for (int e = 0; e < 4; e++)
+                w[e] = pack_bf16(bf16_lo(w[e]) + bf16_lo(b[e]), bf16_hi(w[e]) + bf16_hi(b[e]));
+            }
+            o = __builtin_bit_cast(u32x4, w);
           }
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, w), rC,
-                                                 rl0 + kRPI * j < rows_c && n < N ? off : kOOB, 0, kStoreNT);
-          off += 2 * kRPI * (int)ldc;
+          __builtin_amdgcn_raw_buffer_store_b128(o, rC, rl0 + kRPI * j < rows_c && n < N ? off : kOOB, 0, kStoreNT);
+          off += (int)sizeof(CT) * kRPI * (int)ldc;
         }
       }
       pend = kStoresBF16;
@@ -552,12 +614,14 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
 }
 
 // Sum of the split-K partials in split order, then the same epilogue as the single-pass kernel.
+// (sa, sb null: unscaled bf16 operands; CT float: the bf16-rounded results in fp32, no bias.)
+template <typename CT>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ P, int splits, int M, int N,
                                                             const float *__restrict__ sa, const float *__restrict__ sb,
-                                                            const uint16_t *__restrict__ bias, uint16_t *__restrict__ C,
+                                                            const uint16_t *__restrict__ bias, CT *__restrict__ C,
                                                             int64_t ldc) {
   const int64_t quads = (int64_t)M * (N / 4);
-  const float s = sa[0] * sb[0];
+  const float s = sa ? sa[0] * sb[0] : 1.0f;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < quads; i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t m = i / (N / 4);
     const int n = (int)(i % (N / 4)) * 4;
@@ -569,7 +633,9 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
       w.x = pack_bf16(bf16_lo(w.x) + bf16_lo(bw.x), bf16_hi(w.x) + bf16_hi(bw.x));
       w.y = pack_bf16(bf16_lo(w.y) + bf16_lo(bw.y), bf16_hi(w.y) + bf16_hi(bw.y));
     }
-    *reinterpret_cast<u32x2 *>(C + m * ldc + n) = w;
+    if constexpr (sizeof(CT) == 4)
+      *reinterpret_cast<u32x4 *>(C + m * ldc + n) = u32x4{w.x << 16, w.x & 0xffff0000u, w.y << 16, w.y & 0xffff0000u};
+    else *reinterpret_cast<u32x2 *>(C + m * ldc + n) = w;
   }
 }
 
@@ -636,15 +702,18 @@ static Plan plan_gemm(int64_t M, int64_t N, int64_t K) {
   return ktiles > 0 && tbest[1] < kNarrowGain * tbest[0] ? best[1] : best[0];
 }
 
-// The launch shared by both operand layouts (arguments checked by the entry points).
-template <bool kMN>
-static int launch_gemm(const uint8_t *A, int64_t lda, const float *sa, const uint8_t *B, int64_t ldb, const float *sb,
-                       const uint16_t *bias, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K, void *ws,
+// The launch shared by the operand layouts and types (arguments checked by the entry points; kEl and kC32 as the
+// kernel's). lda, ldb and K in elements.
+template <bool kMN, int kEl = 1, typename CT = uint16_t>
+static int launch_gemm(const void *A, int64_t lda, const float *sa, const void *B, int64_t ldb, const float *sb,
+                       const uint16_t *bias, CT *C, int64_t ldc, int64_t M, int64_t N, int64_t K, void *ws,
                        size_t ws_bytes, hipStream_t st) {
+  constexpr bool kC32 = sizeof(CT) == 4;
   if (M == 0 || N == 0) return GPIC_OK;
   if (K > 0 && (!A || !B)) return GPIC_EINVAL;
   if (!aligned16(A) || !aligned16(B) || !aligned16(C) || (bias && ((uintptr_t)bias & 7u))) return GPIC_EALIGN;
-  const Plan p = K > 0 ? plan_gemm(M, N, K) : Plan{(int)((M + kBM - 1) / kBM), (int)((N + kBN - 1) / kBN), 1, kBK, kBN};
+  // (a K tile is 128 bytes of each operand's K: the plan of a byte matrix kEl times as long)
+  Plan p = K > 0 ? plan_gemm(M, N, K * kEl) : Plan{(int)((M + kBM - 1) / kBM), (int)((N + kBN - 1) / kBN), 1, kBK, kBN};
   float *P = nullptr;
   if (p.splits > 1) {
     const size_t need = (size_t)p.splits * M * N * sizeof(float);
@@ -656,17 +725,18 @@ static int launch_gemm(const uint8_t *A, int64_t lda, const float *sa, const uin
   const int work = p.tiles_m * p.tiles_n * p.splits;
   const int slots = num_cus() & ~7;
   const int grid = work <= slots || slots < 8 ? work : slots;
+  p.ksplit /= kEl;   // in K positions
   // the partial-K-tile load path is compiled only into the instance that needs it
-  auto *kernel = p.bn == 128 ? (K % kBK ? gemm_tn_kernel<true, kMN, 128> : gemm_tn_kernel<false, kMN, 128>)
-                              : (K % kBK ? gemm_tn_kernel<true, kMN, 256> : gemm_tn_kernel<false, kMN, 256>);
+  auto *kernel = p.bn == 128 ? ((K * kEl) % kBK ? gemm_tn_kernel<true, kMN, 128, kEl, kC32> : gemm_tn_kernel<false, kMN, 128, kEl, kC32>)
+                              : ((K * kEl) % kBK ? gemm_tn_kernel<true, kMN, 256, kEl, kC32> : gemm_tn_kernel<false, kMN, 256, kEl, kC32>);
   kernel<<<grid, kThreads, 0, st>>>(
-      A, (int)lda, B, (int)ldb, sa, sb, bias, C, ldc, P, (int)M, (int)N, (int)K, p.ksplit, p.tiles_m, p.tiles_n,
-      p.splits);
+      static_cast<const uint8_t *>(A), (int)lda * kEl, static_cast<const uint8_t *>(B), (int)ldb * kEl, sa, sb, bias, C,
+      ldc, P, (int)M, (int)N, (int)K, p.ksplit, p.tiles_m, p.tiles_n, p.splits);
   if (P) {
     const int64_t quads = M * (N / 4);
     int64_t g = (quads + 255) / 256;
     if (g > 8192) g = 8192;
-    splitk_reduce_kernel<<<(int)g, 256, 0, st>>>(P, p.splits, (int)M, (int)N, sa, sb, bias, C, ldc);
+    splitk_reduce_kernel<CT><<<(int)g, 256, 0, st>>>(P, p.splits, (int)M, (int)N, sa, sb, bias, C, ldc);
   }
   return (int)hipGetLastError();
 }
@@ -707,6 +777,36 @@ int gpic_fp8_gemm_mn(const uint8_t *A, int64_t lda, const float *sa, const uint8
       ldc >= (1 << 22) || M >= (1 << 30))
     return GPIC_ESHAPE;
   return launch_gemm<true>(A, lda, sa, B, ldb, sb, bias, C, ldc, M, N, K, ws, ws_bytes, (hipStream_t)stream);
+}
+
+// every MN-major load offset (K row x row stride) is a 32-bit buffer offset, and so is every C offset
+static bool mn_shape_ok(int64_t lda, int64_t ldb, int64_t ldc, int64_t M, int64_t N, int64_t K, int64_t el, int64_t cbytes) {
+  return M % 16 == 0 && N % 16 == 0 && lda * el % 16 == 0 && ldb * el % 16 == 0 && ldc % 8 == 0 && lda >= M &&
+         ldb >= N && ldc >= N && lda < (1 << 30) && ldb < (1 << 30) && K * lda * el < (int64_t(1) << 31) &&
+         K * ldb * el < (int64_t(1) << 31) && ldc * cbytes < (1 << 23) && M < (1 << 30);
+}
+
+int gpic_fp8_gemm_mn_f32(const uint8_t *A, int64_t lda, const float *sa, const uint8_t *B, int64_t ldb,
+                         const float *sb, float *C, int64_t ldc, int64_t M, int64_t N, int64_t K, void *ws,
+                         size_t ws_bytes, void *stream) {
+  status_scope();
+  if (M < 0 || N < 0 || K < 0 || !sa || !sb || (M > 0 && N > 0 && !C)) return GPIC_EINVAL;
+  if (!mn_shape_ok(lda, ldb, ldc, M, N, K, 1, 4)) return GPIC_ESHAPE;
+  return launch_gemm<true, 1, float>(A, lda, sa, B, ldb, sb, nullptr, C, ldc, M, N, K, ws, ws_bytes,
+                                     (hipStream_t)stream);
+}
+
+int gpic_fp8_bf16_gemm_mn(const uint16_t *A, int64_t lda, const uint16_t *B, int64_t ldb, void *C, int c_dtype,
+                          int64_t ldc, int64_t M, int64_t N, int64_t K, void *ws, size_t ws_bytes, void *stream) {
+  status_scope();
+  if (M < 0 || N < 0 || K < 0 || (M > 0 && N > 0 && !C)) return GPIC_EINVAL;
+  if (c_dtype != GPIC_DTYPE_BF16 && c_dtype != GPIC_DTYPE_F32) return GPIC_EDTYPE;
+  if (!mn_shape_ok(lda, ldb, ldc, M, N, K, 2, c_dtype == GPIC_DTYPE_F32 ? 4 : 2)) return GPIC_ESHAPE;
+  if (c_dtype == GPIC_DTYPE_F32)
+    return launch_gemm<true, 2, float>(A, lda, nullptr, B, ldb, nullptr, nullptr, static_cast<float *>(C), ldc, M, N, K,
+                                       ws, ws_bytes, (hipStream_t)stream);
+  return launch_gemm<true, 2>(A, lda, nullptr, B, ldb, nullptr, nullptr, static_cast<uint16_t *>(C), ldc, M, N, K, ws,
+                              ws_bytes, (hipStream_t)stream);
 }
 
 }  // extern "C"

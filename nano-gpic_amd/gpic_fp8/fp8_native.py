@@ -488,6 +488,68 @@ def _(a, sa, b, sb, bias=None):
     return a.new_empty(a.shape[1], b.shape[1], dtype=torch.bfloat16)
 
 
+@L.step_op("gpic::fp8_wgrad")
+def fp8_wgrad(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Tensor, f32: bool) -> torch.Tensor:
+    """fp8_gemm_mn(a, sa, b, sb), in fp32 when f32 (an fp32 weight's gradient, written by the GEMM itself)."""
+    a2, b2 = _gemm_operand_mn(a, "a"), _gemm_operand_mn(b, "b")
+    (K, M), N = a2.shape, b2.shape[1]
+    if not f32 or K * max(a2.stride(0), b2.stride(0)) >= 2 ** 31 or N >= 2 ** 21:
+        dw = L.call(fp8_gemm_mn, a, sa, b, sb)
+        return dw.float() if f32 else dw
+    L.require_gpu(a2, b2, sa, sb)
+    c = torch.empty(M, N, dtype=torch.float32, device=a.device)
+    with L.on_device(a.device):
+        nws = L.gemm_workspace_bytes(a.device, M, N, K)
+        ws = torch.empty(nws, dtype=torch.uint8, device=a.device) if nws else None
+        L.check(L.lib().gpic_fp8_gemm_mn_f32(a2.data_ptr(), a2.stride(0), sa.data_ptr(), b2.data_ptr(), b2.stride(0),
+                                             sb.data_ptr(), c.data_ptr(), N, M, N, K, L.ptr(ws), nws,
+                                             L.stream_ptr(a.device)), "gpic_fp8_gemm_mn_f32")
+    return c
+
+
+@fp8_wgrad.register_fake
+def _(a, sa, b, sb, f32):
+    return a.new_empty(a.shape[1], b.shape[1], dtype=torch.float32 if f32 else torch.bfloat16)
+
+
+@L.step_op("gpic::fp8_bf16_wgrad")
+def bf16_wgrad(dy: torch.Tensor, x: torch.Tensor, f32: bool) -> torch.Tensor:
+    """(dy [M, N].t() @ x [M, K]) bf16 -> [N, K] bf16, or its values in fp32 (fp8_native.py:202, 225, 264-265): the bf16
+    wgrad on the hand-written GEMM, both operands read with the tokens as their rows, the gradient of an fp32 weight
+    written as fp32."""
+    L.require_gpu(dy, x)
+    dy, x = _prep_rows(dy, dy.shape[1]), _prep_rows(x, x.shape[1])
+    (M, N), K = dy.shape, x.shape[1]
+    dt = torch.float32 if f32 else torch.bfloat16
+    if N % 16 or K % 16 or 2 * M * max(dy.stride(0), x.stride(0)) >= 2 ** 31 or K >= 2 ** 21:
+        return (dy.t() @ x).to(dt)
+    dw = torch.empty(N, K, dtype=dt, device=dy.device)
+    with L.on_device(dy.device):
+        nws = L.gemm_workspace_bytes(dy.device, N, K, 2 * M)   # (planned as an e4m3 GEMM of as many K bytes)
+        ws = torch.empty(nws, dtype=torch.uint8, device=dy.device) if nws else None
+        L.check(L.lib().gpic_fp8_bf16_gemm_mn(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), dw.data_ptr(),
+                                              L.DTYPE_CODE[dt], K, N, K, M, L.ptr(ws), nws, L.stream_ptr(dy.device)),
+                "gpic_fp8_bf16_gemm_mn")
+    return dw
+
+
+@bf16_wgrad.register_fake
+def _(dy, x, f32):
+    return dy.new_empty(dy.shape[1], x.shape[1], dtype=torch.float32 if f32 else torch.bfloat16)
+
+
+def _recorded():
+    """Whether a backward is itself being recorded (create_graph): its operations then have to be differentiable ones."""
+    return torch.is_grad_enabled() and not torch.compiler.is_compiling()
+
+
+def _wgrad16(dy, x, dtype):
+    """(dy.t() @ x).to(dtype)."""
+    if _recorded():
+        return (dy.t() @ x).to(dtype)
+    return L.call(bf16_wgrad, dy, x, dtype == torch.float32).to(dtype)
+
+
 def _mm(xq, sx, wq, sw, fast=True):
     """[M, K] e4m3 x [N, K] e4m3 (each with its tensorwise scale) -> [M, N] bf16 (fp8_native.py:175-178)."""
     return L.call(fp8_gemm, xq, sx, wq, sw, None, fast)
@@ -513,7 +575,7 @@ class _Fp8Linear(torch.autograd.Function):
         x2, w = ctx.saved_tensors
         dy2 = dy.reshape(-1, dy.shape[-1]).to(torch.bfloat16)
         dx = (dy2 @ w.to(torch.bfloat16)).view(ctx.shape)
-        dw = (dy2.t() @ x2).to(ctx.wdt)
+        dw = _wgrad16(dy2, x2, ctx.wdt)
         db = dy2.sum(0).to(ctx.wdt) if ctx.has_b else None
         return dx, dw, db
 
@@ -590,10 +652,10 @@ class _SwiGLUw3(torch.autograd.Function):
         z, aq, sa, w3 = ctx.saved_tensors
         dy2 = dy.reshape(-1, dy.shape[-1]).to(torch.bfloat16)
         da = dy2 @ w3.to(torch.bfloat16)
-        dw3 = (dy2.t() @ L.call(dequant, aq, sa)).to(ctx.wdt)
-        if not torch.is_grad_enabled() or torch.compiler.is_compiling():
+        dw3 = _wgrad16(dy2, L.call(dequant, aq, sa), ctx.wdt)
+        if not _recorded():
             return L.call(swiglu_dz, z, da).view(ctx.shape), dw3
-        # a backward that is itself recorded (create_graph): the same expression as torch operations
+        # the same expression as torch operations
         z1, z2 = z.chunk(2, dim=-1)
         z1f = z1.float()
         sg = torch.sigmoid(z1f)
@@ -631,8 +693,8 @@ class _Fp8MLP(torch.autograd.Function):
         dz, dzq, sdz = L.call(swiglu_bwd, z, da)
         _, w12tq, s12t = L.call(tcast_t, w12, False)               # [C, 2H]
         dx = _mm(dzq, sdz, w12tq, s12t, fast=False)        # [M, C]
-        dw12 = (dz.t() @ x2).to(ctx.dt[0])
-        dw3 = (dy2.t() @ L.call(dequant, aq, sa)).to(ctx.dt[1])
+        dw12 = _wgrad16(dz, x2, ctx.dt[0])
+        dw3 = _wgrad16(dy2, L.call(dequant, aq, sa), ctx.dt[1])
         return dx.view(ctx.shape), dw12, dw3
 
 
