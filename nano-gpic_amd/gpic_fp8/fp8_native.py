@@ -538,6 +538,11 @@ def _(dy, x, f32):
     return dy.new_empty(dy.shape[1], x.shape[1], dtype=torch.float32 if f32 else torch.bfloat16)
 
 
+def _wgrad8(a, sa, b, sb, dtype):
+    """fp8_gemm_mn(a, sa, b, sb).to(dtype)."""
+    return L.call(fp8_wgrad, a, sa, b, sb, dtype == torch.float32).to(dtype)
+
+
 def _recorded():
     """Whether a backward is itself being recorded (create_graph): its operations then have to be differentiable ones."""
     return torch.is_grad_enabled() and not torch.compiler.is_compiling()
@@ -600,7 +605,7 @@ class _Fp8LinearF8(torch.autograd.Function):
         dy2 = dy.reshape(-1, dy.shape[-1]).to(torch.bfloat16)
         dyq, sdy = L.call(tcast, dy2)
         dx = L.call(fp8_gemm, dyq, sdy, wqt, sw, None, False).view(ctx.shape)     # [M, N] . [K, N]^T
-        dw = L.call(fp8_gemm_mn, dyq, sdy, xq, sx).to(ctx.wdt)                   # [M, N]^T . [M, K]
+        dw = _wgrad8(dyq, sdy, xq, sx, ctx.wdt)                                    # [M, N]^T . [M, K]
         db = dy2.sum(0).to(ctx.wdt) if ctx.has_b else None
         return dx, dw, db, None
 
@@ -629,7 +634,7 @@ class _Fp8HeadsLinearF8(torch.autograd.Function):
         dyq, sdy = L.call(tcast, dy2)
         dx = L.call(fp8_gemm, dyq, sdy, wqt, sw, None, False)                      # [M, N] . [K, N]^T
         do = dx.view(B, N, H, D).transpose(1, 2)
-        dw = L.call(fp8_gemm_mn, dyq, sdy, xq, sx).to(ctx.wdt)                     # [M, N]^T . [M, K]
+        dw = _wgrad8(dyq, sdy, xq, sx, ctx.wdt)                                    # [M, N]^T . [M, K]
         db = dy2.sum(0).to(ctx.wdt) if ctx.has_b else None
         return do, dw, db, None
 
@@ -722,11 +727,11 @@ class _Fp8MLPF8(torch.autograd.Function):
         dy2 = dy.reshape(-1, dy.shape[-1]).to(torch.bfloat16)
         dyq, sdy = L.call(tcast, dy2)
         da = L.call(fp8_gemm, dyq, sdy, w3qt, s3, None, False)           # [M, H]
-        dw3 = L.call(fp8_gemm_mn, dyq, sdy, aq, sa)                      # [M, C]^T . [M, H] = [C, H]
+        dw3 = _wgrad8(dyq, sdy, aq, sa, ctx.dt[1])                       # [M, C]^T . [M, H] = [C, H]
         dzq, sdz = L.call(swiglu_bwd_q, z, da)                           # dz itself is not needed: never written
         dx = L.call(fp8_gemm, dzq, sdz, w12qt, s12, None, False)         # [M, C]
-        dw12 = L.call(fp8_gemm_mn, dzq, sdz, xq, sx)                     # [M, 2H]^T . [M, C] = [2H, C]
-        return dx.view(ctx.shape), dw12.to(ctx.dt[0]), dw3.to(ctx.dt[1]), None, None
+        dw12 = _wgrad8(dzq, sdz, xq, sx, ctx.dt[0])                      # [M, 2H]^T . [M, C] = [2H, C]
+        return dx.view(ctx.shape), dw12, dw3, None, None
 
 
 def fp8_mlp(x, w12, w3):

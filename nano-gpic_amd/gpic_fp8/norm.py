@@ -27,7 +27,7 @@ from typing import Optional
 import torch
 
 from . import _lib as L
-from .fp8_native import (E4, Fp8LinearF8, fp8_gemm, fp8_gemm_mn, fp8_linear_f8, swiglu_bwd_q, swiglu_tcast, tcast,
+from .fp8_native import (E4, Fp8LinearF8, _wgrad8, fp8_gemm, fp8_linear_f8, swiglu_bwd_q, swiglu_tcast, tcast,
                          tcast_t)
 
 
@@ -290,7 +290,7 @@ class _Fp8ModRMSNormLinear(torch.autograd.Function):
         dy2 = dy.reshape(B * N, -1).to(torch.bfloat16)
         dyq, sdy = L.call(tcast, dy2)
         dh = L.call(fp8_gemm, dyq, sdy, wqt, sw, None, False).view(B, N, C)
-        dweight = L.call(fp8_gemm_mn, dyq, sdy, hq2, sh).to(ctx.wdt)
+        dweight = _wgrad8(dyq, sdy, hq2, sh, ctx.wdt)
         db = dy2.sum(0).to(ctx.wdt) if ctx.has_b else None
         dx, _, _, dw, dsh, dsc = _norm_backward(dh, None, x, None, None, w_norm, scale, rstd)
         _, dw, dshift, dscale = _param_grads(B, C, None, dw, dsh, dsc, None, w_norm, shift, scale)
@@ -323,13 +323,13 @@ class _Fp8ResModRMSNormMLP(torch.autograd.Function):
         dy2 = dy.reshape(B * N, -1).to(torch.bfloat16)
         dyq, sdy = L.call(tcast, dy2)
         da_ = L.call(fp8_gemm, dyq, sdy, w3qt, s3, None, False)
-        dw3 = L.call(fp8_gemm_mn, dyq, sdy, aq, sa)
+        dw3 = _wgrad8(dyq, sdy, aq, sa, ctx.dt[1])
         dzq, sdz = L.call(swiglu_bwd_q, z, da_)
         dh = L.call(fp8_gemm, dzq, sdz, w12qt, s12, None, False).view(B, N, C)
-        dw12 = L.call(fp8_gemm_mn, dzq, sdz, hq2, sh)
+        dw12 = _wgrad8(dzq, sdz, hq2, sh, ctx.dt[0])
         dx, da, dg, dw, dsh, dsc = _norm_backward(dh, dxn, xn, a, gate, w_norm, scale, rstd)
         dgate, dw, dshift, dscale = _param_grads(B, C, dg, dw, dsh, dsc, gate, w_norm, shift, scale)
-        return dx, da, dgate, dw, dshift, dscale, None, dw12.to(ctx.dt[0]), dw3.to(ctx.dt[1])
+        return dx, da, dgate, dw, dshift, dscale, None, dw12, dw3
 
 
 def fp8_mod_rmsnorm_linear(x, w_norm, shift, scale, eps, weight, bias: Optional[torch.Tensor] = None):
