@@ -195,6 +195,15 @@ int gpic_fp8_swiglu_dz(const uint16_t *z, const uint16_t *da, int64_t M, int64_t
 int gpic_fp8_dequant(const uint8_t *q, const float *s, int64_t n, uint16_t *y, void *stream);
 
 /*
+ * The bias gradient: db[n] = bf16(sum_m dy[m, n]) with fp32 sums in a fixed order, stored as bf16 or (the same values)
+ * fp32, dtype GPIC_DTYPE_*. dy [M, N] bf16, row stride ld; N, ld % 8 == 0, dy 16-byte aligned; any M. Replaces
+ * dy2.sum(0).to(wdt) (fp8_native.py:203). ws: gpic_fp8_bias_grad_workspace_bytes(M, N) bytes of scratch.
+ */
+size_t gpic_fp8_bias_grad_workspace_bytes(int64_t M, int64_t N);
+int gpic_fp8_bias_grad(const uint16_t *dy, int64_t ld, int64_t M, int64_t N, void *db, int dtype, void *ws,
+                       size_t ws_bytes, void *stream);
+
+/*
  * The norm sites' producer with the cast of its output folded in. Replaces gpic::res_mod_rmsnorm_fwd
  * (baselines/PixelGen/src/models/layers/fused_norm.py:150-175, kernel :64-91) followed by the FP8 linear's tcast of
  * its output h (fp8_native.py:114-122), as one producer (the reference keeps them apart, fp8_native.py:3-6):

@@ -767,6 +767,70 @@ __global__ __launch_bounds__(kCastThreads) void dequant_kernel(const uint8_t *__
   }
 }
 
+// The bias gradient: column sums of dy [M, N] bf16 (row stride ld, N % 8 == 0) in fp32, rounded once to bf16 (as
+// torch's bf16 sum) and stored as bf16 or fp32, in a fixed order. Bound by reading dy once: a workgroup takes 256
+// columns (32 lanes x 8, 512-byte row segments) of every P-th group of 8 rows, its 8 row lanes with kSumRows rows in
+// flight each, adds them in LDS and writes one partial row; the second kernel adds the P partials, 16 columns a
+XX
+// sum with the memset it queues (and 4 us for the conversion to an fp32 bias's gradient).
+constexpr int kSumCols = 256, kSumLanes = 8, kSumRows = 4, kSumBlocks = 1024, kMaxSumParts = 256;
+__global__ __launch_bounds__(256) void colsum_kernel(const uint16_t *__restrict__ dy, int64_t M, int64_t N, int64_t ld,
+                                                     float *__restrict__ part) {
+  __shared__ float red[kSumLanes][kSumCols];
+  const int cg = threadIdx.x & 31, rl = threadIdx.x >> 5;
+  const int64_t c = (int64_t)blockIdx.x * kSumCols + 8 * cg;
+  const int64_t step = (int64_t)gridDim.y * kSumLanes;
+  float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  if (c < N) {
+    const uint16_t *p = dy + c;
+    int64_t r = (int64_t)blockIdx.y * kSumLanes + rl;
+    auto add = [&](u32x4 w) {
+      float v[8];
+      unpack8(w, v);
+#pragma unroll
+      for (int e = 0; e < 8; e++) s[e] = s[e] + v[e];
+    };
+    for (; r + (kSumRows - 1) * step < M; r += kSumRows * step) {
+      u32x4 w[kSumRows];
+#pragma unroll
+      for (int k = 0; k < kSumRows; k++) w[k] = *reinterpret_cast<const u32x4 *>(p + (r + k * step) * ld);
+#pragma unroll
+      for (int k = 0; k < kSumRows; k++) add(w[k]);
+    }
+    for (; r < M; r += step) add(*reinterpret_cast<const u32x4 *>(p + r * ld));
+  }
+#pragma unroll
+  for (int e = 0; e < 8; e++) red[rl][8 * cg + e] = s[e];
+  __syncthreads();
+  const int64_t col = (int64_t)blockIdx.x * kSumCols + threadIdx.x;
+  if (col >= N) return;
+  float v = red[0][threadIdx.x];
+#pragma unroll
+  for (int k = 1; k < kSumLanes; k++) v = v + red[k][threadIdx.x];
+  part[(int64_t)blockIdx.y * N + col] = v;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void colsum_reduce_kernel(const float *__restrict__ part, int P, int64_t N,
+                                                            T *__restrict__ db) {
+  __shared__ float chunk[16][16];
+  const int cl = threadIdx.x & 15, k = threadIdx.x >> 4;
+  const int64_t c = (int64_t)blockIdx.x * 16 + cl;   // (N % 8 == 0: the last 16 columns may be half)
+  const int per = (P + 15) / 16, q0 = k * per, q1 = min(P, q0 + per);
+  float s = 0.0f;
+  if (c < N)
+    for (int q = q0; q < q1; q++) s = s + part[(int64_t)q * N + c];
+  chunk[k][cl] = s;
+  __syncthreads();
+  if (k != 0 || c >= N) return;
+  s = chunk[0][cl];
+#pragma unroll
+  for (int i = 1; i < 16; i++) s = s + chunk[i][cl];
+  const uint32_t h = bf16_rne(s);
+  if constexpr (sizeof(T) == 4) db[c] = __uint_as_float(h << 16);
+  else db[c] = (T)h;
+}
+
 // ------------------------------------------------------------------------------------------- host side
 
 static inline int grid_for(int64_t units, int cap) {
@@ -2198,6 +2262,39 @@ int gpic_fp8_dequant(const uint8_t *q, const float *s, int64_t n, uint16_t *y, v
   if (n == 0) return GPIC_OK;
   const int grid = grid_for((n / 16 + kUnroll - 1) / kUnroll, kMaxCastBlocks);
   dequant_kernel<<<grid, kCastThreads, 0, (hipStream_t)stream>>>(q, s, n, y);
+  return (int)hipGetLastError();
+}
+
+// partial rows of the column sums: enough workgroups to fill the device, each with at least one round of rows in flight
+static int64_t colsum_parts(int64_t M, int64_t N) {
+  const int64_t cb = (N + kSumCols - 1) / kSumCols;
+  const int64_t fill = std::max<int64_t>(1, kSumBlocks / std::max<int64_t>(cb, 1));
+  const int64_t need = (M + kSumLanes * kSumRows - 1) / (kSumLanes * kSumRows);
+  return std::max<int64_t>(1, std::min<int64_t>(std::min(fill, need), kMaxSumParts));
+}
+
+size_t gpic_fp8_bias_grad_workspace_bytes(int64_t M, int64_t N) {
+  return M < 0 || N <= 0 ? 0 : (size_t)(colsum_parts(M, N) * N) * sizeof(float);
+}
+
+int gpic_fp8_bias_grad(const uint16_t *dy, int64_t ld, int64_t M, int64_t N, void *db, int dtype, void *ws,
+                       size_t ws_bytes, void *stream) {
+  status_scope();
+  if (M < 0 || N < 0 || (N > 0 && (!db || !ws)) || (M > 0 && N > 0 && !dy)) return GPIC_EINVAL;
+  if (dtype != GPIC_DTYPE_BF16 && dtype != GPIC_DTYPE_F32) return GPIC_EDTYPE;
+  if (N % 8 != 0 || ld % 8 != 0 || ld < N || N > (int64_t(1) << 30)) return GPIC_ESHAPE;
+  if (!aligned16(dy) || !aligned16(ws)) return GPIC_EALIGN;
+  if (N == 0) return GPIC_OK;
+  if (ws_bytes < gpic_fp8_bias_grad_workspace_bytes(M, N)) return GPIC_EWORKSPACE;
+  hipStream_t st = (hipStream_t)stream;
+  float *part = static_cast<float *>(ws);
+  const int P = (int)colsum_parts(M, N);
+  colsum_kernel<<<dim3((unsigned)((N + kSumCols - 1) / kSumCols), (unsigned)P), 256, 0, st>>>(dy, M, N, ld, part);
+  const int grid = (int)((N + 15) / 16);
+  if (dtype == GPIC_DTYPE_F32)
+    colsum_reduce_kernel<<<grid, 256, 0, st>>>(part, P, N, static_cast<float *>(db));
+  else
+    colsum_reduce_kernel<<<grid, 256, 0, st>>>(part, P, N, static_cast<uint16_t *>(db));
   return (int)hipGetLastError();
 }
 

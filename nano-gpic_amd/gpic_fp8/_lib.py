@@ -36,6 +36,8 @@ SIGNATURES = {
     "gpic_fp8_swiglu_bwd_t": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _vp, _vp]),
     "gpic_fp8_swiglu_dz": (_int, [_vp, _vp, _i64, _i64, _i64, _i64, _vp, _vp]),
     "gpic_fp8_dequant": (_int, [_vp, _vp, _i64, _vp, _vp]),
+    "gpic_fp8_bias_grad_workspace_bytes": (_sz, [_i64, _i64]),
+    "gpic_fp8_bias_grad": (_int, [_vp, _i64, _i64, _i64, _vp, _int, _vp, _sz, _vp]),
     "gpic_fp8_res_mod_rmsnorm": (_int, [_vp, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _i64, _i64, _i64, _i64,
                                          ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "gpic_fp8_res_mod_rmsnorm_bwd_workspace_bytes": (_sz, [_i64, _i64, _i64]),

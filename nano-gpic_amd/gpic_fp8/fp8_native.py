@@ -51,6 +51,16 @@ def _prep_rows(t, min_cols):
     return t
 
 
+def _rows(t):
+    """_prep_rows of a 2-D tensor with a multiple of 8 columns, and its row stride; the stride of a single row, which may
+    be any number, counts as the row's length."""
+    if t.shape[0] <= 1:
+        t = L.aligned(t.contiguous())
+        return t, t.shape[1]
+    t = _prep_rows(t, t.shape[1])
+    return t, t.stride(0)
+
+
 # ------------------------------------------------------------------------------------------------ casts
 
 @L.custom_op("gpic::fp8_tcast")
@@ -512,23 +522,47 @@ def _(a, sa, b, sb, f32):
     return a.new_empty(a.shape[1], b.shape[1], dtype=torch.float32 if f32 else torch.bfloat16)
 
 
+@L.step_op("gpic::fp8_bias_grad")
+def bias_grad(dy: torch.Tensor, f32: bool) -> torch.Tensor:
+    """dy [M, N] bf16 -> dy.sum(0) (fp32 sums, one bf16 rounding), as bf16 or its values in fp32 (fp8_native.py:203)."""
+    L.require_gpu(dy)
+    dt = torch.float32 if f32 else torch.bfloat16
+    M, N = dy.shape
+    if N % 8:
+        return dy.sum(0).to(dt)
+    dy, ld = _rows(dy)
+    db = torch.empty(N, dtype=dt, device=dy.device)
+    with L.on_device(dy.device):
+        nws = L.lib().gpic_fp8_bias_grad_workspace_bytes(M, N)
+        ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=dy.device)
+        L.check(L.lib().gpic_fp8_bias_grad(dy.data_ptr(), ld, M, N, db.data_ptr(), L.DTYPE_CODE[dt],
+                                           ws.data_ptr(), nws, L.stream_ptr(dy.device)), "gpic_fp8_bias_grad")
+    return db
+
+
+@bias_grad.register_fake
+def _(dy, f32):
+    return dy.new_empty(dy.shape[1], dtype=torch.float32 if f32 else torch.bfloat16)
+
+
 @L.step_op("gpic::fp8_bf16_wgrad")
 def bf16_wgrad(dy: torch.Tensor, x: torch.Tensor, f32: bool) -> torch.Tensor:
     """(dy [M, N].t() @ x [M, K]) bf16 -> [N, K] bf16, or its values in fp32 (fp8_native.py:202, 225, 264-265): the bf16
     wgrad on the hand-written GEMM, both operands read with the tokens as their rows, the gradient of an fp32 weight
     written as fp32."""
     L.require_gpu(dy, x)
-    dy, x = _prep_rows(dy, dy.shape[1]), _prep_rows(x, x.shape[1])
     (M, N), K = dy.shape, x.shape[1]
     dt = torch.float32 if f32 else torch.bfloat16
-    if N % 16 or K % 16 or 2 * M * max(dy.stride(0), x.stride(0)) >= 2 ** 31 or K >= 2 ** 21:
+    if N % 16 == 0 and K % 16 == 0:
+        (dy, ldy), (x, ldx) = _rows(dy), _rows(x)
+    if N % 16 or K % 16 or 2 * M * max(ldy, ldx) >= 2 ** 31 or K >= 2 ** 21:
         return (dy.t() @ x).to(dt)
     dw = torch.empty(N, K, dtype=dt, device=dy.device)
     with L.on_device(dy.device):
         nws = L.gemm_workspace_bytes(dy.device, N, K, 2 * M)   # (planned as an e4m3 GEMM of as many K bytes)
         ws = torch.empty(nws, dtype=torch.uint8, device=dy.device) if nws else None
-        L.check(L.lib().gpic_fp8_bf16_gemm_mn(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), dw.data_ptr(),
-                                              L.DTYPE_CODE[dt], K, N, K, M, L.ptr(ws), nws, L.stream_ptr(dy.device)),
+        L.check(L.lib().gpic_fp8_bf16_gemm_mn(dy.data_ptr(), ldy, x.data_ptr(), ldx, dw.data_ptr(), L.DTYPE_CODE[dt],
+                                              K, N, K, M, L.ptr(ws), nws, L.stream_ptr(dy.device)),
                 "gpic_fp8_bf16_gemm_mn")
     return dw
 
@@ -536,6 +570,11 @@ def bf16_wgrad(dy: torch.Tensor, x: torch.Tensor, f32: bool) -> torch.Tensor:
 @bf16_wgrad.register_fake
 def _(dy, x, f32):
     return dy.new_empty(dy.shape[1], x.shape[1], dtype=torch.float32 if f32 else torch.bfloat16)
+
+
+def _bias_grad(dy, dtype):
+    """dy.sum(0).to(dtype)."""
+    return dy.sum(0).to(dtype) if _recorded() else L.call(bias_grad, dy, dtype == torch.float32).to(dtype)
 
 
 def _wgrad8(a, sa, b, sb, dtype):
@@ -581,7 +620,7 @@ class _Fp8Linear(torch.autograd.Function):
         dy2 = dy.reshape(-1, dy.shape[-1]).to(torch.bfloat16)
         dx = (dy2 @ w.to(torch.bfloat16)).view(ctx.shape)
         dw = _wgrad16(dy2, x2, ctx.wdt)
-        db = dy2.sum(0).to(ctx.wdt) if ctx.has_b else None
+        db = _bias_grad(dy2, ctx.wdt) if ctx.has_b else None
         return dx, dw, db
 
 
@@ -606,7 +645,7 @@ class _Fp8LinearF8(torch.autograd.Function):
         dyq, sdy = L.call(tcast, dy2)
         dx = L.call(fp8_gemm, dyq, sdy, wqt, sw, None, False).view(ctx.shape)     # [M, N] . [K, N]^T
         dw = _wgrad8(dyq, sdy, xq, sx, ctx.wdt)                                    # [M, N]^T . [M, K]
-        db = dy2.sum(0).to(ctx.wdt) if ctx.has_b else None
+        db = _bias_grad(dy2, ctx.wdt) if ctx.has_b else None
         return dx, dw, db, None
 
 
@@ -635,7 +674,7 @@ class _Fp8HeadsLinearF8(torch.autograd.Function):
         dx = L.call(fp8_gemm, dyq, sdy, wqt, sw, None, False)                      # [M, N] . [K, N]^T
         do = dx.view(B, N, H, D).transpose(1, 2)
         dw = _wgrad8(dyq, sdy, xq, sx, ctx.wdt)                                    # [M, N]^T . [M, K]
-        db = dy2.sum(0).to(ctx.wdt) if ctx.has_b else None
+        db = _bias_grad(dy2, ctx.wdt) if ctx.has_b else None
         return do, dw, db, None
 
 

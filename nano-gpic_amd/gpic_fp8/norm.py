@@ -27,8 +27,8 @@ from typing import Optional
 import torch
 
 from . import _lib as L
-from .fp8_native import (E4, Fp8LinearF8, _wgrad8, fp8_gemm, fp8_linear_f8, swiglu_bwd_q, swiglu_tcast, tcast,
-                         tcast_t)
+from .fp8_native import (E4, Fp8LinearF8, _bias_grad, _wgrad8, fp8_gemm, fp8_linear_f8, swiglu_bwd_q, swiglu_tcast,
+                         tcast, tcast_t)
 
 
 # The widest rows the backward kernel takes (its per-column sums live in registers); the forward takes any width.
@@ -291,7 +291,7 @@ class _Fp8ModRMSNormLinear(torch.autograd.Function):
         dyq, sdy = L.call(tcast, dy2)
         dh = L.call(fp8_gemm, dyq, sdy, wqt, sw, None, False).view(B, N, C)
         dweight = _wgrad8(dyq, sdy, hq2, sh, ctx.wdt)
-        db = dy2.sum(0).to(ctx.wdt) if ctx.has_b else None
+        db = _bias_grad(dy2, ctx.wdt) if ctx.has_b else None
         dx, _, _, dw, dsh, dsc = _norm_backward(dh, None, x, None, None, w_norm, scale, rstd)
         _, dw, dshift, dscale = _param_grads(B, C, None, dw, dsh, dsc, None, w_norm, shift, scale)
         return dx, dw, dshift, dscale, None, dweight, db
