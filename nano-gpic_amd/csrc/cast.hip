@@ -771,8 +771,8 @@ __global__ __launch_bounds__(kCastThreads) void dequant_kernel(const uint8_t *__
 // torch's bf16 sum) and stored as bf16 or fp32, in a fixed order. Bound by reading dy once: a workgroup takes 256
 // columns (32 lanes x 8, 512-byte row segments) of every P-th group of 8 rows, its 8 row lanes with kSumRows rows in
 // flight each, adds them in LDS and writes one partial row; the second kernel adds the P partials, 16 columns a
-XX
-// sum with the memset it queues (and 4 us for the conversion to an fp32 bias's gradient).
+// workgroup, each column in 16 chunks and the chunks in order. [32768 x 1024]: 13.0 + 5.2 us, against 39 us for torch's
+// sum with the memset it queues and 4 us for the conversion to an fp32 bias's gradient.
 constexpr int kSumCols = 256, kSumLanes = 8, kSumRows = 4, kSumBlocks = 1024, kMaxSumParts = 256;
 __global__ __launch_bounds__(256) void colsum_kernel(const uint16_t *__restrict__ dy, int64_t M, int64_t N, int64_t ld,
                                                      float *__restrict__ part) {
