@@ -96,14 +96,26 @@ int gpic_fp8_tcast_t(const void *x, int dtype, int64_t rows, int64_t cols, uint8
  * count transposing casts in one call: tensor i is x[i] [rows[i], cols[i]] -> q[i] (or NULL), qt[i] [cols[i], ldt[i]],
  * dequant[i], each with its own amax: the same bytes and scales as gpic_fp8_tcast_t on each tensor in order. No
  * counterpart in the reference, whose linears cast their weights one at a time inside each forward; this is for a
- * caller that casts a block's weights together before the block runs. bf16 tensors that fit the device together
- * (d12: the four weights, 1024 tiles of 128 x 128) are cast in ONE launch, each tensor over its own workgroups;
- * otherwise (fp32, more than 8 tensors, empty or larger tensors) the call makes the per-tensor calls. Every tensor is
+ * caller that casts a block's weights together before the block runs. Tensors that fit the device together
+ * (d12: the four weights, 1024 tiles of 128 x 128, in bf16 or fp32) are cast in ONE launch, each tensor over its own
+ * workgroups; otherwise (more than 8 tensors, empty or larger tensors) the call makes the per-tensor calls. Every tensor is
  * checked first, as gpic_fp8_tcast_t checks it; on an error nothing is launched.
  */
 int gpic_fp8_tcast_t_group(int count, const void *const *x, int dtype, const int64_t *rows, const int64_t *cols,
                            uint8_t *const *q, uint8_t *const *qt, const int64_t *ldt, float *const *dequant, void *ws,
                            void *stream);
+
+/*
+ * count casts in one call, each of its own kind: tensor i is x[i] [rows[i], cols[i]] of dtype[i]; with qt[i] NULL its
+ * flat cast to q[i] (gpic_fp8_tcast's bytes), else its transposing cast to q[i] (or NULL) and qt[i] [cols[i], ldt[i]]
+ * (gpic_fp8_tcast_t's), each with its own amax. Tensors that are not empty, fit the device together and are of one of
+ * these sets of kinds go in ONE launch: all transposing of one dtype; flat bf16; flat bf16 and flat fp32; flat bf16 and
+ * transposing of one dtype. Otherwise the call makes the per-tensor calls. For a linear's input and weights: small
+ * casts cost their launches and round trips, not their bytes.
+ */
+int gpic_fp8_cast_group(int count, const void *const *x, const int *dtype, const int64_t *rows, const int64_t *cols,
+                        uint8_t *const *q, uint8_t *const *qt, const int64_t *ldt, float *const *dequant, void *ws,
+                        void *stream);
 
 /*
  * The attention output's cast with its head merge folded in: the cast of proj's input, read from the attention's own

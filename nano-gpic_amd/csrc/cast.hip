@@ -2,15 +2,14 @@
 // dgrad / wgrad operands), the SwiGLU product cast and the SwiGLU backward.
 //
 // Two designs, chosen per call by size:
-//  * Single pass (flat bf16 tensors of at most 100 MiB, fp32 of 48 MiB, transposing bf16 casts of 64 MiB; hybrids up
-//    to 8x that; the SwiGLU casts, whose limits are stated with their kernels): ONE launch. Each workgroup holds its
+//  * Single pass (flat bf16 tensors of at most 100 MiB, fp32 of 48 MiB, transposing casts of 64 MiB; but for fp32 transposing
+//    casts hybrids up to 8x that; the SwiGLU casts, whose limits are stated with their kernels): ONE launch. Each workgroup holds its
 //    share of x on chip, publishes a partial maximum tagged with the call's number, folds every workgroup's partial and
 //    casts from what it holds (3 B/elem moved for bf16). The call number lives in the
 //    workspace (an epoch word the last workgroup of each call advances), so the workspace carries state from call to
 //    call: it is zeroed once when created, and calls that may run at the same time (different streams) need
 //    different workspaces. Graph capture is fine: a replayed launch reads the epoch the previous call left.
-//  * Two passes (larger tensors, the SwiGLU kernels past their single passes, fp32 transposing casts): two
-//    stream-ordered launches,
+//  * Two passes (larger tensors, the SwiGLU kernels past their single passes): two stream-ordered launches,
 //      1. an amax pass: each workgroup reduces its share to one partial maximum (|x| bit patterns, NaN ignored) and
 //         writes it to partial[blockIdx.x] -- no atomics, so nothing has to be zeroed beforehand;
 //      2. a cast pass: each workgroup folds all partials (<= kMaxParts words, served from L2), derives the scale with
@@ -867,45 +866,72 @@ static void launch_cast_t(Src src, int64_t rows, int64_t cols, int nparts, uint8
   cast_t_kernel<Src><<<grid, 256, 0, st>>>(src, rows, cols, partial, nparts, q, ldq, qt, ldt, dequant);
 }
 
-// A 128 x 128 bf16 tile (rows r0.., columns c0..) as thread tid's 8 raw chunks: chunk i is row id / 16, columns
-// 8 (id % 16) .. + 7 of the tile, id = tid + 256 i; zero outside x.
+// A 128 x 128 tile (rows r0.., columns c0..) of T as thread tid's 16-byte words: word i is row id / kC, columns
+// kE (id % kC) + [0, kE) of the tile, id = tid + 256 i (bf16: 8 words of 8 elements, fp32: 16 of 4); zero outside x.
 constexpr int kTPitch = kTT / 4 + 1;            // words per LDS row of the e4m3 tile (one word of padding)
-constexpr int kTPer = kTT * (kTT / 8) / 256;    // 8-element chunks per thread per tile: 8
-__device__ __forceinline__ void load_tile_bf16(const uint16_t *__restrict__ x, int64_t ld, int64_t rows, int64_t cols,
-                                               int64_t r0, int64_t c0, u32x4 (&R)[kTPer]) {
+template <typename T>
+struct TileOf {
+  static constexpr int kE = 16 / sizeof(T), kC = kTT / kE, kW = kTT * kC / 256;
+};
+constexpr int kTPer = TileOf<uint16_t>::kW;
+template <typename T>
+__device__ __forceinline__ void load_tile(const T *__restrict__ x, int64_t ld, int64_t rows, int64_t cols, int64_t r0,
+                                          int64_t c0, u32x4 (&R)[TileOf<T>::kW]) {
+  typedef TileOf<T> L;
+  if constexpr (sizeof(T) == 2) {
 #pragma unroll
-  for (int i = 0; i < kTPer; i++) {
-    const int id = threadIdx.x + 256 * i;
-    const int64_t gr = r0 + (id >> 4), gc = c0 + 8 * (id & 15);
-    R[i] = gr < rows && gc < cols ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x + gr * ld + gc))
-                                  : u32x4{0u, 0u, 0u, 0u};
+    for (int i = 0; i < L::kW; i++) {
+      const int id = threadIdx.x + 256 * i;
+      const int64_t gr = r0 + id / L::kC, gc = c0 + L::kE * (id % L::kC);
+      R[i] = gr < rows && gc < cols ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x + gr * ld + gc))
+                                    : u32x4{0u, 0u, 0u, 0u};
+    }
+  } else {   // twice as many words: a uniform base for each and one 32-bit offset per lane, not 16 lane addresses (a lane's
+             // row is below 8, and a tensor of at most 8192 tiles has at most 2^20 columns)
+    const int r = threadIdx.x / L::kC, c = L::kE * (threadIdx.x % L::kC);
+    const uint32_t off = (uint32_t)r * (uint32_t)ld + c;
+#pragma unroll
+    for (int i = 0; i < L::kW; i++) {
+      const int64_t ri = r0 + (256 / L::kC) * i;
+      R[i] = ri + r < rows && c0 + c < cols
+                 ? __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x + ri * ld + c0 + off))
+                 : u32x4{0u, 0u, 0u, 0u};
+    }
   }
 }
 
-// The tile held in R (as load_tile_bf16 left it) as e4m3 bytes with `scale`: 8 bytes per chunk.
-__device__ __forceinline__ void cvt_tile_bf16(const u32x4 (&R)[kTPer], float scale, u32x2 (&E)[kTPer]) {
+// The e4m3 bytes of a word: kE bytes.
+template <typename T>
+using CastWord = std::conditional_t<sizeof(T) == 2, u32x2, uint32_t>;
+__device__ __forceinline__ u32x2 cast_word(const uint16_t *, u32x4 w, float scale) { return cast8_bf16(w, scale); }
+__device__ __forceinline__ uint32_t cast_word(const float *, u32x4 w, float scale) { return cast4_f32(w, scale); }
+
+// The tile held in R (as load_tile left it) as e4m3 bytes with `scale`.
+template <typename T>
+__device__ __forceinline__ void cvt_tile(const u32x4 (&R)[TileOf<T>::kW], float scale, CastWord<T> (&E)[TileOf<T>::kW]) {
 #pragma unroll
-  for (int i = 0; i < kTPer; i++) {
-    float v[8];
-    unpack8(R[i], v);
-    E[i].x = e4m3x4(sat(v[0] * scale), sat(v[1] * scale), sat(v[2] * scale), sat(v[3] * scale));
-    E[i].y = e4m3x4(sat(v[4] * scale), sat(v[5] * scale), sat(v[6] * scale), sat(v[7] * scale));
-  }
+  for (int i = 0; i < TileOf<T>::kW; i++) E[i] = cast_word((const T *)nullptr, R[i], scale);
 }
 
-// Stores a tile's e4m3 bytes E (from cvt_tile_bf16): q rows from registers, qt through the LDS buffer `tile`
+// Stores a tile's e4m3 bytes E (from cvt_tile): q rows from registers, qt through the LDS buffer `tile`
 // ([row][col / 4] e4m3 words), which is free again when this returns. Same bytes as cast_t_kernel.
-__device__ __forceinline__ void emit_tile(const u32x2 (&E)[kTPer], int64_t r0, int64_t c0, int64_t rows, int64_t cols,
-                                          uint8_t *__restrict__ q, int64_t ldq, uint8_t *__restrict__ qt, int64_t ldt,
-                                          uint32_t *tile) {
+template <typename T>
+__device__ __forceinline__ void emit_tile(const CastWord<T> (&E)[TileOf<T>::kW], int64_t r0, int64_t c0, int64_t rows,
+                                          int64_t cols, uint8_t *__restrict__ q, int64_t ldq, uint8_t *__restrict__ qt,
+                                          int64_t ldt, uint32_t *tile) {
+  typedef TileOf<T> L;
 #pragma unroll
-  for (int i = 0; i < kTPer; i++) {
+  for (int i = 0; i < L::kW; i++) {
     const int id = threadIdx.x + 256 * i;
-    const int r = id >> 4, cc = id & 15;
-    const int64_t gr = r0 + r, gc = c0 + 8 * cc;
-    if (q && gr < rows && gc < cols) *reinterpret_cast<u32x2 *>(q + gr * ldq + gc) = E[i];
-    tile[r * kTPitch + 2 * cc] = E[i].x;
-    tile[r * kTPitch + 2 * cc + 1] = E[i].y;
+    const int r = id / L::kC, cc = id % L::kC;
+    const int64_t gr = r0 + r, gc = c0 + L::kE * cc;
+    if (q && gr < rows && gc < cols) *reinterpret_cast<CastWord<T> *>(q + gr * ldq + gc) = E[i];
+    if constexpr (sizeof(T) == 2) {
+      tile[r * kTPitch + 2 * cc] = E[i].x;
+      tile[r * kTPitch + 2 * cc + 1] = E[i].y;
+    } else {
+      tile[r * kTPitch + cc] = E[i];
+    }
   }
   lds_barrier();
   // qt rows c0 + 4k .. c0 + 4k + 3 get bytes r0 + 16p .. r0 + 16p + 15 of their columns, k = tid / 8, p = tid % 8
@@ -949,7 +975,7 @@ __global__ __launch_bounds__(256) void cast_t_bf16_kernel(const uint16_t *__rest
   const int64_t tiles_c = (cols + kTT - 1) / kTT, tiles = tiles_c * ((ldt + kTT - 1) / kTT);
   int64_t t = blockIdx.x;   // < tiles: the grid never exceeds the tile count
   u32x4 R[kTPer];
-  load_tile_bf16(x, ld, rows, cols, ((tiles - 1 - t) / tiles_c) * kTT, ((tiles - 1 - t) % tiles_c) * kTT, R);
+  load_tile(x, ld, rows, cols, ((tiles - 1 - t) / tiles_c) * kTT, ((tiles - 1 - t) % tiles_c) * kTT, R);
   float scale, deq;
   scales_from_amax(fold_partials(partial, nparts), scale, deq);   // its barriers wait for LDS only
   if (blockIdx.x == 0 && threadIdx.x == 0) *dequant = deq;
@@ -957,14 +983,14 @@ __global__ __launch_bounds__(256) void cast_t_bf16_kernel(const uint16_t *__rest
     const int64_t tn = t + gridDim.x;
     u32x4 Rn[kTPer];
     if (tn < tiles) {
-      load_tile_bf16(x, ld, rows, cols, ((tiles - 1 - tn) / tiles_c) * kTT, ((tiles - 1 - tn) % tiles_c) * kTT, Rn);
+      load_tile(x, ld, rows, cols, ((tiles - 1 - tn) / tiles_c) * kTT, ((tiles - 1 - tn) % tiles_c) * kTT, Rn);
     } else {
 #pragma unroll
       for (int i = 0; i < kTPer; i++) Rn[i] = u32x4{0u, 0u, 0u, 0u};
     }
     u32x2 E[kTPer];
-    cvt_tile_bf16(R, scale, E);
-    emit_tile(E, ((tiles - 1 - t) / tiles_c) * kTT, ((tiles - 1 - t) % tiles_c) * kTT, rows, cols, q, ldq, qt, ldt, tile);
+    cvt_tile<uint16_t>(R, scale, E);
+    emit_tile<uint16_t>(E, ((tiles - 1 - t) / tiles_c) * kTT, ((tiles - 1 - t) % tiles_c) * kTT, rows, cols, q, ldq, qt, ldt, tile);
 #pragma unroll
     for (int i = 0; i < kTPer; i++) R[i] = Rn[i];
   }
@@ -1017,8 +1043,8 @@ __global__ __launch_bounds__(256) void swiglu_bwd_cast_t_kernel(const uint16_t *
         E2[b + i] = ok[i] ? cast8_bf16(h2, scale) : u32x2{0u, 0u};
       }
     }
-    emit_tile(E1, r0, h0, M, H, dzq, 2 * H, dzqt, ldt, tile);
-    emit_tile(E2, r0, h0, M, H, dzq + H, 2 * H, dzqt + H * ldt, ldt, tile);
+    emit_tile<uint16_t>(E1, r0, h0, M, H, dzq, 2 * H, dzqt, ldt, tile);
+    emit_tile<uint16_t>(E2, r0, h0, M, H, dzq + H, 2 * H, dzqt + H * ldt, ldt, tile);
   }
 }
 
@@ -1048,8 +1074,7 @@ static_assert(kMaxParts * 4 + kLutSize * 4 <= (int)kOnceTagged, "two-pass scratc
 template <typename T>
 constexpr int kOnceWords = sizeof(T) == 2 ? 16 : 12;   // 16-byte words a thread of the flat kernel holds (fp32: 12,
                                                         // which its wider narrowing code needs to fit 128 VGPRs)
-constexpr int kOnceTiles = 2;       // 128 x 128 bf16 tiles a workgroup of the transposing kernel holds (64 VGPRs)
-constexpr int kHybridTiles = 8;     // the transposing kernel takes up to this many tiles per workgroup (2 held)
+constexpr int kHybridTiles = 8;     // the transposing kernel takes up to this many tiles per workgroup (bf16: 2 held, fp32: 1)
 constexpr int kHybridFlat = 8;      // the flat kernel takes up to this many times the words it can hold
 constexpr int kStream = 8;          // streamed words in flight per thread (flat hybrid)
 
@@ -1110,24 +1135,22 @@ __device__ __forceinline__ uint32_t words_amax(const u32x4 (&w)[W]) {
   return m;
 }
 
-// Flat single-pass cast. x as nw 16-byte words (8 bf16 or 4 fp32 elements) plus `tail` (< 8 or < 4) elements;
+// Flat single-pass cast, run by the G workgroups [first, first + G) of a launch. x as nw 16-byte words (8 bf16 or 4 fp32 elements) plus `tail` (< 8 or < 4) elements;
 // workgroup b holds words [b P, (b + 1) P), P = 256 wpt, thread t words b P + 256 j + t, j < wpt <= kOnceWords<T>.
 // Hybrid (sgroups > 0, x larger than the grid holds): the 256-word groups past the held words, G P + 256 s + t, are
 // streamed by workgroup s % G twice -- for the maximum, then (last first, for MALL hits) for the cast -- so only
 // what does not fit is read twice. Map: the source word of each output word (the tail is read flat: HeadMap sources
 // have none).
-template <typename T, class Map = FlatMap>
-__global__ __launch_bounds__(256, 4) void cast_once_kernel(const T *__restrict__ x, int64_t n, int wpt,
-                                                           int64_t sgroups, uint8_t *__restrict__ q,
-                                                           float *__restrict__ dequant, void *ws,
-                                                           uint32_t wait_ticks, const Map map = Map()) {
-  const uint32_t ep = once_epoch(ws);   // (before the first loads: its latency passes behind them)
+template <typename T, class Map>
+__device__ __forceinline__ void cast_once_run(const T *__restrict__ x, int64_t n, int wpt, int64_t sgroups,
+                                              uint8_t *__restrict__ q, float *__restrict__ dequant, void *ws,
+                                              uint32_t wait_ticks, uint32_t ep, int64_t blk, int64_t G, int first,
+                                              const Map map) {
   constexpr int kE = 16 / sizeof(T);   // elements per word
   const int64_t nw = n / kE;
   const int tail = (int)(n % kE);
   const u32x4 *xv = reinterpret_cast<const u32x4 *>(x);
   const int64_t P = 256 * (int64_t)wpt;
-  const int64_t G = gridDim.x;
   auto word = [&](int64_t b, int j) { return b * P + 256 * j + threadIdx.x; };
   // streamed word index (below 2^31: a hybrid x is at most kHybridFlat x 4 Mi words)
   auto sword = [&](int64_t s) { return (uint32_t)(G * P + 256 * s) + threadIdx.x; };
@@ -1149,7 +1172,7 @@ __global__ __launch_bounds__(256, 4) void cast_once_kernel(const T *__restrict__
   u32x4 w[kW];
 #pragma unroll
   for (int j = 0; j < kW; j++) {
-    const int64_t i = word(blockIdx.x, j);
+    const int64_t i = word(blk, j);
     w[j] = j < wpt && i < nw ? __builtin_nontemporal_load(xv + map(i)) : u32x4{0u, 0u, 0u, 0u};
   }
   // every workgroup folds the tail elements into its partial, so a partial computed from x includes them as well
@@ -1164,10 +1187,10 @@ __global__ __launch_bounds__(256, 4) void cast_once_kernel(const T *__restrict__
     return a;
   };
   uint32_t m0 = max(words_amax<T, kW>(w), tail_amax());
-  if (sgroups > 0) m0 = max(m0, stream_amax(blockIdx.x));
+  if (sgroups > 0) m0 = max(m0, stream_amax(blk));
   const uint32_t m = block_max_u32(m0);
   uint32_t tk;
-  const uint32_t g = once_fold(m, ws, ep, wait_ticks, tk, [&](int c) {
+  const uint32_t g = once_fold_range(m, ws, ep, wait_ticks, tk, first, (int)G, [&](int c) {
     uint32_t a = tail_amax();
     for (int j = 0; j < wpt; j++) {
       const int64_t i = word(c, j);
@@ -1179,8 +1202,8 @@ __global__ __launch_bounds__(256, 4) void cast_once_kernel(const T *__restrict__
   hold(w);
   float scale, deq;
   scales_from_amax(g, scale, deq);
-  if (blockIdx.x == 0 && threadIdx.x == 0) *dequant = deq;
-  const int64_t b2 = opaque_s64(blockIdx.x);   // the store addresses are recomputed, not kept from the loads
+  if (blk == 0 && threadIdx.x == 0) *dequant = deq;
+  const int64_t b2 = opaque_s64(blk);   // the store addresses are recomputed, not kept from the loads
 #pragma unroll
   for (int j = 0; j < kW; j++) {
     const int64_t i = word(b2, j);
@@ -1189,24 +1212,24 @@ __global__ __launch_bounds__(256, 4) void cast_once_kernel(const T *__restrict__
       else __builtin_nontemporal_store(cast4_f32(w[j], scale), reinterpret_cast<uint32_t *>(q) + i);
     }
   }
-  if (blockIdx.x == 0 && threadIdx.x < tail) {
+  if (blk == 0 && threadIdx.x < tail) {
     const int64_t i = nw * kE + threadIdx.x;
     const float v = sizeof(T) == 2 ? bf16_lo(reinterpret_cast<const uint16_t *>(x)[i]) : reinterpret_cast<const float *>(x)[i];
     q[i] = (uint8_t)e4m3x4(sat(v * scale), 0.f, 0.f, 0.f);
   }
   // hybrid: the streamed groups again, this workgroup's last first, kStream loads in flight
-  if (sgroups > (int64_t)blockIdx.x) {
-    const int64_t cnt = (sgroups - 1 - blockIdx.x) / G + 1;   // streamed groups of this workgroup
+  if (sgroups > blk) {
+    const int64_t cnt = (sgroups - 1 - blk) / G + 1;   // streamed groups of this workgroup
     for (int64_t k0 = cnt - 1; k0 >= 0; k0 -= kStream) {
       u32x4 S[kStream];
 #pragma unroll
       for (int k = 0; k < kStream; k++) {
-        const int64_t i = sword(blockIdx.x + (k0 - k) * G);
+        const int64_t i = sword(blk + (k0 - k) * G);
         S[k] = k0 - k >= 0 && i < nw ? __builtin_nontemporal_load(xv + map(i)) : u32x4{0u, 0u, 0u, 0u};
       }
 #pragma unroll
       for (int k = 0; k < kStream; k++) {
-        const int64_t i = sword(blockIdx.x + (k0 - k) * G);
+        const int64_t i = sword(blk + (k0 - k) * G);
         if (k0 - k >= 0 && i < nw) {
           if constexpr (sizeof(T) == 2) __builtin_nontemporal_store(cast8_bf16(S[k], scale), reinterpret_cast<u32x2 *>(q) + i);
           else __builtin_nontemporal_store(cast4_f32(S[k], scale), reinterpret_cast<uint32_t *>(q) + i);
@@ -1217,46 +1240,61 @@ __global__ __launch_bounds__(256, 4) void cast_once_kernel(const T *__restrict__
   once_done(ws, tk);
 }
 
-// Transposing single-pass cast of a bf16 source, run by the G workgroups [first, first + G) of a launch: workgroup b of
-// them holds tiles b and b + G (when there is one) in registers.
-// A larger x (at most kHybridTiles tiles) takes the same kernel as a hybrid: workgroup b's further tiles b + k G,
-// k >= 2, are streamed once for the maximum and once more, last first, for the cast, so only the part of x that does
-// not fit is read twice.
-__device__ __forceinline__ void cast_t_once_run(const uint16_t *__restrict__ x, int64_t ld, int64_t rows, int64_t cols,
+template <typename T, class Map = FlatMap>
+__global__ __launch_bounds__(256, 4) void cast_once_kernel(const T *__restrict__ x, int64_t n, int wpt,
+                                                           int64_t sgroups, uint8_t *__restrict__ q,
+                                                           float *__restrict__ dequant, void *ws,
+                                                           uint32_t wait_ticks, const Map map = Map()) {
+  const uint32_t ep = once_epoch(ws);   // (before the first loads: its latency passes behind them)
+  cast_once_run<T, Map>(x, n, wpt, sgroups, q, dequant, ws, wait_ticks, ep, blockIdx.x, gridDim.x, 0, map);
+}
+
+// Transposing single-pass cast, run by the G workgroups [first, first + G) of a launch: workgroup b of them holds
+// tiles b + h G, h < kHeldT (where there is one), in 64 registers a thread: two of bf16, one of fp32.
+// A larger x (at most kHybridTiles x as many tiles as workgroups) takes the same kernel as a hybrid: workgroup b's
+// further tiles are streamed once for the maximum and once more, last first, for the cast, so only the part of x that
+// does not fit is read twice.
+// kHyb: the hybrid's code is there (bf16 only: beside a tile of fp32 held it does not fit the 128 registers).
+template <typename T>
+constexpr int kHeldT = 16 / TileOf<T>::kW;
+template <typename T, bool kHyb>
+__device__ __forceinline__ void cast_t_once_run(const T *__restrict__ x, int64_t ld, int64_t rows, int64_t cols,
                                                 uint8_t *__restrict__ q, int64_t ldq, uint8_t *__restrict__ qt,
                                                 int64_t ldt, float *__restrict__ dequant, void *ws, uint32_t wait_ticks,
-                                                uint32_t ep, int64_t b, int64_t G, int first) {
-  static_assert(kOnceTiles == 2, "two tiles per workgroup");
-  __shared__ uint32_t tile[kTT * kTPitch];
+                                                uint32_t ep, int64_t b, int64_t G, int first, uint32_t *tile) {
+  typedef TileOf<T> L;
+  constexpr int kH = kHeldT<T>;
   const int64_t tiles_c = (cols + kTT - 1) / kTT, tiles = tiles_c * ((ldt + kTT - 1) / kTT);
-  const int64_t t0 = b, t1 = b + G;   // t0 < tiles: the grid never exceeds the tile count
   auto r0_of = [&](int64_t t) { return (t / tiles_c) * kTT; };
   auto c0_of = [&](int64_t t) { return (t % tiles_c) * kTT; };
-  u32x4 R[2 * kTPer];
-  u32x4(&R0)[kTPer] = *reinterpret_cast<u32x4(*)[kTPer]>(R);
-  u32x4(&R1)[kTPer] = *reinterpret_cast<u32x4(*)[kTPer]>(R + kTPer);
-  load_tile_bf16(x, ld, rows, cols, r0_of(t0), c0_of(t0), R0);
-  if (t1 < tiles) {
-    load_tile_bf16(x, ld, rows, cols, r0_of(t1), c0_of(t1), R1);
-  } else {
+  typedef u32x4 tile_t[L::kW];
+  u32x4 R[kH * L::kW];   // b < tiles: the grid never exceeds the tile count
 #pragma unroll
-    for (int i = 0; i < kTPer; i++) R1[i] = u32x4{0u, 0u, 0u, 0u};
+  for (int h = 0; h < kH; h++) {
+    tile_t &Rh = *reinterpret_cast<tile_t *>(R + h * L::kW);
+    if (h == 0 || b + h * G < tiles) {
+      load_tile<T>(x, ld, rows, cols, r0_of(b + h * G), c0_of(b + h * G), Rh);
+    } else {
+#pragma unroll
+      for (int i = 0; i < L::kW; i++) Rh[i] = u32x4{0u, 0u, 0u, 0u};
+    }
   }
-  uint32_t m = words_amax<uint16_t, 2 * kTPer>(R);
-  for (int64_t t = b + 2 * G; t < tiles; t += G) {   // hybrid: the tiles that are not held
-    u32x4 S[kTPer];
-    load_tile_bf16(x, ld, rows, cols, r0_of(t), c0_of(t), S);
-    m = max(m, words_amax<uint16_t, kTPer>(S));
-  }
+  uint32_t m = words_amax<T, kH * L::kW>(R);
+  if constexpr (kHyb)
+    for (int64_t t = b + kH * G; t < tiles; t += G) {   // hybrid: the tiles that are not held
+      u32x4 S[L::kW];
+      load_tile<T>(x, ld, rows, cols, r0_of(t), c0_of(t), S);
+      m = max(m, words_amax<T, L::kW>(S));
+    }
   uint32_t tk;
   const uint32_t g = once_fold_range(block_max_u32(m), ws, ep, wait_ticks, tk, first, (int)G, [&](int c) {
     uint32_t a = 0;
     for (int64_t t = c; t < tiles; t += G) {
       const int64_t r0 = r0_of(t), c0 = c0_of(t);
-      for (int i = 0; i < kTPer; i++) {
+      for (int i = 0; i < L::kW; i++) {
         const int id = threadIdx.x + 256 * i;
-        const int64_t gr = r0 + (id >> 4), gc = c0 + 8 * (id & 15);
-        if (gr < rows && gc < cols) a = max(a, word_amax_exact<uint16_t>(*reinterpret_cast<const u32x4 *>(x + gr * ld + gc)));
+        const int64_t gr = r0 + id / L::kC, gc = c0 + L::kE * (id % L::kC);
+        if (gr < rows && gc < cols) a = max(a, word_amax_exact<T>(*reinterpret_cast<const u32x4 *>(x + gr * ld + gc)));
       }
     }
     return block_max_u32(a);
@@ -1265,59 +1303,110 @@ __device__ __forceinline__ void cast_t_once_run(const uint16_t *__restrict__ x, 
   float scale, deq;
   scales_from_amax(g, scale, deq);
   if (b == 0 && threadIdx.x == 0) *dequant = deq;
-  u32x2 E0[kTPer], E1[kTPer];   // both tiles narrowed first: 32 VGPRs live instead of 64
-  cvt_tile_bf16(R0, scale, E0);
-  cvt_tile_bf16(R1, scale, E1);
+  CastWord<T> E[kH][L::kW];   // every held tile narrowed first: at most half the registers live
+#pragma unroll
+  for (int h = 0; h < kH; h++) cvt_tile<T>(*reinterpret_cast<tile_t *>(R + h * L::kW), scale, E[h]);
   // hybrid: the streamed tiles again, last first (the most recently read are the likeliest still in the MALL), the
   // next one's loads in flight while the current one is cast
-  int64_t ts = b + 2 * G;
+  int64_t ts = b + kH * G;
   if (ts < tiles) ts += ((tiles - 1 - ts) / G) * G;   // the last tile of this workgroup
-  u32x4 S[kTPer];
-  if (ts < tiles) load_tile_bf16(x, ld, rows, cols, r0_of(ts), c0_of(ts), S);
-  const int64_t u0 = opaque_s64(t0), u1 = u0 + G;
-  emit_tile(E0, r0_of(u0), c0_of(u0), rows, cols, q, ldq, qt, ldt, tile);
-  if (u1 < tiles) emit_tile(E1, r0_of(u1), c0_of(u1), rows, cols, q, ldq, qt, ldt, tile);
-  for (; ts >= 2 * G && ts < tiles; ts -= G) {
-    u32x2 E[kTPer];
-    cvt_tile_bf16(S, scale, E);
-    if (ts - G >= 2 * G) load_tile_bf16(x, ld, rows, cols, r0_of(ts - G), c0_of(ts - G), S);
-    emit_tile(E, r0_of(ts), c0_of(ts), rows, cols, q, ldq, qt, ldt, tile);
+  u32x4 S[L::kW];
+  if constexpr (kHyb)
+    if (ts < tiles) load_tile<T>(x, ld, rows, cols, r0_of(ts), c0_of(ts), S);
+  const int64_t u0 = opaque_s64(b);
+#pragma unroll
+  for (int h = 0; h < kH; h++) {
+    const int64_t u = u0 + h * G;
+    if (h == 0 || u < tiles) emit_tile<T>(E[h], r0_of(u), c0_of(u), rows, cols, q, ldq, qt, ldt, tile);
   }
+  if constexpr (kHyb)
+    for (; ts >= kH * G && ts < tiles; ts -= G) {
+      CastWord<T> Es[L::kW];
+      cvt_tile<T>(S, scale, Es);
+      if (ts - G >= kH * G) load_tile<T>(x, ld, rows, cols, r0_of(ts - G), c0_of(ts - G), S);
+      emit_tile<T>(Es, r0_of(ts), c0_of(ts), rows, cols, q, ldq, qt, ldt, tile);
+    }
   once_done(ws, tk);
 }
 
-__global__ __launch_bounds__(256, 4) void cast_t_once_kernel(const uint16_t *__restrict__ x, int64_t ld, int64_t rows,
+template <typename T>
+__global__ __launch_bounds__(256, 4) void cast_t_once_kernel(const T *__restrict__ x, int64_t ld, int64_t rows,
                                                              int64_t cols, uint8_t *__restrict__ q, int64_t ldq,
                                                              uint8_t *__restrict__ qt, int64_t ldt,
                                                              float *__restrict__ dequant, void *ws,
                                                              uint32_t wait_ticks) {
   const uint32_t ep = once_epoch(ws);   // (before the first loads: its latency passes behind them)
-  cast_t_once_run(x, ld, rows, cols, q, ldq, qt, ldt, dequant, ws, wait_ticks, ep, blockIdx.x, gridDim.x, 0);
+  __shared__ uint32_t tile[kTT * kTPitch];
+  cast_t_once_run<T, sizeof(T) == 2>(x, ld, rows, cols, q, ldq, qt, ldt, dequant, ws, wait_ticks, ep, blockIdx.x,
+                                     gridDim.x, 0, tile);
 }
 
-// Several transposing casts in one launch: tensor i takes workgroups [first[i], first[i + 1]), each holding at most
-// two of its tiles (no hybrid), and folds over its own workgroups' partials; one epoch and one done count for the
-// launch. The same bytes and scales as one cast_t_once_kernel launch per tensor.
-constexpr int kMaxTGroup = 8;
-struct TGroup {
-  const uint16_t *x[kMaxTGroup];
-  uint8_t *q[kMaxTGroup];
-  uint8_t *qt[kMaxTGroup];
-  float *dequant[kMaxTGroup];
-  int64_t rows[kMaxTGroup], cols[kMaxTGroup], ldt[kMaxTGroup];
-  int first[kMaxTGroup + 1];
-  int count;
+// Several casts in one launch, flat (qt null) or transposing, of bf16 or fp32: tensor i takes workgroups [first[i],
+// first[i + 1]) and folds over its own workgroups' partials; one epoch and one done count for the launch. Every tensor
+// is held whole (no hybrid). The same bytes and scales as one launch per tensor: what it saves is a launch's fixed time
+// (the epoch, the fold's round trips, the gap to the next), ~6 us of every small cast. The four fp32 weights of a d12
+// block: 27.3 us (100.7 MB, 3.7 TB/s; eight launches reading each weight twice: 49.1); a lone fp32 [8192 x 1024] in the
+// transposing single pass 14.4 us against 18.4 for the two passes, [1024 x 1024] 7.7 against 7.7.
+constexpr int kMaxGroup = 8;
+struct CastItem {   // 64 bytes: one scalar load
+  const void *x;
+  uint8_t *q, *qt;
+  float *dequant;
+  int64_t rows, cols, ldt;   // (a flat tensor is one row)
+  int wpt, f32;
 };
-__global__ __launch_bounds__(256, 4) void cast_t_group_kernel(const TGroup g, void *ws,
-                                                              uint32_t wait_ticks) {
+struct CastGroup {
+  int first[kMaxGroup + 1];   // (past the last tensor: the grid size)
+  CastItem item[kMaxGroup];
+};
+// kKinds: which kinds of tensor the instance holds code for (all in one kernel spill at 128 registers).
+enum { kFlat16 = 1, kFlat32 = 2, kTr16 = 4, kTr32 = 8 };
+template <int kKinds>
+__global__ __launch_bounds__(256, 4) void cast_group_kernel(const CastGroup g, void *ws, uint32_t wait_ticks) {
   const uint32_t ep = once_epoch(ws);
-  int i = 0;
-  while (i + 1 < g.count && (int)blockIdx.x >= g.first[i + 1]) i++;
-  i = __builtin_amdgcn_readfirstlane(i);
-  const int first = g.first[i];
-  cast_t_once_run(g.x[i], g.cols[i], g.rows[i], g.cols[i], g.q[i], g.cols[i], g.qt[i], g.ldt[i], g.dequant[i], ws,
-                  wait_ticks, ep, (int)blockIdx.x - first, g.first[i + 1] - first, first);
+  int i = 0, first = 0;   // (no chain of dependent loads)
+#pragma unroll
+  for (int k = 1; k < kMaxGroup; k++)
+    if ((int)blockIdx.x >= g.first[k]) {
+      i = k;
+      first = g.first[k];
+    }
+  const CastItem &p = g.item[i];
+  const int G = g.first[i + 1] - first, b = (int)blockIdx.x - first;
+  auto flat = [&](auto *x) {
+    cast_once_run(x, p.rows * p.cols, p.wpt, 0, p.q, p.dequant, ws, wait_ticks, ep, b, G, first, FlatMap());
+  };
+  auto transposing = [&](auto *x) {
+    __shared__ uint32_t tile[kTT * kTPitch];
+    cast_t_once_run<std::remove_const_t<std::remove_pointer_t<decltype(x)>>, false>(
+        x, p.cols, p.rows, p.cols, p.q, p.cols, p.qt, p.ldt, p.dequant, ws, wait_ticks, ep, b, G, first, tile);
+  };
+  const uint16_t *x16 = static_cast<const uint16_t *>(p.x);
+  const float *x32 = static_cast<const float *>(p.x);
+  constexpr bool kFlat = kKinds & (kFlat16 | kFlat32), kTr = kKinds & (kTr16 | kTr32);
+  if (kTr && (!kFlat || p.qt)) {
+    if constexpr (kKinds & kTr32) transposing(x32);
+    else if constexpr (kKinds & kTr16) transposing(x16);
+  } else if ((kKinds & kFlat32) && (!(kKinds & kFlat16) || p.f32)) {
+    if constexpr (kKinds & kFlat32) flat(x32);
+  } else {
+    if constexpr (kKinds & kFlat16) flat(x16);
+  }
 }
+typedef void (*GroupKernel)(const CastGroup, void *, uint32_t);
+// The instance for a set of kinds, or null; `slot`: its capacity's cache.
+static GroupKernel group_kernel(int kinds, int &slot) {
+  switch (kinds) {
+    case kTr16: slot = 0; return cast_group_kernel<kTr16>;
+    case kTr32: slot = 1; return cast_group_kernel<kTr32>;
+    case kFlat16: slot = 2; return cast_group_kernel<kFlat16>;
+    case kFlat16 | kFlat32: slot = 3; return cast_group_kernel<kFlat16 | kFlat32>;
+    case kFlat16 | kTr16: slot = 4; return cast_group_kernel<kFlat16 | kTr16>;
+    case kFlat16 | kTr32: slot = 5; return cast_group_kernel<kFlat16 | kTr32>;
+    default: return nullptr;
+  }
+}
+constexpr int kGroupKernels = 6;
 
 // ------------------------------------------------------------------------------------------- single-pass SwiGLU
 
@@ -1816,13 +1905,15 @@ uint32_t once_wait_ticks() { return (uint32_t)std::max(0, g_once_wait_us.load(st
 
 bool once_enabled() { return g_once_enabled.load(std::memory_order_relaxed) != 0; }
 
-static DeviceCache g_cap_flat_bf16, g_cap_flat_f32, g_cap_t, g_cap_sw, g_cap_bw, g_cap_wide, g_cap_tg, g_cap_heads,
-    g_cap_heads_wide;
+static DeviceCache g_cap_flat_bf16, g_cap_flat_f32, g_cap_t, g_cap_t32, g_cap_sw, g_cap_bw, g_cap_wide, g_cap_heads,
+    g_cap_heads_wide, g_cap_group[kGroupKernels];
 struct DeviceCacheInit {   // every slot starts at -1 (not yet computed)
   DeviceCacheInit() {
     for (int i = 0; i < kMaxDevices; i++)
-      g_cap_flat_bf16[i] = g_cap_flat_f32[i] = g_cap_t[i] = g_cap_sw[i] = g_cap_bw[i] = g_cap_wide[i] = g_cap_tg[i] =
+      g_cap_flat_bf16[i] = g_cap_flat_f32[i] = g_cap_t[i] = g_cap_t32[i] = g_cap_sw[i] = g_cap_bw[i] = g_cap_wide[i] =
           g_cap_heads[i] = g_cap_heads_wide[i] = -1;
+    for (auto &c : g_cap_group)
+      for (int i = 0; i < kMaxDevices; i++) c[i] = -1;
   }
 };
 static DeviceCacheInit g_device_cache_init;
@@ -1922,47 +2013,63 @@ static bool launch_swiglu_bwd_once(const uint16_t *z, const uint16_t *da, int64_
 }
 
 // The single-pass transposing cast of a bf16 source when it fits (false, nothing launched, otherwise).
-static bool launch_tcast_t_once(const uint16_t *x, int64_t rows, int64_t cols, uint8_t *q, uint8_t *qt, int64_t ldt,
+template <typename T>
+static bool launch_tcast_t_once(const T *x, int64_t rows, int64_t cols, uint8_t *q, uint8_t *qt, int64_t ldt,
                                 float *dequant, void *ws, hipStream_t st) {
-  const int cap = once_capacity(reinterpret_cast<const void *>(&cast_t_once_kernel), g_cap_t, 256);
+  const int cap = once_capacity(reinterpret_cast<const void *>(&cast_t_once_kernel<T>), sizeof(T) == 2 ? g_cap_t : g_cap_t32, 256);
   const int64_t tiles = ((cols + kTT - 1) / kTT) * ((ldt + kTT - 1) / kTT);
-  if (!once_enabled() || cap <= 0 || tiles <= 0 || tiles > (int64_t)kHybridTiles * cap)
+  if (!once_enabled() || cap <= 0 || tiles <= 0 || tiles > (int64_t)(sizeof(T) == 2 ? kHybridTiles : 1) * cap)
     return false;
   const int grid = (int)std::min<int64_t>(tiles, cap);
-  cast_t_once_kernel<<<grid, 256, 0, st>>>(x, cols, rows, cols, q, cols, qt, ldt, dequant, ws, once_wait_ticks());
+  cast_t_once_kernel<T><<<grid, 256, 0, st>>>(x, cols, rows, cols, q, cols, qt, ldt, dequant, ws, once_wait_ticks());
   return true;
 }
 
-// The grouped transposing cast when every tensor fits (false, nothing launched, otherwise): one tile per workgroup
-// when the tiles fit the device at once, else two.
-static bool launch_tcast_t_group(int count, const uint16_t *const *x, const int64_t *rows, const int64_t *cols,
-                                 uint8_t *const *q, uint8_t *const *qt, const int64_t *ldt, float *const *dequant,
-                                 void *ws, hipStream_t st) {
-  const int cap = once_capacity(reinterpret_cast<const void *>(&cast_t_group_kernel), g_cap_tg, 256);
-  if (!once_enabled() || cap <= 0 || count < 1 || count > kMaxTGroup) return false;
-  int64_t tiles[kMaxTGroup], all = 0, halves = 0;
-  for (int i = 0; i < count; i++) {
-    tiles[i] = ((cols[i] + kTT - 1) / kTT) * ((ldt[i] + kTT - 1) / kTT);
-    if (rows[i] <= 0 || tiles[i] <= 0) return false;
-    all += tiles[i];
-    halves += (tiles[i] + 1) / 2;
+// The grouped cast when every tensor fits (false, nothing launched, otherwise). Workgroups: a transposing tensor takes
+// one per tile, or, when that is more than the device holds, one per kHeldT tiles; a flat one enough for kFlatWords words
+// a thread, or for as many as a thread holds.
+constexpr int kFlatWords = 4;
+static bool launch_cast_group(int count, const void *const *x, const int *dtype, const int64_t *rows,
+                              const int64_t *cols, uint8_t *const *q, uint8_t *const *qt, const int64_t *ldt,
+                              float *const *dequant, void *ws, hipStream_t st) {
+  if (!once_enabled() || count < 1 || count > kMaxGroup) return false;
+  int kinds = 0, slot = 0;
+  for (int i = 0; i < count; i++)
+    kinds |= dtype[i] == GPIC_DTYPE_F32 ? (qt[i] ? kTr32 : kFlat32) : (qt[i] ? kTr16 : kFlat16);
+  const GroupKernel kernel = group_kernel(kinds, slot);
+  if (!kernel) return false;
+  const int cap = once_capacity(reinterpret_cast<const void *>(kernel), g_cap_group[slot], 256);
+  if (cap <= 0) return false;
+  CastGroup g{};
+  for (int dense = 0; dense < 2; dense++) {
+    int64_t total = 0;
+    for (int i = 0; i < count; i++) {
+      const bool f32 = dtype[i] == GPIC_DTYPE_F32;
+      if (rows[i] <= 0 || cols[i] <= 0) return false;
+      int64_t wgs;
+      int wpt = 0;
+      if (qt[i]) {
+        const int64_t tiles = ((cols[i] + kTT - 1) / kTT) * ((ldt[i] + kTT - 1) / kTT);
+        const int held = f32 ? kHeldT<float> : kHeldT<uint16_t>;
+        wgs = dense ? (tiles + held - 1) / held : tiles;
+      } else {
+        const int most = dense ? (f32 ? kOnceWords<float> : kOnceWords<uint16_t>) : kFlatWords;
+        const int64_t groups = std::max<int64_t>(1, (rows[i] * cols[i] / (f32 ? 4 : 8) + 255) / 256);   // of 256 words
+        wgs = (groups + most - 1) / most;
+        wpt = (int)((groups + wgs - 1) / wgs);
+      }
+      g.item[i] = CastItem{x[i], q[i], qt[i], dequant[i], rows[i], cols[i], ldt[i], wpt, f32};
+      total += wgs;
+      if (total > cap) break;
+      g.first[i + 1] = (int)total;
+    }
+    if (total <= cap) {
+      for (int i = count + 1; i <= kMaxGroup; i++) g.first[i] = (int)total;
+      kernel<<<(int)total, 256, 0, st>>>(g, ws, once_wait_ticks());
+      return true;
+    }
   }
-  if (halves > cap) return false;
-  TGroup g{};
-  g.count = count;
-  g.first[0] = 0;
-  for (int i = 0; i < count; i++) {
-    g.x[i] = x[i];
-    g.q[i] = q[i];
-    g.qt[i] = qt[i];
-    g.dequant[i] = dequant[i];
-    g.rows[i] = rows[i];
-    g.cols[i] = cols[i];
-    g.ldt[i] = ldt[i];
-    g.first[i + 1] = g.first[i] + (int)(all <= cap ? tiles[i] : (tiles[i] + 1) / 2);
-  }
-  cast_t_group_kernel<<<g.first[count], 256, 0, st>>>(g, ws, once_wait_ticks());
-  return true;
+  return false;
 }
 
 // ------------------------------------------------------------------------------------------- allocation-free cast
@@ -2093,12 +2200,46 @@ int gpic_fp8_tcast_t_group(int count, const void *const *x, int dtype, const int
     if (dtype != GPIC_DTYPE_BF16 && dtype != GPIC_DTYPE_F32) return GPIC_EDTYPE;
     if (!aligned16(x[i]) || (q[i] && !aligned16(q[i])) || !aligned16(qt[i]) || !aligned16(ws)) return GPIC_EALIGN;
   }
-  if (dtype == GPIC_DTYPE_BF16 &&
-      launch_tcast_t_group(count, reinterpret_cast<const uint16_t *const *>(x), rows, cols, q, qt, ldt, dequant, ws,
-                           (hipStream_t)stream))
+  int dt[kMaxGroup];
+  bool rows_ok = count <= kMaxGroup;
+  for (int i = 0; i < count && rows_ok; i++) {
+    dt[i] = dtype;
+    rows_ok = qt[i] != nullptr && rows[i] > 0 && cols[i] > 0;
+  }
+  if (rows_ok && launch_cast_group(count, x, dt, rows, cols, q, qt, ldt, dequant, ws, (hipStream_t)stream))
     return (int)hipGetLastError();
   for (int i = 0; i < count; i++) {   // otherwise one call per tensor, in order
     const int rc = gpic_fp8_tcast_t(x[i], dtype, rows[i], cols[i], q[i], qt[i], ldt[i], dequant[i], ws, stream);
+    if (rc != GPIC_OK) return rc;
+  }
+  return GPIC_OK;
+}
+
+int gpic_fp8_cast_group(int count, const void *const *x, const int *dtype, const int64_t *rows, const int64_t *cols,
+                        uint8_t *const *q, uint8_t *const *qt, const int64_t *ldt, float *const *dequant, void *ws,
+                        void *stream) {
+  status_scope();
+  if (count < 0 || (count > 0 && (!x || !dtype || !rows || !cols || !q || !qt || !ldt || !dequant || !ws)))
+    return GPIC_EINVAL;
+  int64_t r[kMaxGroup], c[kMaxGroup];   // (a flat tensor as one row)
+  bool one = count <= kMaxGroup;
+  for (int i = 0; i < count; i++) {
+    if (rows[i] < 0 || cols[i] < 0 || !dequant[i] || (rows[i] > 0 && cols[i] > 0 && (!x[i] || (!q[i] && !qt[i]))))
+      return GPIC_EINVAL;
+    if (dtype[i] != GPIC_DTYPE_BF16 && dtype[i] != GPIC_DTYPE_F32) return GPIC_EDTYPE;
+    if (qt[i] && (cols[i] % 16 != 0 || ldt[i] % 16 != 0 || ldt[i] < rows[i])) return GPIC_ESHAPE;
+    if (!aligned16(x[i]) || !aligned16(q[i]) || !aligned16(qt[i]) || !aligned16(ws)) return GPIC_EALIGN;
+    if (one && (rows[i] == 0 || cols[i] == 0)) one = false;
+    if (one) {
+      r[i] = qt[i] ? rows[i] : 1;
+      c[i] = qt[i] ? cols[i] : rows[i] * cols[i];
+    }
+  }
+  if (one && launch_cast_group(count, x, dtype, r, c, q, qt, ldt, dequant, ws, (hipStream_t)stream))
+    return (int)hipGetLastError();
+  for (int i = 0; i < count; i++) {   // otherwise one call per tensor, in order
+    const int rc = qt[i] ? gpic_fp8_tcast_t(x[i], dtype[i], rows[i], cols[i], q[i], qt[i], ldt[i], dequant[i], ws, stream)
+                         : gpic_fp8_tcast(x[i], dtype[i], rows[i] * cols[i], q[i], dequant[i], ws, stream);
     if (rc != GPIC_OK) return rc;
   }
   return GPIC_OK;
@@ -2114,8 +2255,10 @@ int gpic_fp8_tcast_t(const void *x, int dtype, int64_t rows, int64_t cols, uint8
   if (!aligned16(x) || (q && !aligned16(q)) || !aligned16(qt) || !aligned16(ws)) return GPIC_EALIGN;
   hipStream_t st = (hipStream_t)stream;
   uint32_t *partial = static_cast<uint32_t *>(ws);
-  if (dtype == GPIC_DTYPE_BF16 && rows > 0 && cols > 0 &&
-      launch_tcast_t_once(static_cast<const uint16_t *>(x), rows, cols, q, qt, ldt, dequant, ws, st))
+  if (rows > 0 && cols > 0 &&
+      (dtype == GPIC_DTYPE_BF16
+           ? launch_tcast_t_once(static_cast<const uint16_t *>(x), rows, cols, q, qt, ldt, dequant, ws, st)
+           : launch_tcast_t_once(static_cast<const float *>(x), rows, cols, q, qt, ldt, dequant, ws, st)))
     return (int)hipGetLastError();
   const int64_t n = rows * cols;
   const int ga = grid_for((n / 16 + kUnroll - 1) / kUnroll, kAmaxBlocks);

@@ -194,6 +194,53 @@ def _(xs):
     return out
 
 
+FLAT, BOTH, TRANSPOSED = 0, 1, 2   # a cast_group tensor's outputs: q; q and qt; qt
+
+
+@L.step_op("gpic::fp8_cast_group")
+def cast_group(xs: list[torch.Tensor], kinds: list[int]) -> list[torch.Tensor]:
+    """The casts of xs in one call: per tensor (q, qt, dequant) as tcast (FLAT: qt empty) or tcast_t (BOTH; TRANSPOSED: q
+    empty) gives them, in one launch where gpic_fp8_cast_group makes it one: a layer's input and its weights."""
+    L.require_gpu(*xs)
+    dev, n = xs[0].device, len(xs)
+    for x, k in zip(xs, kinds):
+        if x.device != dev:
+            raise ValueError("cast_group: every tensor must be on the same device")
+        if k != FLAT and (x.dim() != 2 or x.shape[1] % 16):
+            raise ValueError(f"tcast_t needs a 2-D tensor with a multiple of 16 columns, got {tuple(x.shape)}")
+    xc = [_prep(x) for x in xs]
+    out, rows, cols, ldt = [], [], [], []
+    for x, k in zip(xc, kinds):
+        R, C = (1, x.numel()) if k == FLAT else x.shape
+        out += [torch.empty(x.shape if k != TRANSPOSED else (0,), dtype=E4, device=dev),
+                torch.empty((0,) if k == FLAT else (C, _r16(R)), dtype=E4, device=dev),
+                torch.empty(1, dtype=torch.float32, device=dev)]
+        rows.append(R)
+        cols.append(C)
+        ldt.append(0 if k == FLAT else _r16(R))
+    arr = lambda t, v: (t * n)(*v)
+    with L.on_device(dev):
+        ws = L.cast_workspace(dev)
+        L.check(L.lib().gpic_fp8_cast_group(
+            n, arr(ctypes.c_void_p, [x.data_ptr() for x in xc]), arr(ctypes.c_int, [L.DTYPE_CODE[x.dtype] for x in xc]),
+            arr(ctypes.c_int64, rows), arr(ctypes.c_int64, cols),
+            arr(ctypes.c_void_p, [None if k == TRANSPOSED else out[3 * i].data_ptr() for i, k in enumerate(kinds)]),
+            arr(ctypes.c_void_p, [None if k == FLAT else out[3 * i + 1].data_ptr() for i, k in enumerate(kinds)]),
+            arr(ctypes.c_int64, ldt), arr(ctypes.c_void_p, [out[3 * i + 2].data_ptr() for i in range(n)]),
+            ws.data_ptr(), L.stream_ptr(dev)), "gpic_fp8_cast_group")
+    return out
+
+
+@cast_group.register_fake
+def _(xs, kinds):
+    out = []
+    for x, k in zip(xs, kinds):
+        out += [x.new_empty(x.shape if k != TRANSPOSED else (0,), dtype=E4),
+                x.new_empty((0,) if k == FLAT else (x.shape[1], _r16(x.shape[0])), dtype=E4),
+                x.new_empty(1, dtype=torch.float32)]
+    return out
+
+
 class WeightCast(tuple):
     """A weight's (q, qt, dequant) from weight_casts, which also records the weight it was cast from (its storage
     pointer and version counter, which every in-place update such as an optimizer step advances), so that a cast
@@ -601,14 +648,19 @@ def _mm(xq, sx, wq, sw, fast=True):
 
 # ------------------------------------------------------------------------------------------------ autograd
 
+def _cast_xw(x2, *ws, kind):
+    """x2's (q, dequant) and each weight's cast_group triple, cast together."""
+    o = L.call(cast_group, [x2, *ws], [FLAT] + [kind] * len(ws))
+    return o[0], o[2], *(tuple(o[3 * i:3 * i + 3]) for i in range(1, len(ws) + 1))
+
+
 class _Fp8Linear(torch.autograd.Function):
     """fp8_native.py:181-204: FP8 forward GEMM; bf16 dgrad and wgrad from the saved bf16 input and weight."""
     @staticmethod
     def forward(ctx, x, w, b):
         shape = x.shape
         x2 = x.reshape(-1, shape[-1])
-        xq, sx = L.call(tcast, x2)
-        wq, sw = L.call(tcast, w)
+        xq, sx, (wq, _, sw) = _cast_xw(x2, w, kind=FLAT)
         y = L.call(fp8_gemm, xq, sx, wq, sw, None if b is None else b.to(torch.bfloat16))
         ctx.save_for_backward(x2, w)
         ctx.has_b, ctx.shape, ctx.wdt = b is not None, shape, w.dtype
@@ -631,8 +683,10 @@ class _Fp8LinearF8(torch.autograd.Function):
     def forward(ctx, x, w, b, wcast=None):
         shape = x.shape
         x2 = x.reshape(-1, shape[-1])
-        xq, sx = L.call(tcast, x2)
-        wq, wqt, sw = L.call(tcast_t, w) if wcast is None else wcast
+        if wcast is None:
+            xq, sx, (wq, wqt, sw) = _cast_xw(x2, w, kind=BOTH)
+        else:
+            (xq, sx), (wq, wqt, sw) = L.call(tcast, x2), wcast
         y = L.call(fp8_gemm, xq, sx, wq, sw, None if b is None else b.to(torch.bfloat16))
         ctx.save_for_backward(xq, sx, wqt, sw)
         ctx.has_b, ctx.shape, ctx.wdt = b is not None, shape, w.dtype
@@ -717,11 +771,9 @@ class _Fp8MLP(torch.autograd.Function):
     def forward(ctx, x, w12, w3):
         shape = x.shape
         x2 = x.reshape(-1, shape[-1])
-        xq, sx = L.call(tcast, x2)
-        w12q, s12 = L.call(tcast, w12)
+        xq, sx, (w12q, _, s12), (w3q, _, s3) = _cast_xw(x2, w12, w3, kind=FLAT)
         z = _mm(xq, sx, w12q, s12)
         aq, sa = L.call(swiglu_tcast, z)
-        w3q, s3 = L.call(tcast, w3)
         y = _mm(aq, sa, w3q, s3)
         ctx.save_for_backward(x2, z, aq, sa, w12, w3)
         ctx.shape, ctx.dt = shape, (w12.dtype, w3.dtype)
@@ -731,11 +783,10 @@ class _Fp8MLP(torch.autograd.Function):
     def backward(ctx, dy):
         x2, z, aq, sa, w12, w3 = ctx.saved_tensors
         dy2 = dy.reshape(-1, dy.shape[-1]).to(torch.bfloat16)
-        dyq, sdy = L.call(tcast, dy2)
-        _, w3tq, s3t = L.call(tcast_t, w3, False)                  # [H, C]: the dgrad's B operand
+        # the weights' transposed bytes, the dgrads' B operands: [H, C] and [C, 2H]
+        dyq, sdy, (_, w12tq, s12t), (_, w3tq, s3t) = _cast_xw(dy2, w12, w3, kind=TRANSPOSED)
         da = _mm(dyq, sdy, w3tq, s3t, fast=False)          # [M, H]
         dz, dzq, sdz = L.call(swiglu_bwd, z, da)
-        _, w12tq, s12t = L.call(tcast_t, w12, False)               # [C, 2H]
         dx = _mm(dzq, sdz, w12tq, s12t, fast=False)        # [M, C]
         dw12 = _wgrad16(dz, x2, ctx.dt[0])
         dw3 = _wgrad16(dy2, L.call(dequant, aq, sa), ctx.dt[1])
@@ -750,11 +801,14 @@ class _Fp8MLPF8(torch.autograd.Function):
     def forward(ctx, x, w12, w3, w12cast=None, w3cast=None):
         shape = x.shape
         x2 = x.reshape(-1, shape[-1])
-        xq, sx = L.call(tcast, x2)
-        w12q, w12qt, s12 = L.call(tcast_t, w12) if w12cast is None else w12cast
+        if w12cast is None and w3cast is None:
+            xq, sx, (w12q, w12qt, s12), (w3q, w3qt, s3) = _cast_xw(x2, w12, w3, kind=BOTH)
+        else:
+            xq, sx = L.call(tcast, x2)
+            w12q, w12qt, s12 = L.call(tcast_t, w12) if w12cast is None else w12cast
+            w3q, w3qt, s3 = L.call(tcast_t, w3) if w3cast is None else w3cast
         z = L.call(fp8_gemm, xq, sx, w12q, s12)
         aq, sa = L.call(swiglu_tcast, z)
-        w3q, w3qt, s3 = L.call(tcast_t, w3) if w3cast is None else w3cast
         y = L.call(fp8_gemm, aq, sa, w3q, s3)
         ctx.save_for_backward(xq, sx, z, aq, sa, w12qt, s12, w3qt, s3)
         ctx.shape, ctx.dt = shape, (w12.dtype, w3.dtype)

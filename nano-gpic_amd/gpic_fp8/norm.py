@@ -27,8 +27,8 @@ from typing import Optional
 import torch
 
 from . import _lib as L
-from .fp8_native import (E4, Fp8LinearF8, _bias_grad, _wgrad8, fp8_gemm, fp8_linear_f8, swiglu_bwd_q, swiglu_tcast,
-                         tcast, tcast_t)
+from .fp8_native import (BOTH, E4, Fp8LinearF8, _bias_grad, _wgrad8, cast_group, fp8_gemm, fp8_linear_f8,
+                         swiglu_bwd_q, swiglu_tcast, tcast, tcast_t)
 
 
 # The widest rows the backward kernel takes (its per-column sums live in registers); the forward takes any width.
@@ -307,10 +307,9 @@ class _Fp8ResModRMSNormMLP(torch.autograd.Function):
         _check_bwd_width(C, ctx)
         xn, _, hq, sh, rstd = L.call(res_mod_rmsnorm_q, x, a, gate, w_norm, shift, scale, eps, True, False)
         hq2 = hq.view(B * N, C)
-        w12q, w12qt, s12 = L.call(tcast_t, w12)
+        w12q, w12qt, s12, w3q, w3qt, s3 = L.call(cast_group, [w12, w3], [BOTH, BOTH])
         z = L.call(fp8_gemm, hq2, sh, w12q, s12)
         aq, sa = L.call(swiglu_tcast, z)
-        w3q, w3qt, s3 = L.call(tcast_t, w3)
         y = L.call(fp8_gemm, aq, sa, w3q, s3)
         ctx.save_for_backward(xn, a, gate, w_norm, shift, scale, rstd, hq2, sh, z, aq, sa, w12qt, s12, w3qt, s3)
         ctx.dt = (w12.dtype, w3.dtype)
