@@ -7,12 +7,14 @@ torch is imported before the library is opened, so libgpic_fp8.so binds to the H
 """
 import contextlib
 import ctypes
+import importlib.util
 import os
 import threading
 
 import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libgpic_fp8.so")
+HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_gpic_host.so")
 
 _vp = ctypes.c_void_p
 _i64 = ctypes.c_int64
@@ -70,6 +72,39 @@ def lib():
             f.argtypes = args
         _lib = L
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The native host module (csrc/host.cpp), loaded once, after the library it calls."""
+    global _host
+    if _host is None:
+        lib()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python nano-gpic_amd/gpic_fp8/build.py`")
+        spec = importlib.util.spec_from_file_location("_gpic_host", HOST_PATH)
+        m = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(m)
+        _host = m
+    return _host
+
+
+def native(name, t, *args):
+    """The host module's function `name` on args (t: one of them, which says the device), or None where it does not take
+    the call: while torch.compile traces, for tensors on another device than the current one, or not of the usual form."""
+    device = t.device
+    if device.type != "cuda" or _raw_stream is None or torch.compiler.is_compiling():
+        return None
+    index = torch.cuda.current_device()
+    if device.index != index:
+        return None
+    stream = _raw_stream(index)
+    ws = _WORKSPACES.get((index, stream))
+    if ws is None:
+        ws = cast_workspace(device)
+    return getattr(_host or host(), name)(*args, index, ws.data_ptr(), stream)
 
 
 def check(status, what):

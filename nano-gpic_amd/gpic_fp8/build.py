@@ -21,8 +21,24 @@ FLAGS = [
 ]
 
 
+HOST = os.path.join(HERE, "_gpic_host.so")
+CXX = os.environ.get("CXX", "g++")
+
+
+def _host_command(out):
+    """The native host module (host.cpp): plain C++ over torch's headers, linked to the kernel library beside it."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    inc = [f for p in cpp_extension.include_paths() + [sysconfig.get_paths()["include"]] for f in ("-isystem", p)]
+    return [CXX, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+            *inc, "-o", out, os.path.join(CSRC, "host.cpp"), *[f"-L{p}" for p in cpp_extension.library_paths()],
+            "-lc10", "-ltorch_cpu", "-ltorch_python", f"-L{HERE}", "-l:libgpic_fp8.so", "-Wl,-rpath,$ORIGIN"]
+
+
 def build(verbose=False):
-    """Each source compiled to an object in its own hipcc process (in parallel), then linked into the library."""
+    """Each source compiled to an object in its own hipcc process (in parallel), then linked into the library; then the
+    host module, which links to it."""
     objdir = os.path.join(HERE, "_build")
     os.makedirs(objdir, exist_ok=True)
     compile_flags = [f for f in FLAGS if f != "-shared"]
@@ -47,6 +63,13 @@ def build(verbose=False):
     if r.returncode != 0:
         raise RuntimeError(f"hipcc link failed ({r.returncode}):\n{r.stderr[-6000:]}")
     os.replace(tmp, LIB)
+    cmd = _host_command(HOST + ".tmp")
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{CXX} failed on host.cpp ({r.returncode}):\n{r.stderr[-6000:]}")
+    os.replace(HOST + ".tmp", HOST)
     return LIB
 
 

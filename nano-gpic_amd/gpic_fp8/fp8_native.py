@@ -20,6 +20,7 @@ Phases (convert_native / convert_fp8 recipes):
 """
 from typing import Optional
 
+import contextlib
 import ctypes
 
 import torch
@@ -201,6 +202,9 @@ FLAT, BOTH, TRANSPOSED = 0, 1, 2   # a cast_group tensor's outputs: q; q and qt;
 def cast_group(xs: list[torch.Tensor], kinds: list[int]) -> list[torch.Tensor]:
     """The casts of xs in one call: per tensor (q, qt, dequant) as tcast (FLAT: qt empty) or tcast_t (BOTH; TRANSPOSED: q
     empty) gives them, in one launch where gpic_fp8_cast_group makes it one: a layer's input and its weights."""
+    o = L.native("casts", xs[0], xs, kinds)
+    if o is not None:
+        return o
     L.require_gpu(*xs)
     dev, n = xs[0].device, len(xs)
     for x, k in zip(xs, kinds):
@@ -454,6 +458,9 @@ def fp8_gemm(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Tenso
     C [M, N] bf16 = bf16(sa * sb * a @ b^T), then bf16(C + bias) when bias [N] is given.
     Replaces torch._scaled_mm(a, b.t(), scale_a=sa, scale_b=sb, out_dtype=bf16) of _mm (fp8_native.py:175-178) and the
     bias add of _Fp8Linear.forward (:189-190). `fast` (use_fast_accum) changes nothing: MFMA accumulates in fp32."""
+    c = L.native("gemm", a, a, sa, b, sb, bias)
+    if c is not None:
+        return c
     L.require_gpu(a, b, sa, sb, bias)
     a = _gemm_operand(a, "a")
     b = _gemm_operand(b, "b")
@@ -548,6 +555,9 @@ def _(a, sa, b, sb, bias=None):
 @L.step_op("gpic::fp8_wgrad")
 def fp8_wgrad(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Tensor, f32: bool) -> torch.Tensor:
     """fp8_gemm_mn(a, sa, b, sb), in fp32 when f32 (an fp32 weight's gradient, written by the GEMM itself)."""
+    c = L.native("wgrad", a, a, sa, b, sb, f32)
+    if c is not None:
+        return c
     a2, b2 = _gemm_operand_mn(a, "a"), _gemm_operand_mn(b, "b")
     (K, M), N = a2.shape, b2.shape[1]
     if not f32 or K * max(a2.stride(0), b2.stride(0)) >= 2 ** 31 or N >= 2 ** 21:
@@ -654,14 +664,36 @@ def _cast_xw(x2, *ws, kind):
     return o[0], o[2], *(tuple(o[3 * i:3 * i + 3]) for i in range(1, len(ws) + 1))
 
 
+def _linear_fwd(x2, w, b, kind):
+    """The forward of a linear: (y, xq, sx, wqt, sw), the weight cast with x in one launch (kind BOTH: wqt its transposed
+    bytes, FLAT: an empty tensor)."""
+    b = None if b is None else b.to(torch.bfloat16)
+    r = L.native("linear_fwd", x2, x2, w, b, kind == BOTH)
+    if r is not None:
+        return r
+    xq, sx, (wq, wqt, sw) = _cast_xw(x2, w, kind=kind)
+    return L.call(fp8_gemm, xq, sx, wq, sw, b), xq, sx, wqt, sw
+
+
+def _linear_bwd(dy2, xq, sx, wqt, sw, has_b, dtype):
+    """The phase-3 backward of a linear: (dx [M, K] = [M, N] . [K, N]^T, dw [N, K] = [M, N]^T . [M, K], db or None)."""
+    # (a backward that is itself recorded: the bias gradient is then a differentiable operation)
+    r = None if has_b and _recorded() else L.native("linear_bwd", dy2, dy2, xq, sx, wqt, sw, has_b, dtype == torch.float32)
+    if r is not None:
+        dx, dw, db = r
+        return dx, dw.to(dtype), None if db is None else db.to(dtype)
+    dyq, sdy = L.call(tcast, dy2)
+    dx = L.call(fp8_gemm, dyq, sdy, wqt, sw, None, False)
+    return dx, _wgrad8(dyq, sdy, xq, sx, dtype), _bias_grad(dy2, dtype) if has_b else None
+
+
 class _Fp8Linear(torch.autograd.Function):
     """fp8_native.py:181-204: FP8 forward GEMM; bf16 dgrad and wgrad from the saved bf16 input and weight."""
     @staticmethod
     def forward(ctx, x, w, b):
         shape = x.shape
         x2 = x.reshape(-1, shape[-1])
-        xq, sx, (wq, _, sw) = _cast_xw(x2, w, kind=FLAT)
-        y = L.call(fp8_gemm, xq, sx, wq, sw, None if b is None else b.to(torch.bfloat16))
+        y = _linear_fwd(x2, w, b, FLAT)[0]
         ctx.save_for_backward(x2, w)
         ctx.has_b, ctx.shape, ctx.wdt = b is not None, shape, w.dtype
         return y.view(*shape[:-1], w.shape[0])
@@ -684,10 +716,10 @@ class _Fp8LinearF8(torch.autograd.Function):
         shape = x.shape
         x2 = x.reshape(-1, shape[-1])
         if wcast is None:
-            xq, sx, (wq, wqt, sw) = _cast_xw(x2, w, kind=BOTH)
+            y, xq, sx, wqt, sw = _linear_fwd(x2, w, b, BOTH)
         else:
             (xq, sx), (wq, wqt, sw) = L.call(tcast, x2), wcast
-        y = L.call(fp8_gemm, xq, sx, wq, sw, None if b is None else b.to(torch.bfloat16))
+            y = L.call(fp8_gemm, xq, sx, wq, sw, None if b is None else b.to(torch.bfloat16))
         ctx.save_for_backward(xq, sx, wqt, sw)
         ctx.has_b, ctx.shape, ctx.wdt = b is not None, shape, w.dtype
         return y.view(*shape[:-1], w.shape[0])
@@ -696,11 +728,8 @@ class _Fp8LinearF8(torch.autograd.Function):
     def backward(ctx, dy):
         xq, sx, wqt, sw = ctx.saved_tensors
         dy2 = dy.reshape(-1, dy.shape[-1]).to(torch.bfloat16)
-        dyq, sdy = L.call(tcast, dy2)
-        dx = L.call(fp8_gemm, dyq, sdy, wqt, sw, None, False).view(ctx.shape)     # [M, N] . [K, N]^T
-        dw = _wgrad8(dyq, sdy, xq, sx, ctx.wdt)                                    # [M, N]^T . [M, K]
-        db = _bias_grad(dy2, ctx.wdt) if ctx.has_b else None
-        return dx, dw, db, None
+        dx, dw, db = _linear_bwd(dy2, xq, sx, wqt, sw, ctx.has_b, ctx.wdt)
+        return dx.view(ctx.shape), dw, db, None
 
 
 class _Fp8HeadsLinearF8(torch.autograd.Function):
@@ -724,11 +753,8 @@ class _Fp8HeadsLinearF8(torch.autograd.Function):
         xq, sx, wqt, sw = ctx.saved_tensors
         B, H, N, D = ctx.shape
         dy2 = dy.reshape(-1, dy.shape[-1]).to(torch.bfloat16)
-        dyq, sdy = L.call(tcast, dy2)
-        dx = L.call(fp8_gemm, dyq, sdy, wqt, sw, None, False)                      # [M, N] . [K, N]^T
+        dx, dw, db = _linear_bwd(dy2, xq, sx, wqt, sw, ctx.has_b, ctx.wdt)
         do = dx.view(B, N, H, D).transpose(1, 2)
-        dw = _wgrad8(dyq, sdy, xq, sx, ctx.wdt)                                    # [M, N]^T . [M, K]
-        db = _bias_grad(dy2, ctx.wdt) if ctx.has_b else None
         return do, dw, db, None
 
 
@@ -827,18 +853,25 @@ class _Fp8MLPF8(torch.autograd.Function):
         return dx.view(ctx.shape), dw12, dw3, None, None
 
 
+def _no_autocast():
+    """torch.autocast("cuda", enabled=False), where autocast is on (or torch.compile traces)."""
+    if torch.compiler.is_compiling() or torch.is_autocast_enabled("cuda"):
+        return torch.autocast("cuda", enabled=False)
+    return contextlib.nullcontext()
+
+
 def fp8_mlp(x, w12, w3):
-    with torch.autocast("cuda", enabled=False):
+    with _no_autocast():
         return _Fp8MLP.apply(x.to(torch.bfloat16), w12, w3)
 
 
 def fp8_linear(x, w, b=None):
-    with torch.autocast("cuda", enabled=False):
+    with _no_autocast():
         return _Fp8Linear.apply(x.to(torch.bfloat16), w, b)
 
 
 def fp8_swiglu_w3(z, w3):
-    with torch.autocast("cuda", enabled=False):
+    with _no_autocast():
         return _SwiGLUw3.apply(z.to(torch.bfloat16), w3)
 
 
@@ -859,7 +892,7 @@ def fp8_linear_f8(x, w, b=None, wcast=None):
     that was cast from another tensor or before w's last in-place update is refused; of a plain tuple only the
     shapes are checked. The check reads w's version counter, which in-place ops on w advance (torch.optim's updates,
     made under no_grad); writes through w.data do not (w.data has a counter of its own), so cast again after those."""
-    with torch.autocast("cuda", enabled=False):
+    with _no_autocast():
         return _Fp8LinearF8.apply(x.to(torch.bfloat16), w, b, _check_cast("wcast", w, wcast))
 
 
@@ -871,13 +904,13 @@ def fp8_heads_linear_f8(o, w, b=None, wcast=None):
         raise ValueError(f"fp8_heads_linear_f8 needs o [B, H, N, D], got {tuple(o.shape)}")
     if o.shape[1] * o.shape[3] != w.shape[1]:
         raise ValueError(f"o {tuple(o.shape)} merges to {o.shape[1] * o.shape[3]} features, w has {w.shape[1]}")
-    with torch.autocast("cuda", enabled=False):
+    with _no_autocast():
         return _Fp8HeadsLinearF8.apply(o.to(torch.bfloat16), w, b, _check_cast("wcast", w, wcast))
 
 
 def fp8_mlp_f8(x, w12, w3, w12cast=None, w3cast=None):
     """Phase 3 fp8_mlp: every GEMM of the SwiGLU MLP in FP8. w12cast / w3cast: as fp8_linear_f8's wcast."""
-    with torch.autocast("cuda", enabled=False):
+    with _no_autocast():
         return _Fp8MLPF8.apply(x.to(torch.bfloat16), w12, w3, _check_cast("w12cast", w12, w12cast),
                                _check_cast("w3cast", w3, w3cast))
 

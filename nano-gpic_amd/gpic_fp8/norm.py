@@ -27,7 +27,7 @@ from typing import Optional
 import torch
 
 from . import _lib as L
-from .fp8_native import (BOTH, E4, Fp8LinearF8, _bias_grad, _wgrad8, cast_group, fp8_gemm, fp8_linear_f8,
+from .fp8_native import (BOTH, E4, Fp8LinearF8, _linear_bwd, _no_autocast, _wgrad8, cast_group, fp8_gemm, fp8_linear_f8,
                          swiglu_bwd_q, swiglu_tcast, tcast, tcast_t)
 
 
@@ -288,11 +288,8 @@ class _Fp8ModRMSNormLinear(torch.autograd.Function):
         x, w_norm, shift, scale, rstd, hq2, sh, wqt, sw = ctx.saved_tensors
         B, N, C = x.shape
         dy2 = dy.reshape(B * N, -1).to(torch.bfloat16)
-        dyq, sdy = L.call(tcast, dy2)
-        dh = L.call(fp8_gemm, dyq, sdy, wqt, sw, None, False).view(B, N, C)
-        dweight = _wgrad8(dyq, sdy, hq2, sh, ctx.wdt)
-        db = _bias_grad(dy2, ctx.wdt) if ctx.has_b else None
-        dx, _, _, dw, dsh, dsc = _norm_backward(dh, None, x, None, None, w_norm, scale, rstd)
+        dh, dweight, db = _linear_bwd(dy2, hq2, sh, wqt, sw, ctx.has_b, ctx.wdt)
+        dx, _, _, dw, dsh, dsc = _norm_backward(dh.view(B, N, C), None, x, None, None, w_norm, scale, rstd)
         _, dw, dshift, dscale = _param_grads(B, C, None, dw, dsh, dsc, None, w_norm, shift, scale)
         return dx, dw, dshift, dscale, None, dweight, db
 
@@ -333,14 +330,14 @@ class _Fp8ResModRMSNormMLP(torch.autograd.Function):
 
 def fp8_mod_rmsnorm_linear(x, w_norm, shift, scale, eps, weight, bias: Optional[torch.Tensor] = None):
     """linear(mod_rmsnorm(x, w_norm, shift, scale, eps)) with every GEMM in FP8 and the cast of h in the norm."""
-    with torch.autocast("cuda", enabled=False):
+    with _no_autocast():
         return _Fp8ModRMSNormLinear.apply(x.to(torch.bfloat16), w_norm, shift, scale, eps, weight, bias)
 
 
 def fp8_res_mod_rmsnorm_mlp(x, a, gate, w_norm, shift, scale, eps, w12, w3):
     """(x_new, mlp(h)) for x_new, h = res_mod_rmsnorm(x, a, gate, w_norm, shift, scale, eps), the SwiGLU MLP in FP8
     (every GEMM) and the cast of h in the norm."""
-    with torch.autocast("cuda", enabled=False):
+    with _no_autocast():
         return _Fp8ResModRMSNormMLP.apply(x.to(torch.bfloat16), a.to(torch.bfloat16), gate, w_norm, shift, scale, eps,
                                           w12, w3)
 

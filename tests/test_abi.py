@@ -160,3 +160,24 @@ def test_loader_fails_loudly_without_library(monkeypatch, tmp_path):
     monkeypatch.setattr(L, "_lib", None)
     with pytest.raises(RuntimeError, match="no CPU fallback"):
         L.lib()
+
+
+def test_host_module_takes_no_cpu_tensors():
+    """The native host module loads beside the library and leaves every tensor that is not on the current GPU to the
+    general form."""
+    import torch
+    h = L.host()
+    x, w = torch.zeros(16, 16, dtype=torch.bfloat16), torch.zeros(16, 16)
+    q, s = torch.zeros(16, 16).to(torch.float8_e4m3fn), torch.ones(1)
+    assert h.casts([x, w], [0, 1], 0, 0, 0) is None
+    assert h.gemm(q, s, q, s, None, 0, 0, 0) is None and h.wgrad(q, s, q, s, True, 0, 0, 0) is None
+    assert h.linear_fwd(x, w, None, True, 0, 0, 0) is None
+    assert h.linear_bwd(x, q, s, q, s, False, True, 0, 0, 0) is None
+    assert L.native("linear_fwd", x, x, w, None, True) is None
+
+
+def test_missing_host_module_is_an_error(monkeypatch, tmp_path):
+    monkeypatch.setattr(L, "HOST_PATH", str(tmp_path / "missing.so"))
+    monkeypatch.setattr(L, "_host", None)
+    with pytest.raises(RuntimeError, match="missing"):
+        L.host()
