@@ -1075,6 +1075,8 @@ template <typename T>
 constexpr int kOnceWords = sizeof(T) == 2 ? 16 : 12;   // 16-byte words a thread of the flat kernel holds (fp32: 12,
                                                         // which its wider narrowing code needs to fit 128 VGPRs)
 constexpr int kHybridTiles = 8;     // the transposing kernel takes up to this many tiles per workgroup (bf16: 2 held, fp32: 1)
+constexpr int kFlatWords = 4;       // words a thread of the flat kernel takes at least: fewer workgroups fold faster
+                                    // (bf16 [2048 x 2048]: 6.8 us against 8.0 with one; no gain from 8)
 constexpr int kHybridFlat = 8;      // the flat kernel takes up to this many times the words it can hold
 constexpr int kStream = 8;          // streamed words in flight per thread (flat hybrid)
 
@@ -1960,7 +1962,7 @@ static bool launch_tcast_once(const T *x, int64_t n, uint8_t *q, float *dequant,
     return true;
   }
   const int64_t groups = std::max<int64_t>(1, (nw + 255) / 256);   // 256-word groups
-  const int grid = (int)std::min<int64_t>(groups, cap);
+  const int grid = (int)std::min<int64_t>((groups + kFlatWords - 1) / kFlatWords, cap);
   const int wpt = (int)((groups + grid - 1) / grid);
   cast_once_kernel<T, Map><<<grid, 256, 0, st>>>(x, n, wpt, 0, q, dequant, ws, once_wait_ticks(), map);
   return true;
@@ -2026,9 +2028,8 @@ static bool launch_tcast_t_once(const T *x, int64_t rows, int64_t cols, uint8_t 
 }
 
 // The grouped cast when every tensor fits (false, nothing launched, otherwise). Workgroups: a transposing tensor takes
-// one per tile, or, when that is more than the device holds, one per kHeldT tiles; a flat one enough for kFlatWords words
-// a thread, or for as many as a thread holds.
-constexpr int kFlatWords = 4;
+// one per tile, or, when that is more than the device holds, one per kHeldT tiles; a flat one as many as give a thread
+// kFlatWords words, or the next larger number of words with which everything fits.
 static bool launch_cast_group(int count, const void *const *x, const int *dtype, const int64_t *rows,
                               const int64_t *cols, uint8_t *const *q, uint8_t *const *qt, const int64_t *ldt,
                               float *const *dequant, void *ws, hipStream_t st) {
@@ -2041,9 +2042,13 @@ static bool launch_cast_group(int count, const void *const *x, const int *dtype,
   const int cap = once_capacity(reinterpret_cast<const void *>(kernel), g_cap_group[slot], 256);
   if (cap <= 0) return false;
   CastGroup g{};
-  for (int dense = 0; dense < 2; dense++) {
+  const int most = !(kinds & (kFlat16 | kFlat32)) ? kFlatWords : kinds & kFlat32 ? kOnceWords<float> : kOnceWords<uint16_t>;
+  // tried in turn: kFlatWords..most words a thread with one tile per workgroup, then the same with kHeldT tiles
+  for (int k = 0; k < 2 * (most - kFlatWords + 1); k++) {
+    const bool dense = k > most - kFlatWords;
+    const int words = kFlatWords + k % (most - kFlatWords + 1);
     int64_t total = 0;
-    for (int i = 0; i < count; i++) {
+    for (int i = 0; i < count && total <= cap; i++) {
       const bool f32 = dtype[i] == GPIC_DTYPE_F32;
       if (rows[i] <= 0 || cols[i] <= 0) return false;
       int64_t wgs;
@@ -2053,14 +2058,13 @@ static bool launch_cast_group(int count, const void *const *x, const int *dtype,
         const int held = f32 ? kHeldT<float> : kHeldT<uint16_t>;
         wgs = dense ? (tiles + held - 1) / held : tiles;
       } else {
-        const int most = dense ? (f32 ? kOnceWords<float> : kOnceWords<uint16_t>) : kFlatWords;
         const int64_t groups = std::max<int64_t>(1, (rows[i] * cols[i] / (f32 ? 4 : 8) + 255) / 256);   // of 256 words
-        wgs = (groups + most - 1) / most;
+        wgs = (groups + words - 1) / words;
         wpt = (int)((groups + wgs - 1) / wgs);
       }
-      g.item[i] = CastItem{x[i], q[i], qt[i], dequant[i], rows[i], cols[i], ldt[i], wpt, f32};
       total += wgs;
       if (total > cap) break;
+      g.item[i] = CastItem{x[i], q[i], qt[i], dequant[i], rows[i], cols[i], ldt[i], wpt, f32};
       g.first[i + 1] = (int)total;
     }
     if (total <= cap) {
@@ -2235,7 +2239,8 @@ int gpic_fp8_cast_group(int count, const void *const *x, const int *dtype, const
       c[i] = qt[i] ? cols[i] : rows[i] * cols[i];
     }
   }
-  if (one && launch_cast_group(count, x, dtype, r, c, q, qt, ldt, dequant, ws, (hipStream_t)stream))
+  // (one tensor: the per-tensor call, which also has the kernel for the largest flat ones)
+  if (one && count > 1 && launch_cast_group(count, x, dtype, r, c, q, qt, ldt, dequant, ws, (hipStream_t)stream))
     return (int)hipGetLastError();
   for (int i = 0; i < count; i++) {   // otherwise one call per tensor, in order
     const int rc = qt[i] ? gpic_fp8_tcast_t(x[i], dtype[i], rows[i], cols[i], q[i], qt[i], ldt[i], dequant[i], ws, stream)
