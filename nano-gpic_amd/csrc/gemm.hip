@@ -613,6 +613,114 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
   }
 }
 
+// The small class, K-major e4m3 only: one tile of kSM x kSN per workgroup of 4 waves (2 x 2, each half the tile's sides),
+// for shapes whose 256 x 128 tiles leave most CUs idle (a few hundred to a few thousand rows). There a tile's time is
+// latency, not rate: the ping-pong spends ~1 us on each K tile of its 48 KiB however few workgroups run. Here kSS stages
+// of K = 128 are in flight, one barrier per K tile, several workgroups share a CU's 160 KiB of LDS and hide one another's
+// waits, and a lane stores its runs of 8 columns (col_of, as above) straight from the accumulators. The K tiles are
+// summed in the same order with the same instruction, so an unsplit result has the same bits as the other classes'.
+template <int kSM, int kSN, int kSS, bool kTail>
+__global__ __launch_bounds__(256) void gemm_small_kernel(const uint8_t *__restrict__ A, int lda,
+                                                         const uint8_t *__restrict__ B, int ldb,
+                                                         const float *__restrict__ sa, const float *__restrict__ sb,
+                                                         const uint16_t *__restrict__ bias, uint16_t *__restrict__ C,
+                                                         int64_t ldc, int M, int N, int K, int tiles_n) {
+  constexpr int kA = kSM * kBK, kStage = (kSM + kSN) * kBK;   // bytes of a stage's A part, of a stage
+  constexpr int kLA = kSM / 32, kLB = kSN / 32, kL = kLA + kLB;   // loads per wave and K tile: 8 rows each
+  constexpr int kFM = kSM / 32, kFN = kSN / 32;               // 16 x 16 tiles per wave
+  static_assert(kFN % 2 == 0 && kSS >= 3 && (kSS - 2) * kL < 64, "pairs of 16-column tiles; vmcnt is 6 bits");
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kSS * kStage];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int lid = xcd_remap(blockIdx.x, gridDim.x);
+  const int m0 = (lid / tiles_n) * kSM, n0 = (lid % tiles_n) * kSN;
+  const int nk = (K + kBK - 1) / kBK;
+  const v4i rA = buffer_rsrc(A + (int64_t)m0 * lda, min(M - m0, kSM) * lda);
+  const v4i rB = buffer_rsrc(B + (int64_t)n0 * ldb, min(N - n0, kSN) * ldb);
+  // load i of a wave fills LDS rows 32 i + 8 wave + lane / 8; swz and col_of of a row do not depend on i beyond + 32 i
+  const int lrow = wave * 8 + (lane >> 3);
+  const int kchunk = 16 * ((lane & 7) ^ swz(lrow));
+  const int baseA = lrow * lda + kchunk, baseB = col_of(lrow) * ldb + kchunk;
+  auto send = [&](int kt) {
+    const int k0 = kt * kBK;
+    const uint32_t to = lds_addr(smem) + (kt % kSS) * kStage + wave * 8 * kBK;
+    const bool in = !kTail || k0 + kchunk < K;   // the last, partial K tile: chunks past K read zeros
+#pragma unroll
+    for (int i = 0; i < kLA; i++) {
+      const int vo = baseA + 32 * i * lda;
+      if (kTail) lds_dma16(rA, in ? vo + k0 : kOOB, 0, to + 32 * i * kBK);
+      else lds_dma16(rA, vo, k0, to + 32 * i * kBK);
+    }
+#pragma unroll
+    for (int i = 0; i < kLB; i++) {
+      const int vo = baseB + 32 * i * ldb;
+      if (kTail) lds_dma16(rB, in ? vo + k0 : kOOB, 0, to + kA + 32 * i * kBK);
+      else lds_dma16(rB, vo, k0, to + kA + 32 * i * kBK);
+    }
+  };
+#pragma unroll
+  for (int kt = 0; kt < kSS - 1; kt++)
+    if (kt < nk) send(kt);
+  v4f acc[kFN][kFM];
+#pragma unroll
+  for (int i = 0; i < kFN; i++)
+#pragma unroll
+    for (int j = 0; j < kFM; j++) acc[i][j] = v4f{};
+  const int frow = lane & 15, fsw = swz(frow), c0 = 2 * (lane >> 4);
+  const int lo = 16 * (c0 ^ fsw), hi = 16 * ((c0 + 1) ^ fsw);
+  for (int kt = 0; kt < nk; kt++) {
+    // K tile kt has landed when at most the loads of the tiles sent after it (kSS - 2, fewer at the end) are in flight;
+    // every wave waits for its own and meets the others, which also says that all have read the stage sent next
+    const int after = min(kSS - 2, nk - 1 - kt);
+    if (after == kSS - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kSS - 2) * kL) : "memory");
+    else if (kSS > 3 && after == kSS - 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kSS - 3) * kL) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (kt + kSS - 1 < nk) send(kt + kSS - 1);
+    const GPIC_LDS uint8_t *st = (const GPIC_LDS uint8_t *)smem + (kt % kSS) * kStage;
+    auto frag = [&](int row) {
+      const GPIC_LDS uint8_t *p = st + (row + frow) * kBK;
+      const u32x4 x0 = *(const GPIC_LDS u32x4 *)(p + lo), x1 = *(const GPIC_LDS u32x4 *)(p + hi);
+      return v8i{(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w, (int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
+    };
+    v8i fa[kFM], fb[kFN];
+#pragma unroll
+    for (int j = 0; j < kFM; j++) fa[j] = frag(wm * (kSM / 2) + 16 * j);
+#pragma unroll
+    for (int j = 0; j < kFN; j++) fb[j] = frag(kSM + wn * (kSN / 2) + 16 * j);
+#pragma unroll
+    for (int ni = 0; ni < kFN; ni++)
+#pragma unroll
+      for (int mi = 0; mi < kFM; mi++)
+        acc[ni][mi] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[ni], fa[mi], acc[ni][mi], 0, 0, 0, 0, 0, 0);
+  }
+  const float s = sa[0] * sb[0];
+#pragma unroll
+  for (int p = 0; p < kFN / 2; p++) {
+    const int n = n0 + wn * (kSN / 2) + 32 * p + 8 * (lane >> 4);   // 8 columns (N % 16 == 0: all inside or none)
+    u32x4 b{0u, 0u, 0u, 0u};
+    if (bias && n < N) {
+      const u32x2 b0 = *reinterpret_cast<const u32x2 *>(bias + n), b1 = *reinterpret_cast<const u32x2 *>(bias + n + 4);
+      b = u32x4{b0.x, b0.y, b1.x, b1.y};
+    }
+#pragma unroll
+    for (int mi = 0; mi < kFM; mi++) {
+      const int m = m0 + wm * (kSM / 2) + 16 * mi + frow;
+      const v4f &x = acc[2 * p][mi], &y = acc[2 * p + 1][mi];
+      u32x4 w{pack_bf16(x[0] * s, x[1] * s), pack_bf16(x[2] * s, x[3] * s), pack_bf16(y[0] * s, y[1] * s),
+              pack_bf16(y[2] * s, y[3] * s)};
+      if (bias) {   // bf16(bf16(acc * s) + bias)
+#pragma unroll
+        for (int e = 0; e < 4; e++) w[e] = pack_bf16(bf16_lo(w[e]) + bf16_lo(b[e]), bf16_hi(w[e]) + bf16_hi(b[e]));
+      }
+      if (m < M && n < N) *reinterpret_cast<u32x4 *>(C + m * ldc + n) = w;
+    }
+  }
+}
+
 // Sum of the split-K partials in split order, then the same epilogue as the single-pass kernel.
 // (sa, sb null: unscaled bf16 operands; CT float: the bf16-rounded results in fp32, no bias.)
 template <typename CT>
@@ -702,6 +810,34 @@ static Plan plan_gemm(int64_t M, int64_t N, int64_t K) {
   return ktiles > 0 && tbest[1] < kNarrowGain * tbest[0] ? best[1] : best[0];
 }
 
+template <int kSM, int kSN, int kSS>
+static void launch_small(const void *A, int64_t lda, const float *sa, const void *B, int64_t ldb, const float *sb,
+                         const uint16_t *bias, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+  const int tiles_n = (int)((N + kSN - 1) / kSN), tiles = (int)((M + kSM - 1) / kSM) * tiles_n;
+  auto *kernel = K % kBK ? gemm_small_kernel<kSM, kSN, kSS, true> : gemm_small_kernel<kSM, kSN, kSS, false>;
+  kernel<<<tiles, 256, 0, st>>>(static_cast<const uint8_t *>(A), (int)lda, static_cast<const uint8_t *>(B), (int)ldb, sa,
+                                sb, bias, C, ldc, (int)M, (int)N, (int)K, tiles_n);
+}
+
+// The small class where its tiles are few enough for the device (false, nothing launched, otherwise). Only unsplit
+// plans: a shape whose plan splits K keeps its partials and their order, which the MN-major layout shares. The limits are
+// where each tile stopped being the fastest, device time at K = 1024 (tiles per CU in brackets):
+//   [512 x 1024] 32 x 64 4.1 us (1), 64 x 64 4.8, 256 x 128 10.1;   [1024 x 1024] 4.7 (2), 5.0, 10.3
+//   [1024 x 3072] 32 x 64 9.7 (6), 64 x 64 7.7 (3), 128 x 64 8.2, 256 x 128 10.7;   [2048 x 1024] 7.6, 5.9 (2), 6.6, 10.2
+//   [4096 x 1024] 64 x 64 9.9 (4), 128 x 64 8.4 (2), 128 x 128 9.2, 256 x 128 11.0
+//   [2048 x 3072] 64 x 64 13.0 (6), 128 x 64 13.0 (3), 256 x 128 11.7: past these the bytes a small tile reads per flop
+//   (through L2) cost more than its latency saves.
+static bool launch_small_class(const void *A, int64_t lda, const float *sa, const void *B, int64_t ldb, const float *sb,
+                               const uint16_t *bias, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K,
+                               hipStream_t st) {
+  const int64_t cus = num_cus(), n64 = (N + 63) / 64;
+  if ((M + 31) / 32 * n64 <= 2 * cus) launch_small<32, 64, 4>(A, lda, sa, B, ldb, sb, bias, C, ldc, M, N, K, st);
+  else if ((M + 63) / 64 * n64 <= 3 * cus) launch_small<64, 64, 3>(A, lda, sa, B, ldb, sb, bias, C, ldc, M, N, K, st);
+  else if ((M + 127) / 128 * n64 <= 2 * cus) launch_small<128, 64, 3>(A, lda, sa, B, ldb, sb, bias, C, ldc, M, N, K, st);
+  else return false;
+  return true;
+}
+
 // The launch shared by the operand layouts and types (arguments checked by the entry points; kEl and kC32 as the
 // kernel's). lda, ldb and K in elements.
 template <bool kMN, int kEl = 1, typename CT = uint16_t>
@@ -715,6 +851,10 @@ static int launch_gemm(const void *A, int64_t lda, const float *sa, const void *
   // (a K tile is 128 bytes of each operand's K: the plan of a byte matrix kEl times as long)
   Plan p = K > 0 ? plan_gemm(M, N, K * kEl) : Plan{(int)((M + kBM - 1) / kBM), (int)((N + kBN - 1) / kBN), 1, kBK, kBN};
   float *P = nullptr;
+  if constexpr (!kMN && kEl == 1) {
+    if (K > 0 && p.splits == 1 && launch_small_class(A, lda, sa, B, ldb, sb, bias, C, ldc, M, N, K, st))
+      return (int)hipGetLastError();
+  }
   if (p.splits > 1) {
     const size_t need = (size_t)p.splits * M * N * sizeof(float);
     if (!ws || ws_bytes < need) return GPIC_EWORKSPACE;

@@ -1,0 +1,36 @@
+"""The small GEMM class: the same bits as the 256-wide classes' summation order (the MN-major kernel on the transposed
+bytes, which never takes it), at the edges of its tiles (32 x 64, 64 x 64, 128 x 64), partial K tiles, one to many K
+tiles of its ring of stages, with bias and padded rows, and within the elementwise bound of the float64 product."""
+import pytest
+import torch
+
+import gpic_fp8 as G
+from parity import assert_elementwise
+
+pytestmark = pytest.mark.gpu
+
+# the last of each group lies just past the class's limit (256 CUs)
+SHAPES = [(1, 16, 16), (31, 48, 128), (33, 80, 144), (32, 64, 256), (512, 1024, 384), (511, 1008, 400), (512, 1024, 1024),
+          (1025, 1024, 512), (1024, 3072, 640), (4096, 768, 768), (4095, 784, 784), (4097, 1024, 1024), (2048, 1792, 1792),
+          (4096, 1040, 1040), (2049, 3072, 1024)]
+
+
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_small_gemm(dev, M, N, K, bias):
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    def operand(r):   # rows of a wider buffer, whose padding holds NaN bytes
+        buf = torch.full((r, K + 16), 0x7f, dtype=torch.uint8, device=dev)
+        buf[:, :K] = torch.randn(r, K, generator=g, device=dev).to(G.E4).view(torch.uint8)
+        return buf.view(G.E4)[:, :K]
+    a, b = operand(M), operand(N)
+    sa, sb = torch.tensor([0.37], device=dev), torch.tensor([1.9], device=dev)
+    bi = torch.randn(N, generator=g, device=dev).to(torch.bfloat16) if bias else None
+    y = G.fp8_gemm(a, sa, b, sb, bi)
+    if not bias:
+        assert_elementwise(y, a, sa.item(), b, sb.item())
+    # the MN-major kernel takes columns in multiples of 16
+    m16 = M // 16 * 16
+    if m16:
+        t = lambda u: u.contiguous().view(torch.uint8).t().contiguous().view(G.E4)
+        assert torch.equal(y[:m16], G.fp8_gemm_mn(t(a[:m16]), sa, t(b), sb, bi))
