@@ -257,6 +257,14 @@ int gpic_fp8_res_mod_rmsnorm_bwd(const uint16_t *dh, const uint16_t *dxn, const 
                                  float *dshift, float *dscale, float *dgate, float *dw, void *ws, size_t ws_bytes,
                                  void *stream);
 
+/* gpic_fp8_res_mod_rmsnorm_bwd with d_shift, d_scale and d_gate in bf16 (each fp32 sum rounded once): the gradients of a
+ * bf16 modulation, without a conversion launch each. */
+int gpic_fp8_res_mod_rmsnorm_bwd16(const uint16_t *dh, const uint16_t *dxn, const uint16_t *xs, const uint16_t *a,
+                                   const uint16_t *gate, int64_t sg, const float *w, const uint16_t *scale, int64_t ssc,
+                                   const float *rstd, int64_t rows, int64_t ntok, int64_t C, uint16_t *dx, uint16_t *da,
+                                   uint16_t *dshift, uint16_t *dscale, uint16_t *dgate, float *dw, void *ws,
+                                   size_t ws_bytes, void *stream);
+
 /* Bytes of workspace gpic_fp8_gemm needs for this problem (0 when it runs without split-K). */
 size_t gpic_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 
@@ -276,6 +284,14 @@ size_t gpic_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int gpic_fp8_gemm(const uint8_t *A, int64_t lda, const float *sa, const uint8_t *B, int64_t ldb, const float *sb,
                   const uint16_t *bias, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K, int fast_accum,
                   void *ws, size_t ws_bytes, void *stream);
+
+/*
+ * gpic_fp8_gemm with an fp32 bias (16-byte aligned), rounded to bf16 as the bias is read: `b.to(bfloat16)` of
+ * fp8_native.py:190 without a launch of its own.
+ */
+int gpic_fp8_gemm_bias32(const uint8_t *A, int64_t lda, const float *sa, const uint8_t *B, int64_t ldb, const float *sb,
+                         const float *bias, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K, void *ws,
+                         size_t ws_bytes, void *stream);
 
 /*
  * Scaled FP8 GEMM with both operands "MN-major" (K is their row index): the weight gradient straight from the

@@ -140,6 +140,19 @@ __device__ __forceinline__ int opaque_v(int v) {
   return v;
 }
 
+// The bias of columns n .. n + 7 (n % 8 == 0) as packed bf16; an fp32 bias (f32) is rounded here, as .to(bfloat16) rounds
+// it, which saves the conversion's launch.
+__device__ __forceinline__ u32x4 bias8(const void *bias, bool f32, int n) {
+  if (f32) {
+    const v4f *p = reinterpret_cast<const v4f *>(static_cast<const float *>(bias) + n);
+    const v4f x = p[0], y = p[1];
+    return u32x4{pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]), pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3])};
+  }
+  const u32x2 *p = reinterpret_cast<const u32x2 *>(static_cast<const uint16_t *>(bias) + n);
+  const u32x2 x = p[0], y = p[1];
+  return u32x4{x.x, x.y, y.x, y.y};
+}
+
 // Half h of a 32-byte fragment as a bf16 MFMA operand.
 __device__ __forceinline__ v8bf frag16(const v8i &f, int h) {
   return __builtin_bit_cast(v8bf, v4i{f[4 * h], f[4 * h + 1], f[4 * h + 2], f[4 * h + 3]});
@@ -171,7 +184,7 @@ template <bool kTail, bool kMN, int kBNt, int kEl = 1, bool kC32 = false, typena
 __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__restrict__ A, int lda,
                                                             const uint8_t *__restrict__ B, int ldb,
                                                             const float *__restrict__ sa, const float *__restrict__ sb,
-                                                            const uint16_t *__restrict__ bias, CT *__restrict__ C,
+                                                            const void *__restrict__ bias, int bias32, CT *__restrict__ C,
                                                             int64_t ldc, float *__restrict__ P, int M, int N, int K,
                                                             int ksplit, int tiles_m, int tiles_n, int splits) {
   static_assert(kBNt == 256 || kBNt == 128, "tile widths: 256 or 128");
@@ -546,8 +559,9 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
       const int n = cur.n0 + wn * kWTNt + kCol * rc;   // the read-back lane's columns
       uint32_t b[4] = {0, 0, 0, 0};
       if (!kC32 && bias && n < N) {
-        const u32x2 b0 = *reinterpret_cast<const u32x2 *>(bias + n), b1 = *reinterpret_cast<const u32x2 *>(bias + n + 4);
-        b[0] = b0.x, b[1] = b0.y, b[2] = b1.x, b[3] = b1.y;
+        const u32x4 v = bias8(bias, bias32, n);
+#pragma unroll
+        for (int e = 0; e < 4; e++) b[e] = v[e];
       }
 #pragma unroll
       for (int mq = 0; mq < kTM / 2; mq++) {
@@ -623,8 +637,9 @@ template <int kSM, int kSN, int kSS, bool kTail>
 __global__ __launch_bounds__(256) void gemm_small_kernel(const uint8_t *__restrict__ A, int lda,
                                                          const uint8_t *__restrict__ B, int ldb,
                                                          const float *__restrict__ sa, const float *__restrict__ sb,
-                                                         const uint16_t *__restrict__ bias, uint16_t *__restrict__ C,
-                                                         int64_t ldc, int M, int N, int K, int tiles_n) {
+                                                         const void *__restrict__ bias, int bias32,
+                                                         uint16_t *__restrict__ C, int64_t ldc, int M, int N, int K,
+                                                         int tiles_n) {
   constexpr int kA = kSM * kBK, kStage = (kSM + kSN) * kBK;   // bytes of a stage's A part, of a stage
   constexpr int kLA = kSM / 32, kLB = kSN / 32, kL = kLA + kLB;   // loads per wave and K tile: 8 rows each
   constexpr int kFM = kSM / 32, kFN = kSN / 32;               // 16 x 16 tiles per wave
@@ -702,10 +717,7 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(const uint8_t *__restri
   for (int p = 0; p < kFN / 2; p++) {
     const int n = n0 + wn * (kSN / 2) + 32 * p + 8 * (lane >> 4);   // 8 columns (N % 16 == 0: all inside or none)
     u32x4 b{0u, 0u, 0u, 0u};
-    if (bias && n < N) {
-      const u32x2 b0 = *reinterpret_cast<const u32x2 *>(bias + n), b1 = *reinterpret_cast<const u32x2 *>(bias + n + 4);
-      b = u32x4{b0.x, b0.y, b1.x, b1.y};
-    }
+    if (bias && n < N) b = bias8(bias, bias32, n);
 #pragma unroll
     for (int mi = 0; mi < kFM; mi++) {
       const int m = m0 + wm * (kSM / 2) + 16 * mi + frow;
@@ -726,8 +738,8 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(const uint8_t *__restri
 template <typename CT>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ P, int splits, int M, int N,
                                                             const float *__restrict__ sa, const float *__restrict__ sb,
-                                                            const uint16_t *__restrict__ bias, CT *__restrict__ C,
-                                                            int64_t ldc) {
+                                                            const void *__restrict__ bias, int bias32,
+                                                            CT *__restrict__ C, int64_t ldc) {
   const int64_t quads = (int64_t)M * (N / 4);
   const float s = sa ? sa[0] * sb[0] : 1.0f;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < quads; i += (int64_t)gridDim.x * blockDim.x) {
@@ -737,7 +749,13 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restr
     for (int z = 1; z < splits; z++) sum += *reinterpret_cast<const v4f *>(P + ((int64_t)z * M + m) * N + n);
     u32x2 w{pack_bf16(sum[0] * s, sum[1] * s), pack_bf16(sum[2] * s, sum[3] * s)};
     if (bias) {   // the output is rounded, then the bias add is rounded again
-      const u32x2 bw = *reinterpret_cast<const u32x2 *>(bias + n);
+      u32x2 bw;
+      if (bias32) {
+        const v4f x = *reinterpret_cast<const v4f *>(static_cast<const float *>(bias) + n);
+        bw = u32x2{pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3])};
+      } else {
+        bw = *reinterpret_cast<const u32x2 *>(static_cast<const uint16_t *>(bias) + n);
+      }
       w.x = pack_bf16(bf16_lo(w.x) + bf16_lo(bw.x), bf16_hi(w.x) + bf16_hi(bw.x));
       w.y = pack_bf16(bf16_lo(w.y) + bf16_lo(bw.y), bf16_hi(w.y) + bf16_hi(bw.y));
     }
@@ -812,11 +830,12 @@ static Plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 
 template <int kSM, int kSN, int kSS>
 static void launch_small(const void *A, int64_t lda, const float *sa, const void *B, int64_t ldb, const float *sb,
-                         const uint16_t *bias, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+                         const void *bias, int bias32, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K,
+                         hipStream_t st) {
   const int tiles_n = (int)((N + kSN - 1) / kSN), tiles = (int)((M + kSM - 1) / kSM) * tiles_n;
   auto *kernel = K % kBK ? gemm_small_kernel<kSM, kSN, kSS, true> : gemm_small_kernel<kSM, kSN, kSS, false>;
   kernel<<<tiles, 256, 0, st>>>(static_cast<const uint8_t *>(A), (int)lda, static_cast<const uint8_t *>(B), (int)ldb, sa,
-                                sb, bias, C, ldc, (int)M, (int)N, (int)K, tiles_n);
+                                sb, bias, bias32, C, ldc, (int)M, (int)N, (int)K, tiles_n);
 }
 
 // The small class where its tiles are few enough for the device (false, nothing launched, otherwise). Only unsplit
@@ -828,12 +847,12 @@ static void launch_small(const void *A, int64_t lda, const float *sa, const void
 //   [2048 x 3072] 64 x 64 13.0 (6), 128 x 64 13.0 (3), 256 x 128 11.7: past these the bytes a small tile reads per flop
 //   (through L2) cost more than its latency saves.
 static bool launch_small_class(const void *A, int64_t lda, const float *sa, const void *B, int64_t ldb, const float *sb,
-                               const uint16_t *bias, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K,
+                               const void *bias, int bias32, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K,
                                hipStream_t st) {
   const int64_t cus = num_cus(), n64 = (N + 63) / 64;
-  if ((M + 31) / 32 * n64 <= 2 * cus) launch_small<32, 64, 4>(A, lda, sa, B, ldb, sb, bias, C, ldc, M, N, K, st);
-  else if ((M + 63) / 64 * n64 <= 3 * cus) launch_small<64, 64, 3>(A, lda, sa, B, ldb, sb, bias, C, ldc, M, N, K, st);
-  else if ((M + 127) / 128 * n64 <= 2 * cus) launch_small<128, 64, 3>(A, lda, sa, B, ldb, sb, bias, C, ldc, M, N, K, st);
+  if ((M + 31) / 32 * n64 <= 2 * cus) launch_small<32, 64, 4>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, st);
+  else if ((M + 63) / 64 * n64 <= 3 * cus) launch_small<64, 64, 3>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, st);
+  else if ((M + 127) / 128 * n64 <= 2 * cus) launch_small<128, 64, 3>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, st);
   else return false;
   return true;
 }
@@ -842,17 +861,17 @@ static bool launch_small_class(const void *A, int64_t lda, const float *sa, cons
 // kernel's). lda, ldb and K in elements.
 template <bool kMN, int kEl = 1, typename CT = uint16_t>
 static int launch_gemm(const void *A, int64_t lda, const float *sa, const void *B, int64_t ldb, const float *sb,
-                       const uint16_t *bias, CT *C, int64_t ldc, int64_t M, int64_t N, int64_t K, void *ws,
-                       size_t ws_bytes, hipStream_t st) {
+                       const void *bias, CT *C, int64_t ldc, int64_t M, int64_t N, int64_t K, void *ws,
+                       size_t ws_bytes, hipStream_t st, int bias32 = 0) {
   constexpr bool kC32 = sizeof(CT) == 4;
   if (M == 0 || N == 0) return GPIC_OK;
   if (K > 0 && (!A || !B)) return GPIC_EINVAL;
-  if (!aligned16(A) || !aligned16(B) || !aligned16(C) || (bias && ((uintptr_t)bias & 7u))) return GPIC_EALIGN;
+  if (!aligned16(A) || !aligned16(B) || !aligned16(C) || (bias && ((uintptr_t)bias & (bias32 ? 15u : 7u)))) return GPIC_EALIGN;
   // (a K tile is 128 bytes of each operand's K: the plan of a byte matrix kEl times as long)
   Plan p = K > 0 ? plan_gemm(M, N, K * kEl) : Plan{(int)((M + kBM - 1) / kBM), (int)((N + kBN - 1) / kBN), 1, kBK, kBN};
   float *P = nullptr;
   if constexpr (!kMN && kEl == 1) {
-    if (K > 0 && p.splits == 1 && launch_small_class(A, lda, sa, B, ldb, sb, bias, C, ldc, M, N, K, st))
+    if (K > 0 && p.splits == 1 && launch_small_class(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, st))
       return (int)hipGetLastError();
   }
   if (p.splits > 1) {
@@ -870,13 +889,13 @@ static int launch_gemm(const void *A, int64_t lda, const float *sa, const void *
   auto *kernel = p.bn == 128 ? ((K * kEl) % kBK ? gemm_tn_kernel<true, kMN, 128, kEl, kC32> : gemm_tn_kernel<false, kMN, 128, kEl, kC32>)
                               : ((K * kEl) % kBK ? gemm_tn_kernel<true, kMN, 256, kEl, kC32> : gemm_tn_kernel<false, kMN, 256, kEl, kC32>);
   kernel<<<grid, kThreads, 0, st>>>(
-      static_cast<const uint8_t *>(A), (int)lda * kEl, static_cast<const uint8_t *>(B), (int)ldb * kEl, sa, sb, bias, C,
+      static_cast<const uint8_t *>(A), (int)lda * kEl, static_cast<const uint8_t *>(B), (int)ldb * kEl, sa, sb, bias, bias32, C,
       ldc, P, (int)M, (int)N, (int)K, p.ksplit, p.tiles_m, p.tiles_n, p.splits);
   if (P) {
     const int64_t quads = M * (N / 4);
     int64_t g = (quads + 255) / 256;
     if (g > 8192) g = 8192;
-    splitk_reduce_kernel<CT><<<(int)g, 256, 0, st>>>(P, p.splits, (int)M, (int)N, sa, sb, bias, C, ldc);
+    splitk_reduce_kernel<CT><<<(int)g, 256, 0, st>>>(P, p.splits, (int)M, (int)N, sa, sb, bias, bias32, C, ldc);
   }
   return (int)hipGetLastError();
 }
@@ -893,17 +912,29 @@ size_t gpic_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   return p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
 }
 
+// (the epilogue's C offsets, row within the tile x ldc x 2 bytes, are 32-bit: ldc < 2^22)
+static bool tn_shape_ok(int64_t lda, int64_t ldb, int64_t ldc, int64_t M, int64_t N, int64_t K) {
+  return K % 16 == 0 && N % 16 == 0 && lda % 16 == 0 && ldb % 16 == 0 && ldc % 8 == 0 && lda >= K && ldb >= K &&
+         ldc >= N && lda < (1 << 23) && ldb < (1 << 23) && ldc < (1 << 22) && M < (1 << 30);
+}
+
 int gpic_fp8_gemm(const uint8_t *A, int64_t lda, const float *sa, const uint8_t *B, int64_t ldb, const float *sb,
                   const uint16_t *bias, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K, int fast_accum,
                   void *ws, size_t ws_bytes, void *stream) {
   status_scope();
   (void)fast_accum;
   if (M < 0 || N < 0 || K < 0 || !sa || !sb || (M > 0 && N > 0 && !C)) return GPIC_EINVAL;
-  if (K % 16 != 0 || N % 16 != 0 || lda % 16 != 0 || ldb % 16 != 0 || ldc % 8 != 0) return GPIC_ESHAPE;
-  // (the epilogue's C offsets, row within the tile x ldc x 2 bytes, are 32-bit: ldc < 2^22)
-  if (lda < K || ldb < K || ldc < N || lda >= (1 << 23) || ldb >= (1 << 23) || ldc >= (1 << 22) || M >= (1 << 30))
-    return GPIC_ESHAPE;
+  if (!tn_shape_ok(lda, ldb, ldc, M, N, K)) return GPIC_ESHAPE;
   return launch_gemm<false>(A, lda, sa, B, ldb, sb, bias, C, ldc, M, N, K, ws, ws_bytes, (hipStream_t)stream);
+}
+
+int gpic_fp8_gemm_bias32(const uint8_t *A, int64_t lda, const float *sa, const uint8_t *B, int64_t ldb, const float *sb,
+                         const float *bias, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K, void *ws,
+                         size_t ws_bytes, void *stream) {
+  status_scope();
+  if (M < 0 || N < 0 || K < 0 || !sa || !sb || !bias || (M > 0 && N > 0 && !C)) return GPIC_EINVAL;
+  if (!tn_shape_ok(lda, ldb, ldc, M, N, K)) return GPIC_ESHAPE;
+  return launch_gemm<false>(A, lda, sa, B, ldb, sb, bias, C, ldc, M, N, K, ws, ws_bytes, (hipStream_t)stream, 1);
 }
 
 int gpic_fp8_gemm_mn(const uint8_t *A, int64_t lda, const float *sa, const uint8_t *B, int64_t ldb, const float *sb,

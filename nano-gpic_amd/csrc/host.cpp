@@ -90,7 +90,7 @@ void cast_group(int n, const at::Tensor *const *xs, const int *kinds, void *ws, 
 }
 
 bool bias_ok(const std::optional<at::Tensor> &b, int64_t N, int dev) {
-  return !b || (b->scalar_type() == at::kBFloat16 && b->dim() == 1 && b->size(0) == N && plain(*b, dev));
+  return !b || (castable(*b, dev) && b->dim() == 1 && b->size(0) == N);
 }
 // a [M, K], b [N, K] -> bf16(sa sb a b^T) (+ bias) [M, N]
 at::Tensor gemm_tn(const at::Tensor &a, const at::Tensor &sa, const at::Tensor &b, const at::Tensor &sb,
@@ -98,6 +98,12 @@ at::Tensor gemm_tn(const at::Tensor &a, const at::Tensor &sa, const at::Tensor &
   const int64_t M = a.size(0), K = a.size(1), N = b.size(0);
   at::Tensor c = make(a, {M, N}, at::kBFloat16);
   const Scratch w(a, M, N, K);
+  if (bias && bias->scalar_type() == at::kFloat) {
+    check(gpic_fp8_gemm_bias32(ptr<uint8_t>(a), K, ptr<float>(sa), ptr<uint8_t>(b), K, ptr<float>(sb), ptr<float>(*bias),
+                               ptr<uint16_t>(c), N, M, N, K, w.p(), w.bytes, stream),
+          "gpic_fp8_gemm_bias32");
+    return c;
+  }
   check(gpic_fp8_gemm(ptr<uint8_t>(a), K, ptr<float>(sa), ptr<uint8_t>(b), K, ptr<float>(sb),
                       bias ? ptr<uint16_t>(*bias) : nullptr, ptr<uint16_t>(c), N, M, N, K, 1, w.p(), w.bytes, stream),
         "gpic_fp8_gemm");
@@ -160,7 +166,7 @@ py::object wgrad(const at::Tensor &a, const at::Tensor &sa, const at::Tensor &b,
   return py::cast(gemm_mn(a, sa, b, sb, f32, vp(stream)));
 }
 
-// x [M, K] bf16, w [N, K], bias [N] bf16 or None -> y [M, N], and x's and w's casts: (y, xq, sx, wqt, sw), w's
+// x [M, K] bf16, w [N, K], bias [N] or None -> y [M, N], and x's and w's casts: (y, xq, sx, wqt, sw), w's
 // transposed bytes only when `both` (else an empty tensor)
 py::object linear_fwd(const at::Tensor &x, const at::Tensor &w, const std::optional<at::Tensor> &bias, bool both, int dev,
                       handle ws, handle stream) {

@@ -671,9 +671,14 @@ __global__ __launch_bounds__(256, 2) void norm_bwd_kernel(NormBwdArgs p) {
 // batch, one thread per (batch, column). The next ceil(C / 16) workgroups: d_w [C] over all P partials, 16 columns
 // per workgroup: thread (k, c) adds partials [k P / 16, (k + 1) P / 16) of column c, then the 16 chunk sums of a
 // column are added in chunk order (a single thread per column would wait on P dependent loads).
+// VT: what d_shift, d_scale and d_gate are stored as, fp32 or bf16 (one rounding of the fp32 sum): the modulation is bf16,
+// and its gradients' conversions were three launches of ~4 us each behind this one.
+__device__ __forceinline__ void store_sum(float *p, float v) { *p = v; }
+__device__ __forceinline__ void store_sum(uint16_t *p, float v) { *p = (uint16_t)bf16_rne(v); }
+template <typename VT>
 __global__ __launch_bounds__(256) void norm_bwd_reduce_kernel(const float *__restrict__ part, int P, int tiles_b, int B,
-                                                              int C, bool res, float *__restrict__ dsh,
-                                                              float *__restrict__ dsc, float *__restrict__ dg,
+                                                              int C, bool res, VT *__restrict__ dsh,
+                                                              VT *__restrict__ dsc, VT *__restrict__ dg,
                                                               float *__restrict__ dw) {
   const int64_t nbc = (int64_t)B * C;
   const int64_t wg_bc = (nbc + 255) / 256;
@@ -688,9 +693,9 @@ __global__ __launch_bounds__(256) void norm_bwd_reduce_kernel(const float *__res
       s1 = s1 + part[(1 * (int64_t)P + prow) * C + c];
       if (res) s3 = s3 + part[(3 * (int64_t)P + prow) * C + c];
     }
-    dsh[i] = s0;
-    dsc[i] = s1;
-    if (res) dg[i] = s3;
+    store_sum(dsh + i, s0);
+    store_sum(dsc + i, s1);
+    if (res) store_sum(dg + i, s3);
     return;
   }
   __shared__ float chunk[16][16];
@@ -737,6 +742,53 @@ static void launch_norm_bwd(const NormBwdArgs &p, bool res, hipStream_t st) {
 static int64_t norm_bwd_parts(int64_t rows, int64_t ntok) {
   return ntok > 0 ? (rows / ntok) * ((ntok + kBwdRows - 1) / kBwdRows) : 0;
 }
+
+// The backward (checks, launches), for either type of the modulation's gradients.
+template <typename VT>
+static int norm_bwd(const uint16_t *dh, const uint16_t *dxn, const uint16_t *xs, const uint16_t *a, const uint16_t *gate,
+                    int64_t sg, const float *w, const uint16_t *scale, int64_t ssc, const float *rstd, int64_t rows,
+                    int64_t ntok, int64_t C, uint16_t *dx, uint16_t *da, VT *dshift, VT *dscale, VT *dgate, float *dw,
+                    void *ws, size_t ws_bytes, void *stream) {
+  status_scope();
+  const bool res = a != nullptr;
+  if (rows < 0 || C <= 0 || ntok <= 0 || !w || !scale || !dshift || !dscale || !dw || (res && (!gate || !dgate)))
+    return GPIC_EINVAL;
+  if (rows > 0 && (!dh || !xs || !rstd || !dx || (res && !da) || !ws)) return GPIC_EINVAL;
+  if (!res && (dxn || dgate)) return GPIC_EINVAL;
+  if (C % 4 != 0 || C > 2048 || rows % ntok != 0 || ssc % 4 != 0 || ssc < C || (res && (sg % 4 != 0 || sg < C)))
+    return GPIC_ESHAPE;
+  if (!aligned16(dh) || (dxn && !aligned16(dxn)) || !aligned16(xs) || (a && !aligned16(a)) || !aligned16(w) ||
+      ((uintptr_t)scale & 7u) || ((uintptr_t)gate & 7u) || !aligned16(dx) || (da && !aligned16(da)) ||
+      !aligned16(ws))
+    return GPIC_EALIGN;
+  const int64_t B = rows / ntok;
+  hipStream_t st = (hipStream_t)stream;
+  if (rows == 0) {   // no rows: d_w is zero (the reduce over no partials writes it; no memset, so a graph can hold it)
+    norm_bwd_reduce_kernel<VT><<<(int)((C + 15) / 16), 256, 0, st>>>(nullptr, 0, 0, 0, (int)C, res, dshift, dscale,
+                                                                     dgate, dw);
+    return (int)hipGetLastError();
+  }
+  const int64_t P = norm_bwd_parts(rows, ntok);
+  if (ws_bytes < (size_t)4 * P * C * sizeof(float)) return GPIC_EWORKSPACE;
+  if (P >= (int64_t(1) << 31) / 4 || B * C >= (int64_t(1) << 31)) return GPIC_ESHAPE;
+  NormBwdArgs p{dh, dxn, xs, a, gate, w, scale, rstd, dx, da, static_cast<float *>(ws), rows, ntok, sg, ssc, (int)C,
+                (int)((ntok + kBwdRows - 1) / kBwdRows), (int)P};
+  switch ((C + 255) / 256) {
+    case 1: launch_norm_bwd<1>(p, res, st); break;
+    case 2: launch_norm_bwd<2>(p, res, st); break;
+    case 3: launch_norm_bwd<3>(p, res, st); break;
+    case 4: launch_norm_bwd<4>(p, res, st); break;
+    case 5: launch_norm_bwd<5>(p, res, st); break;
+    case 6: launch_norm_bwd<6>(p, res, st); break;
+    case 7: launch_norm_bwd<7>(p, res, st); break;
+    default: launch_norm_bwd<8>(p, res, st); break;
+  }
+  const int64_t grid = (B * C + 255) / 256 + (C + 15) / 16;
+  norm_bwd_reduce_kernel<VT><<<(int)grid, 256, 0, st>>>(static_cast<const float *>(ws), (int)P, p.tiles_b, (int)B,
+                                                        (int)C, res, dshift, dscale, dgate, dw);
+  return (int)hipGetLastError();
+}
+
 }  // namespace gpic
 
 using namespace gpic;
@@ -799,44 +851,17 @@ int gpic_fp8_res_mod_rmsnorm_bwd(const uint16_t *dh, const uint16_t *dxn, const 
                                  const float *rstd, int64_t rows, int64_t ntok, int64_t C, uint16_t *dx, uint16_t *da,
                                  float *dshift, float *dscale, float *dgate, float *dw, void *ws, size_t ws_bytes,
                                  void *stream) {
-  status_scope();
-  const bool res = a != nullptr;
-  if (rows < 0 || C <= 0 || ntok <= 0 || !w || !scale || !dshift || !dscale || !dw || (res && (!gate || !dgate)))
-    return GPIC_EINVAL;
-  if (rows > 0 && (!dh || !xs || !rstd || !dx || (res && !da) || !ws)) return GPIC_EINVAL;
-  if (!res && (dxn || dgate)) return GPIC_EINVAL;
-  if (C % 4 != 0 || C > 2048 || rows % ntok != 0 || ssc % 4 != 0 || ssc < C || (res && (sg % 4 != 0 || sg < C)))
-    return GPIC_ESHAPE;
-  if (!aligned16(dh) || (dxn && !aligned16(dxn)) || !aligned16(xs) || (a && !aligned16(a)) || !aligned16(w) ||
-      ((uintptr_t)scale & 7u) || ((uintptr_t)gate & 7u) || !aligned16(dx) || (da && !aligned16(da)) ||
-      !aligned16(ws))
-    return GPIC_EALIGN;
-  const int64_t B = rows / ntok;
-  hipStream_t st = (hipStream_t)stream;
-  if (rows == 0) {   // no rows: d_w is zero (the reduce over no partials writes it; no memset, so a graph can hold it)
-    norm_bwd_reduce_kernel<<<(int)((C + 15) / 16), 256, 0, st>>>(nullptr, 0, 0, 0, (int)C, res, dshift, dscale,
-                                                                  dgate, dw);
-    return (int)hipGetLastError();
-  }
-  const int64_t P = norm_bwd_parts(rows, ntok);
-  if (ws_bytes < (size_t)4 * P * C * sizeof(float)) return GPIC_EWORKSPACE;
-  if (P >= (int64_t(1) << 31) / 4 || B * C >= (int64_t(1) << 31)) return GPIC_ESHAPE;
-  NormBwdArgs p{dh, dxn, xs, a, gate, w, scale, rstd, dx, da, static_cast<float *>(ws), rows, ntok, sg, ssc, (int)C,
-                (int)((ntok + kBwdRows - 1) / kBwdRows), (int)P};
-  switch ((C + 255) / 256) {
-    case 1: launch_norm_bwd<1>(p, res, st); break;
-    case 2: launch_norm_bwd<2>(p, res, st); break;
-    case 3: launch_norm_bwd<3>(p, res, st); break;
-    case 4: launch_norm_bwd<4>(p, res, st); break;
-    case 5: launch_norm_bwd<5>(p, res, st); break;
-    case 6: launch_norm_bwd<6>(p, res, st); break;
-    case 7: launch_norm_bwd<7>(p, res, st); break;
-    default: launch_norm_bwd<8>(p, res, st); break;
-  }
-  const int64_t grid = (B * C + 255) / 256 + (C + 15) / 16;
-  norm_bwd_reduce_kernel<<<(int)grid, 256, 0, st>>>(static_cast<const float *>(ws), (int)P, p.tiles_b, (int)B, (int)C,
-                                                     res, dshift, dscale, dgate, dw);
-  return (int)hipGetLastError();
+  return norm_bwd(dh, dxn, xs, a, gate, sg, w, scale, ssc, rstd, rows, ntok, C, dx, da, dshift, dscale, dgate, dw, ws, ws_bytes,
+                  stream);
+}
+
+int gpic_fp8_res_mod_rmsnorm_bwd16(const uint16_t *dh, const uint16_t *dxn, const uint16_t *xs, const uint16_t *a,
+                                   const uint16_t *gate, int64_t sg, const float *w, const uint16_t *scale, int64_t ssc,
+                                   const float *rstd, int64_t rows, int64_t ntok, int64_t C, uint16_t *dx, uint16_t *da,
+                                   uint16_t *dshift, uint16_t *dscale, uint16_t *dgate, float *dw, void *ws, size_t ws_bytes,
+                                   void *stream) {
+  return norm_bwd(dh, dxn, xs, a, gate, sg, w, scale, ssc, rstd, rows, ntok, C, dx, da, dshift, dscale, dgate, dw, ws, ws_bytes,
+                  stream);
 }
 
 }  // extern "C"

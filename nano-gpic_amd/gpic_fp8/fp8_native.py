@@ -667,7 +667,6 @@ def _cast_xw(x2, *ws, kind):
 def _linear_fwd(x2, w, b, kind):
     """The forward of a linear: (y, xq, sx, wqt, sw), the weight cast with x in one launch (kind BOTH: wqt its transposed
     bytes, FLAT: an empty tensor)."""
-    b = None if b is None else b.to(torch.bfloat16)
     r = L.native("linear_fwd", x2, x2, w, b, kind == BOTH)
     if r is not None:
         return r
@@ -719,7 +718,7 @@ class _Fp8LinearF8(torch.autograd.Function):
             y, xq, sx, wqt, sw = _linear_fwd(x2, w, b, BOTH)
         else:
             (xq, sx), (wq, wqt, sw) = L.call(tcast, x2), wcast
-            y = L.call(fp8_gemm, xq, sx, wq, sw, None if b is None else b.to(torch.bfloat16))
+            y = L.call(fp8_gemm, xq, sx, wq, sw, b)
         ctx.save_for_backward(xq, sx, wqt, sw)
         ctx.has_b, ctx.shape, ctx.wdt = b is not None, shape, w.dtype
         return y.view(*shape[:-1], w.shape[0])
@@ -743,7 +742,7 @@ class _Fp8HeadsLinearF8(torch.autograd.Function):
         xq, sx = L.call(tcast_heads, o)
         xq = xq.view(B * N, H * D)
         wq, wqt, sw = L.call(tcast_t, w) if wcast is None else wcast
-        y = L.call(fp8_gemm, xq, sx, wq, sw, None if b is None else b.to(torch.bfloat16))
+        y = L.call(fp8_gemm, xq, sx, wq, sw, b)
         ctx.save_for_backward(xq, sx, wqt, sw)
         ctx.has_b, ctx.shape, ctx.wdt = b is not None, (B, H, N, D), w.dtype
         return y.view(B, N, w.shape[0])

@@ -100,14 +100,8 @@ def _(x, a, gate, w, shift, scale, eps, has_res, want_h, want_q=True):
             x.new_empty(B * N, dtype=torch.float32))
 
 
-@L.custom_op("gpic::fp8_res_mod_rmsnorm_bwd")
-def res_mod_rmsnorm_bwd_k(dh: torch.Tensor, dxn: Optional[torch.Tensor], xs: torch.Tensor, a: Optional[torch.Tensor],
-                          gate: Optional[torch.Tensor], w: torch.Tensor, scale: torch.Tensor, rstd: torch.Tensor
-                          ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    """The norm site's backward (fused_norm.py:94-147, op :249-275) on the HIP kernel: dh [B, N, C] (the gradient of
-    h), dxn (that of x_new, site 2) or None, xs = x_new (site 2) or x, a and gate (site 2) or None, rstd [B * N].
-    Returns dx, da (empty at site 1), d_gate [B, C] (empty at site 1), d_w [C], d_shift [B, C], d_scale [B, C]: fp32
-    column sums taken in a fixed order."""
+def _bwd(dh, dxn, xs, a, gate, w, scale, rstd, vdt):
+    """res_mod_rmsnorm_bwd_k with d_gate, d_shift and d_scale as vdt (fp32, or bf16: the sums rounded once)."""
     L.require_gpu(dh, xs, w, scale, rstd)
     B, N, C = xs.shape
     res = a is not None
@@ -121,21 +115,33 @@ def res_mod_rmsnorm_bwd_k(dh: torch.Tensor, dxn: Optional[torch.Tensor], xs: tor
     dev = xs.device
     dx = torch.empty_like(xsc)
     da = torch.empty_like(xsc) if res else xs.new_empty(0)
-    f32 = dict(dtype=torch.float32, device=dev)
+    f32, vec = dict(dtype=torch.float32, device=dev), dict(dtype=vdt, device=dev)
     if B * N == 0:   # no rows: every column sum is zero
-        z = torch.zeros(B, C, **f32)
-        return dx, da, (z.clone() if res else torch.empty(0, **f32)), torch.zeros(C, **f32), z.clone(), z.clone()
-    dg = torch.empty(B, C, **f32) if res else torch.empty(0, **f32)
-    dw, dsh, dsc = torch.empty(C, **f32), torch.empty(B, C, **f32), torch.empty(B, C, **f32)
+        z = torch.zeros(B, C, **vec)
+        return dx, da, (z.clone() if res else torch.empty(0, **vec)), torch.zeros(C, **f32), z.clone(), z.clone()
+    dg = torch.empty(B, C, **vec) if res else torch.empty(0, **vec)
+    dw, dsh, dsc = torch.empty(C, **f32), torch.empty(B, C, **vec), torch.empty(B, C, **vec)
+    name = "gpic_fp8_res_mod_rmsnorm_bwd" if vdt == torch.float32 else "gpic_fp8_res_mod_rmsnorm_bwd16"
     with L.on_device(dev):
         nws = L.lib().gpic_fp8_res_mod_rmsnorm_bwd_workspace_bytes(B * N, max(N, 1), C)
         ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=dev)
-        L.check(L.lib().gpic_fp8_res_mod_rmsnorm_bwd(
+        L.check(getattr(L.lib(), name)(
             dhc.data_ptr(), L.ptr(dxc), xsc.data_ptr(), L.ptr(ac), L.ptr(g), g.stride(0) if res else 0, wf.data_ptr(),
             sc.data_ptr(), sc.stride(0), rstd.data_ptr(), B * N, max(N, 1), C, dx.data_ptr(),
             da.data_ptr() if res else None, dsh.data_ptr(), dsc.data_ptr(), dg.data_ptr() if res else None,
-            dw.data_ptr(), ws.data_ptr(), nws, L.stream_ptr(dev)), "gpic_fp8_res_mod_rmsnorm_bwd")
+            dw.data_ptr(), ws.data_ptr(), nws, L.stream_ptr(dev)), name)
     return dx, da, dg, dw, dsh, dsc
+
+
+@L.custom_op("gpic::fp8_res_mod_rmsnorm_bwd")
+def res_mod_rmsnorm_bwd_k(dh: torch.Tensor, dxn: Optional[torch.Tensor], xs: torch.Tensor, a: Optional[torch.Tensor],
+                          gate: Optional[torch.Tensor], w: torch.Tensor, scale: torch.Tensor, rstd: torch.Tensor
+                          ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+    """The norm site's backward (fused_norm.py:94-147, op :249-275) on the HIP kernel: dh [B, N, C] (the gradient of
+    h), dxn (that of x_new, site 2) or None, xs = x_new (site 2) or x, a and gate (site 2) or None, rstd [B * N].
+    Returns dx, da (empty at site 1), d_gate [B, C] (empty at site 1), d_w [C], d_shift [B, C], d_scale [B, C]: fp32
+    column sums taken in a fixed order."""
+    return _bwd(dh, dxn, xs, a, gate, w, scale, rstd, torch.float32)
 
 
 @res_mod_rmsnorm_bwd_k.register_fake
@@ -148,10 +154,28 @@ def _(dh, dxn, xs, a, gate, w, scale, rstd):
             xs.new_empty(B, C, **f32))
 
 
-def _norm_backward(dh, dxn, xs, a, gate, w, scale, rstd):
-    """The norm site's backward: (dx, da or None, d_gate or None, d_w, d_shift, d_scale), the column sums fp32."""
-    dx, da, dg, dw, dsh, dsc = L.call(res_mod_rmsnorm_bwd_k, dh, dxn if a is not None else None, xs, a, gate, w,
-                                      scale, rstd)
+@L.step_op("gpic::fp8_res_mod_rmsnorm_bwd16")
+def res_mod_rmsnorm_bwd16(dh: torch.Tensor, dxn: Optional[torch.Tensor], xs: torch.Tensor, a: Optional[torch.Tensor],
+                          gate: Optional[torch.Tensor], w: torch.Tensor, scale: torch.Tensor, rstd: torch.Tensor
+                          ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+    """res_mod_rmsnorm_bwd_k with d_gate, d_shift and d_scale in bf16, the gradients of a bf16 modulation."""
+    return _bwd(dh, dxn, xs, a, gate, w, scale, rstd, torch.bfloat16)
+
+
+@res_mod_rmsnorm_bwd16.register_fake
+def _(dh, dxn, xs, a, gate, w, scale, rstd):
+    B, N, C = xs.shape
+    res = a is not None
+    return (torch.empty_like(xs), torch.empty_like(xs) if res else xs.new_empty(0), xs.new_empty((B, C) if res else (0,)),
+            xs.new_empty(C, dtype=torch.float32), xs.new_empty(B, C), xs.new_empty(B, C))
+
+
+def _norm_backward(dh, dxn, xs, a, gate, w, shift, scale, rstd):
+    """The norm site's backward: (dx, da or None, d_gate or None, d_w, d_shift, d_scale), the column sums fp32, or bf16
+    (but d_w) where the whole modulation is bf16."""
+    bf16 = all(t is None or t.dtype == torch.bfloat16 for t in (gate, shift, scale))
+    dx, da, dg, dw, dsh, dsc = L.call(res_mod_rmsnorm_bwd16 if bf16 else res_mod_rmsnorm_bwd_k, dh,
+                                      dxn if a is not None else None, xs, a, gate, w, scale, rstd)
     if a is None:
         return dx, None, None, dw, dsh, dsc
     return dx, da, dg, dw, dsh, dsc
@@ -242,7 +266,7 @@ class _ResModRMSNorm(torch.autograd.Function):
     def backward(ctx, dxn, dh):
         xs, a, gate, w, shift, scale, rstd = ctx.saved_tensors
         B, _, C = xs.shape
-        dx, da, dg, dw, dsh, dsc = _norm_backward(dh, dxn if ctx.has_res else None, xs, a, gate, w, scale, rstd)
+        dx, da, dg, dw, dsh, dsc = _norm_backward(dh, dxn if ctx.has_res else None, xs, a, gate, w, shift, scale, rstd)
         dgate, dw, dshift, dscale = _param_grads(B, C, dg, dw, dsh, dsc, gate, w, shift, scale)
         return dx, da, dgate, dw, dshift, dscale, None, None
 
@@ -278,7 +302,7 @@ class _Fp8ModRMSNormLinear(torch.autograd.Function):
         _, _, hq, sh, rstd = L.call(res_mod_rmsnorm_q, x, x, x, w_norm, shift, scale, eps, False, False)
         hq2 = hq.view(B * N, C)
         wq, wqt, sw = L.call(tcast_t, weight)
-        y = L.call(fp8_gemm, hq2, sh, wq, sw, None if bias is None else bias.to(torch.bfloat16))
+        y = L.call(fp8_gemm, hq2, sh, wq, sw, bias)
         ctx.save_for_backward(x, w_norm, shift, scale, rstd, hq2, sh, wqt, sw)
         ctx.has_b, ctx.wdt = bias is not None, weight.dtype
         return y.view(B, N, weight.shape[0])
@@ -289,7 +313,7 @@ class _Fp8ModRMSNormLinear(torch.autograd.Function):
         B, N, C = x.shape
         dy2 = dy.reshape(B * N, -1).to(torch.bfloat16)
         dh, dweight, db = _linear_bwd(dy2, hq2, sh, wqt, sw, ctx.has_b, ctx.wdt)
-        dx, _, _, dw, dsh, dsc = _norm_backward(dh.view(B, N, C), None, x, None, None, w_norm, scale, rstd)
+        dx, _, _, dw, dsh, dsc = _norm_backward(dh.view(B, N, C), None, x, None, None, w_norm, shift, scale, rstd)
         _, dw, dshift, dscale = _param_grads(B, C, None, dw, dsh, dsc, None, w_norm, shift, scale)
         return dx, dw, dshift, dscale, None, dweight, db
 
@@ -323,7 +347,7 @@ class _Fp8ResModRMSNormMLP(torch.autograd.Function):
         dzq, sdz = L.call(swiglu_bwd_q, z, da_)
         dh = L.call(fp8_gemm, dzq, sdz, w12qt, s12, None, False).view(B, N, C)
         dw12 = _wgrad8(dzq, sdz, hq2, sh, ctx.dt[0])
-        dx, da, dg, dw, dsh, dsc = _norm_backward(dh, dxn, xn, a, gate, w_norm, scale, rstd)
+        dx, da, dg, dw, dsh, dsc = _norm_backward(dh, dxn, xn, a, gate, w_norm, shift, scale, rstd)
         dgate, dw, dshift, dscale = _param_grads(B, C, dg, dw, dsh, dsc, gate, w_norm, shift, scale)
         return dx, da, dgate, dw, dshift, dscale, None, dw12, dw3
 

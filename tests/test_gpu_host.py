@@ -96,3 +96,19 @@ def test_errors_stay_errors(dev):
         G.fp8_linear_f8(x, torch.randn(24, 32, device=dev))    # N % 16
     with pytest.raises(RuntimeError, match="GPU only"):
         F.fp8_gemm(torch.zeros(16, 16).to(G.E4), torch.ones(1), torch.zeros(16, 16).to(G.E4), torch.ones(1))
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 48, 160), (2048, 1024, 1024), (512, 1024, 4096), (6592, 1024, 4096),
+                                   (333, 3072, 1024), (33000, 272, 1024), (4096, 3072, 1040)])
+def test_fp32_bias(dev, M, N, K):
+    """An fp32 bias read by the GEMM (small, narrow, wide and split-K epilogues) gives the bits of its bf16 rounding."""
+    g = torch.Generator(device=dev).manual_seed(M)
+    a, b = (torch.randn(n, K, generator=g, device=dev).to(G.E4) for n in (M, N))
+    s = torch.tensor([0.3], device=dev)
+    bias = torch.randn(N, generator=g, device=dev)
+    bias[0], bias[1], bias[2] = float("nan"), float("inf"), 1.00390625   # (the last: a tie)
+    y, ref = G.fp8_gemm(a, s, b, s, bias), G.fp8_gemm(a, s, b, s, bias.to(B16))
+    assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
+    buf = torch.zeros(N + 1, device=dev)
+    buf[1:] = bias                                                       # not 16-byte aligned: the general form
+    assert torch.equal(G.fp8_gemm(a, s, b, s, buf[1:]).view(torch.int16), ref.view(torch.int16))
