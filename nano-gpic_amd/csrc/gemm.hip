@@ -635,14 +635,16 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
 // latency, not rate: the ping-pong spends ~1 us on each K tile of its 48 KiB however few workgroups run. Here kSS stages
 // of K = 128 are in flight, one barrier per K tile, several workgroups share a CU's 160 KiB of LDS and hide one another's
 // waits, and a lane stores its runs of 8 columns (col_of, as above) straight from the accumulators. The K tiles are
-// summed in the same order with the same instruction, so an unsplit result has the same bits as the other classes'.
-template <int kSM, int kSN, int kSS, bool kTail>
+// summed in the same order with the same instruction, so the results have the same bits as the other classes': where
+// their plan splits K, the accumulators are folded into a sum after every `per` K tiles (kSplit), as the reduce adds the
+// splits' partials.
+template <int kSM, int kSN, int kSS, bool kTail, bool kSplit>
 __global__ __launch_bounds__(256) void gemm_small_kernel(const uint8_t *__restrict__ A, int lda,
                                                          const uint8_t *__restrict__ B, int ldb,
                                                          const float *__restrict__ sa, const float *__restrict__ sb,
                                                          const void *__restrict__ bias, int bias32,
                                                          uint16_t *__restrict__ C, int64_t ldc, int M, int N, int K,
-                                                         int tiles_n) {
+                                                         int tiles_n, int per) {
   constexpr int kA = kSM * kBK, kStage = (kSM + kSN) * kBK;   // bytes of a stage's A part, of a stage
   constexpr int kLA = kSM / 32, kLB = kSN / 32, kL = kLA + kLB;   // loads per wave and K tile: 8 rows each
   constexpr int kFM = kSM / 32, kFN = kSN / 32;               // 16 x 16 tiles per wave
@@ -685,6 +687,14 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(const uint8_t *__restri
   for (int i = 0; i < kFN; i++)
 #pragma unroll
     for (int j = 0; j < kFM; j++) acc[i][j] = v4f{};
+  v4f sum[kFN][kFM];   // kSplit: the splits before the current one
+  auto fold = [&](bool first) {
+#pragma unroll
+    for (int i = 0; i < kFN; i++)
+#pragma unroll
+      for (int j = 0; j < kFM; j++) sum[i][j] = first ? acc[i][j] : sum[i][j] + acc[i][j];
+  };
+  int next = per;      // the K tile that begins the next split
   const int frow = lane & 15, fsw = swz(frow), c0 = 2 * (lane >> 4);
   const int lo = 16 * (c0 ^ fsw), hi = 16 * ((c0 + 1) ^ fsw);
   for (int kt = 0; kt < nk; kt++) {
@@ -704,6 +714,14 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(const uint8_t *__restri
       const u32x4 x0 = *(const GPIC_LDS u32x4 *)(p + lo), x1 = *(const GPIC_LDS u32x4 *)(p + hi);
       return v8i{(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w, (int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
     };
+    if (kSplit && kt == next) {
+      fold(next == per);
+      next += per;
+#pragma unroll
+      for (int i = 0; i < kFN; i++)
+#pragma unroll
+        for (int j = 0; j < kFM; j++) acc[i][j] = v4f{};
+    }
     v8i fa[kFM], fb[kFN];
 #pragma unroll
     for (int j = 0; j < kFM; j++) fa[j] = frag(wm * (kSM / 2) + 16 * j);
@@ -714,6 +732,13 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(const uint8_t *__restri
 #pragma unroll
       for (int mi = 0; mi < kFM; mi++)
         acc[ni][mi] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[ni], fa[mi], acc[ni][mi], 0, 0, 0, 0, 0, 0);
+  }
+  if constexpr (kSplit) {
+    fold(next == per);
+#pragma unroll
+    for (int i = 0; i < kFN; i++)
+#pragma unroll
+      for (int j = 0; j < kFM; j++) acc[i][j] = sum[i][j];
   }
   const float s = sa[0] * sb[0];
 #pragma unroll
@@ -834,28 +859,34 @@ static Plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 template <int kSM, int kSN, int kSS>
 static void launch_small(const void *A, int64_t lda, const float *sa, const void *B, int64_t ldb, const float *sb,
                          const void *bias, int bias32, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K,
-                         hipStream_t st) {
+                         const Plan &p, hipStream_t st) {
   const int tiles_n = (int)((N + kSN - 1) / kSN), tiles = (int)((M + kSM - 1) / kSM) * tiles_n;
-  auto *kernel = K % kBK ? gemm_small_kernel<kSM, kSN, kSS, true> : gemm_small_kernel<kSM, kSN, kSS, false>;
+  auto *kernel = p.splits > 1 ? (K % kBK ? gemm_small_kernel<kSM, kSN, kSS, true, true> : gemm_small_kernel<kSM, kSN, kSS, false, true>)
+                              : (K % kBK ? gemm_small_kernel<kSM, kSN, kSS, true, false> : gemm_small_kernel<kSM, kSN, kSS, false, false>);
   kernel<<<tiles, 256, 0, st>>>(static_cast<const uint8_t *>(A), (int)lda, static_cast<const uint8_t *>(B), (int)ldb, sa,
-                                sb, bias, bias32, C, ldc, (int)M, (int)N, (int)K, tiles_n);
+                                sb, bias, bias32, C, ldc, (int)M, (int)N, (int)K, tiles_n, p.ksplit / kBK);
 }
 
-// The small class where its tiles are few enough for the device (false, nothing launched, otherwise). Only unsplit
-// plans: a shape whose plan splits K keeps its partials and their order, which the MN-major layout shares. The limits are
+// The small class where its tiles are few enough for the device (false, nothing launched, otherwise). The limits are
 // where each tile stopped being the fastest, device time at K = 1024 (tiles per CU in brackets):
 //   [512 x 1024] 32 x 64 4.1 us (1), 64 x 64 4.8, 256 x 128 10.1;   [1024 x 1024] 4.7 (2), 5.0, 10.3
 //   [1024 x 3072] 32 x 64 9.7 (6), 64 x 64 7.7 (3), 128 x 64 8.2, 256 x 128 10.7;   [2048 x 1024] 7.6, 5.9 (2), 6.6, 10.2
 //   [4096 x 1024] 64 x 64 9.9 (4), 128 x 64 8.4 (2), 128 x 128 9.2, 256 x 128 11.0
 //   [2048 x 3072] 64 x 64 13.0 (6), 128 x 64 13.0 (3), 256 x 128 11.7: past these the bytes a small tile reads per flop
 //   (through L2) cost more than its latency saves.
+// Plans that split K (their partials and the reduce's launch fall away; 32 x 64 / 64 x 64 / 128 x 64 against the plan):
+//   [512 x 768 x 3072] 9.2 / 11.6 / 16.0 us, 17.8;   [1024 x 1024 x 8192] 24.8 / 27.2 / 36.1, 27.1;
+//   [2048 x 1024 x 4096] 25.9 / 18.0 / 20.7, 27.6;   [4096 x 768 x 6144] 49.7 / 34.8 / 34.4, 39.0;
+//   [1632 x 1280 x 10240] 65.8 / 46.9 / 50.0, 42.7: a long K is worth the splits' CUs, so they end at K = 8192.
 static bool launch_small_class(const void *A, int64_t lda, const float *sa, const void *B, int64_t ldb, const float *sb,
                                const void *bias, int bias32, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K,
-                               hipStream_t st) {
-  const int64_t cus = num_cus(), n64 = (N + 63) / 64;
-  if ((M + 31) / 32 * n64 <= 2 * cus) launch_small<32, 64, 4>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, st);
-  else if ((M + 63) / 64 * n64 <= 3 * cus) launch_small<64, 64, 3>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, st);
-  else if ((M + 127) / 128 * n64 <= 2 * cus) launch_small<128, 64, 3>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, st);
+                               const Plan &p, hipStream_t st) {
+  const int64_t cus = num_cus(), n64 = (N + 63) / 64, t32 = (M + 31) / 32 * n64, t64 = (M + 63) / 64 * n64,
+                t128 = (M + 127) / 128 * n64;
+  if (p.splits > 1 && K > 8192) return false;
+  if (t32 <= 2 * cus) launch_small<32, 64, 4>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, p, st);
+  else if (t64 <= 3 * cus) launch_small<64, 64, 3>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, p, st);
+  else if (t128 <= 2 * cus) launch_small<128, 64, 3>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, p, st);
   else return false;
   return true;
 }
@@ -874,7 +905,7 @@ static int launch_gemm(const void *A, int64_t lda, const float *sa, const void *
   Plan p = K > 0 ? plan_gemm(M, N, K * kEl) : Plan{(int)((M + kBM - 1) / kBM), (int)((N + kBN - 1) / kBN), 1, kBK, kBN};
   float *P = nullptr;
   if constexpr (!kMN && kEl == 1) {
-    if (K > 0 && p.splits == 1 && launch_small_class(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, st))
+    if (K > 0 && launch_small_class(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, p, st))
       return (int)hipGetLastError();
   }
   if (p.splits > 1) {

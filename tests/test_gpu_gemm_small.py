@@ -1,6 +1,6 @@
 """The small GEMM class: the same bits as the 256-wide classes' summation order (the MN-major kernel on the transposed
 bytes, which never takes it), at the edges of its tiles (32 x 64, 64 x 64, 128 x 64), partial K tiles, one to many K
-tiles of its ring of stages, with bias and padded rows, and within the elementwise bound of the float64 product."""
+tiles of its ring of stages, plans that split K (the splits' sums folded in their order), with bias and padded rows, and within the elementwise bound of the float64 product."""
 import pytest
 import torch
 
@@ -12,7 +12,10 @@ pytestmark = pytest.mark.gpu
 # the last of each group lies just past the class's limit (256 CUs)
 SHAPES = [(1, 16, 16), (31, 48, 128), (33, 80, 144), (32, 64, 256), (512, 1024, 384), (511, 1008, 400), (512, 1024, 1024),
           (1025, 1024, 512), (1024, 3072, 640), (4096, 768, 768), (4095, 784, 784), (4097, 1024, 1024), (2048, 1792, 1792),
-          (4096, 1040, 1040), (2049, 3072, 1024)]
+          (4096, 1040, 1040), (2049, 3072, 1024),
+          # split plans: even and uneven splits, a partial last K tile, K at and past the limit
+          (300, 768, 3072), (512, 1024, 4096), (1111, 1152, 4608), (257, 1792, 7168), (2048, 768, 6000), (1000, 896, 8192),
+          (1000, 896, 8208), (64, 64, 8192)]
 
 
 @pytest.mark.parametrize("bias", [False, True])
