@@ -904,15 +904,15 @@ static int launch_gemm(const void *A, int64_t lda, const float *sa, const void *
   // (a K tile is 128 bytes of each operand's K: the plan of a byte matrix kEl times as long)
   Plan p = K > 0 ? plan_gemm(M, N, K * kEl) : Plan{(int)((M + kBM - 1) / kBM), (int)((N + kBN - 1) / kBN), 1, kBK, kBN};
   float *P = nullptr;
-  if constexpr (!kMN && kEl == 1) {
-    if (K > 0 && launch_small_class(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, p, st))
-      return (int)hipGetLastError();
-  }
   if (p.splits > 1) {
     const size_t need = (size_t)p.splits * M * N * sizeof(float);
     if (!ws || ws_bytes < need) return GPIC_EWORKSPACE;
     if (!aligned16(ws)) return GPIC_EALIGN;
     P = static_cast<float *>(ws);
+  }
+  if constexpr (!kMN && kEl == 1) {   // (after the workspace's check: what a plan asks for does not depend on the class)
+    if (K > 0 && launch_small_class(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, p, st))
+      return (int)hipGetLastError();
   }
   // One workgroup per CU at most (160 KiB of LDS each); a persistent grid is a multiple of 8, one per XCD.
   const int work = p.tiles_m * p.tiles_n * p.splits;
