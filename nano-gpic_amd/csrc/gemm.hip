@@ -68,6 +68,7 @@ constexpr int kLoads = kBM / 8 / kLoaders;             // 8 wave-instructions (1
 constexpr int kGroupM = 4;
 constexpr int kBufferFlags = 0x00020000;               // raw buffer descriptor word 3 for gfx9-family targets
 constexpr int kOOB = (int)0x80000000;                  // an offset past any descriptor's range: reads zeros
+constexpr int64_t kMaxDescLd = int64_t(1) << 24;       // MN-major: the longest row (elements) whose K tail the descriptor masks
 // Cache policy of the bf16 C stores: nt (non-temporal). C is not read again by the kernel, and the streaming policy
 // keeps each round's 32 MiB burst of C from displacing the A and B panels the XCD's other tiles still read from L2
 // (12 d12 shapes: -3% GEMM time, the block step -2.3%, same process). The split-K partials keep the default policy:
@@ -189,9 +190,11 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
                                                             int ksplit, int tiles_m, int tiles_n, int splits) {
   static_assert(kBNt == 256 || kBNt == 128, "tile widths: 256 or 128");
   static_assert(kMN || (kEl == 1 && !kC32), "bf16 operands and fp32 outputs: MN-major only");
-  static_assert(!(kMN && kTail), "MN-major K rows past the end are masked by the descriptor");
+  static_assert(!(kMN && kTail) || kBNt == 256, "MN-major rows masked lane by lane: the wide tile only");
   constexpr int kKT = kBK / kEl;                  // K positions per K tile
   constexpr int kRowA = kBM * kEl;                // MN-major: bytes of a K row of A's K tile
+  static_assert((kKT - 1) * kMaxDescLd * kEl + kRowA < (int64_t(1) << 31),
+                "up to kMaxDescLd no lane offset of a K tile reaches 2^31, and none that starts from kOOB 2^32");
   constexpr int kRowBK = kBNt * kEl;              // and of B's
   constexpr int kWTNt = kBNt / 2;                 // wave tile columns
   constexpr int kTNt = kWTNt / 16;                // 16-column MFMA tiles per wave: 8 or 4
@@ -265,6 +268,8 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
     // out of range when its lane offset is at or past num_records less the scalar offset, so the K rows past the end of
     // the last, partial K tile read as zeros without a branch (a separate instance that masked them lane by lane ran
     // [8192 x 1024] over 6592 tokens in 72 us, against 57 over 6656; bf16 over 13303 against 13312 tokens: 185, 158).
+    // That holds while no row of the K tile wraps a lane offset around 2^32: row strides up to kMaxDescLd. Longer ones
+    // (below 128 bytes of K then, a single partial K tile) take the kTail instance, which masks the rows lane by lane.
     if constexpr (kMN) {
       const int ma = w.m0 * kEl, nb = w.n0 * kEl;
       w.rA = buffer_rsrc(A + ma, K * lda - ma);
@@ -304,10 +309,12 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__rest
       const int ld = isA ? lda : ldb;
       const int R0 = (i * kLoaders + (wave & 3)) * (kStep / kLoaders);
       const bool flip = kEl == 1 ? i & 2 : i & 1;   // the swizzle's row bit (5, bf16: 3)
-      // (kOOB + these offsets stays in [2^31, 2^32): still past the range, which is below 2^31)
+      // (kOOB + these offsets stays in [2^31, 2^32), past the range, which is below 2^31: row strides up to kMaxDescLd, and
+      // in the kTail instance the rows below K)
       const int vo = (flip ? (isA ? w.voA1 : w.voB1) : (isA ? w.voA : w.voB)) + i * opaque(kStep * ld);
       const uint32_t to = lds_addr(smem) + dst + R0 * kRowA;
-      lds_dma16(isA ? w.rA : w.rB, vo, k0 * ld, to);
+      if (!kTail) lds_dma16(isA ? w.rA : w.rB, vo, k0 * ld, to);
+      else lds_dma16(isA ? w.rA : w.rB, k0 + kStep * i + mrow < w.kend ? vo + k0 * ld : kOOB, 0, to);
     } else {
       const int R0 = (i * kLoaders + (wave & 3)) * 8;
       const int vo = isA ? baseA + i * opaque(32 * lda) : baseB + i * opaque(32 * ldb);
@@ -903,6 +910,8 @@ static int launch_gemm(const void *A, int64_t lda, const float *sa, const void *
   if (!aligned16(A) || !aligned16(B) || !aligned16(C) || (bias && ((uintptr_t)bias & (bias32 ? 15u : 7u)))) return GPIC_EALIGN;
   // (a K tile is 128 bytes of each operand's K: the plan of a byte matrix kEl times as long)
   Plan p = K > 0 ? plan_gemm(M, N, K * kEl) : Plan{(int)((M + kBM - 1) / kBM), (int)((N + kBN - 1) / kBN), 1, kBK, kBN};
+  const bool far = kMN && std::max(lda, ldb) > kMaxDescLd;   // (K x ld is below 2^31 bytes: one K tile, never split)
+  if (far) p = Plan{(int)((M + kBM - 1) / kBM), (int)((N + kBN - 1) / kBN), 1, kBK, kBN};
   float *P = nullptr;
   if (p.splits > 1) {
     const size_t need = (size_t)p.splits * M * N * sizeof(float);
@@ -919,10 +928,13 @@ static int launch_gemm(const void *A, int64_t lda, const float *sa, const void *
   const int slots = num_cus() & ~7;
   const int grid = work <= slots || slots < 8 ? work : slots;
   p.ksplit /= kEl;   // in K positions
-  // the partial-K-tile load path is compiled only into the instances that need it (K-major)
+  // the partial-K-tile load path is compiled only into the instances that need it (K-major; MN-major rows past kMaxDescLd)
   auto *kernel = p.bn == 128 ? gemm_tn_kernel<false, kMN, 128, kEl, kC32> : gemm_tn_kernel<false, kMN, 256, kEl, kC32>;
-  if constexpr (!kMN)
+  if constexpr (!kMN) {
     if (K % kBK) kernel = p.bn == 128 ? gemm_tn_kernel<true, false, 128> : gemm_tn_kernel<true, false, 256>;
+  } else {
+    if (far) kernel = gemm_tn_kernel<true, true, 256, kEl, kC32>;
+  }
   kernel<<<grid, kThreads, 0, st>>>(
       static_cast<const uint8_t *>(A), (int)lda * kEl, static_cast<const uint8_t *>(B), (int)ldb * kEl, sa, sb, bias, bias32, C,
       ldc, P, (int)M, (int)N, (int)K, p.ksplit, p.tiles_m, p.tiles_n, p.splits);
