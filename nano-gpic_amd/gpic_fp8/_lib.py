@@ -94,6 +94,9 @@ def host():
     return _host
 
 
+_CASTING = ("casts", "linear_fwd", "linear_bwd")   # the host module's functions that cast, so need the stream's workspace
+
+
 def native(name, t, *args):
     """The host module's function `name` on args (t: one of them, which says the device), or None where it does not take
     the call: while torch.compile traces, for tensors on another device than the current one, or not of the usual form."""
@@ -104,10 +107,11 @@ def native(name, t, *args):
     if device.index != index:
         return None
     stream = _raw_stream(index)
-    ws = _WORKSPACES.get((index, stream))
-    if ws is None:
-        ws = cast_workspace(device)
-    return getattr(_host or host(), name)(*args, index, ws.data_ptr(), stream)
+    ws = 0   # (a GEMM does not create one: under capture its zero fill would be part of that graph alone)
+    if name in _CASTING:
+        w = _WORKSPACES.get((index, stream))
+        ws = (cast_workspace(device) if w is None else w).data_ptr()
+    return getattr(_host or host(), name)(*args, index, ws, stream)
 
 
 def check(status, what):

@@ -181,3 +181,25 @@ def test_missing_host_module_is_an_error(monkeypatch, tmp_path):
     monkeypatch.setattr(L, "_host", None)
     with pytest.raises(RuntimeError, match="missing"):
         L.host()
+
+
+def test_only_casting_calls_get_a_cast_workspace(monkeypatch):
+    """A GEMM through the host module neither creates nor takes the stream's cast workspace; a call that casts does."""
+    import types
+    import torch
+    made = []
+
+    def workspace(device):
+        made.append(device)
+        return types.SimpleNamespace(data_ptr=lambda: 77)
+    host = types.SimpleNamespace(**{n: (lambda *a: a) for n in ("gemm", "wgrad", "casts", "linear_fwd", "linear_bwd")})
+    monkeypatch.setattr(L, "_host", host)
+    monkeypatch.setattr(L, "_raw_stream", lambda index: 5)
+    monkeypatch.setattr(L, "_WORKSPACES", {})
+    monkeypatch.setattr(L, "cast_workspace", workspace)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    t = types.SimpleNamespace(device=torch.device("cuda", 0))
+    for name in ("gemm", "wgrad"):
+        assert L.native(name, t, "a") == ("a", 0, 0, 5) and not made
+    for name in ("casts", "linear_fwd", "linear_bwd"):
+        assert L.native(name, t, "a") == ("a", 0, 77, 5) and made.pop()

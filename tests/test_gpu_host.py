@@ -112,3 +112,26 @@ def test_fp32_bias(dev, M, N, K):
     buf = torch.zeros(N + 1, device=dev)
     buf[1:] = bias                                                       # not 16-byte aligned: the general form
     assert torch.equal(G.fp8_gemm(a, s, b, s, buf[1:]).view(torch.int16), ref.view(torch.int16))
+
+
+def test_gemm_first_on_a_capturing_stream(dev, monkeypatch):
+    """GEMMs captured on a stream that has no cast workspace make none, in a graph of their own; a later graph on that stream
+    with a cast makes its own and gives the right bytes without the first one's replay."""
+    monkeypatch.setattr(L, "_WORKSPACES", {})
+    a, b, s = torch.randn(64, 128, device=dev).to(G.E4), torch.randn(32, 128, device=dev).to(G.E4), torch.ones(1, device=dev)
+    c, w = F.fp8_gemm(a, s, b, s), F.fp8_wgrad(a, s, a, s, True)
+    torch.cuda.synchronize()
+    first, second, x = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph(), torch.randn(300, 80, device=dev).to(B16)
+    with torch.cuda.graph(first):
+        got = F.fp8_gemm(a, s, b, s), F.fp8_wgrad(a, s, a, s, True)
+    assert not L._WORKSPACES
+    with torch.cuda.graph(second, stream=torch.cuda.graph.default_capture_stream):
+        q, sc = F.tcast(x)
+    for k in range(3):
+        x.mul_(0.5)
+        second.replay()
+        torch.cuda.synchronize()
+        assert sc.item() == x.abs().max().float().div(448).item()
+    first.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], c) and torch.equal(got[1], w)
