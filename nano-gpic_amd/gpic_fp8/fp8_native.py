@@ -427,8 +427,10 @@ def _(z, da):
 @L.step_op("gpic::fp8_dequant")
 def dequant(q: torch.Tensor, s: torch.Tensor) -> torch.Tensor:
     """(q.to(float32) * s).to(bfloat16) for e4m3 q and its scale s [1] fp32, in one pass."""
+    if q.dtype != E4:
+        raise ValueError(f"dequant takes float8_e4m3fn bytes, got {q.dtype}")
     L.require_gpu(q, s)
-    qc = L.aligned(q.contiguous())
+    qc, s = L.aligned(q.contiguous()), _scale(s)
     y = torch.empty(q.shape, dtype=torch.bfloat16, device=q.device)
     with L.on_device(q.device):
         L.check(L.lib().gpic_fp8_dequant(qc.data_ptr(), s.data_ptr(), qc.numel(), y.data_ptr(),
@@ -451,6 +453,11 @@ def _gemm_operand(t, name):
     return t
 
 
+def _scale(s):
+    """A dequantization scale as fp32 [1]."""
+    return s if s.dtype == torch.float32 and s.shape == (1,) else s.to(torch.float32).reshape(1)
+
+
 @L.custom_op("gpic::fp8_gemm")
 def fp8_gemm(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Tensor,
              bias: Optional[torch.Tensor] = None, fast: bool = True) -> torch.Tensor:
@@ -470,10 +477,7 @@ def fp8_gemm(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Tenso
         raise ValueError(f"fp8_gemm: a is [{M}, {K}] but b is {tuple(b.shape)}")
     if K % 16 or N % 16:
         raise ValueError(f"fp8_gemm needs K % 16 == 0 and N % 16 == 0, got M={M} N={N} K={K}")
-    if sa.dtype != torch.float32 or sa.shape != (1,):
-        sa = sa.to(torch.float32).reshape(1)
-    if sb.dtype != torch.float32 or sb.shape != (1,):
-        sb = sb.to(torch.float32).reshape(1)
+    sa, sb = _scale(sa), _scale(sb)
     if bias is not None:
         bias = bias.to(torch.bfloat16).contiguous()
         if bias.numel() != N:
@@ -528,10 +532,7 @@ def fp8_gemm_mn(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Te
             u[:, :K] = t.view(torch.uint8).t()
             return u.view(E4)
         return L.call(fp8_gemm, kmajor(a), sa, kmajor(b), sb, bias, False)
-    if sa.dtype != torch.float32 or sa.shape != (1,):
-        sa = sa.to(torch.float32).reshape(1)
-    if sb.dtype != torch.float32 or sb.shape != (1,):
-        sb = sb.to(torch.float32).reshape(1)
+    sa, sb = _scale(sa), _scale(sb)
     if bias is not None:
         bias = bias.to(torch.bfloat16).contiguous()
         if bias.numel() != N:
@@ -560,10 +561,13 @@ def fp8_wgrad(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Tens
         return c
     a2, b2 = _gemm_operand_mn(a, "a"), _gemm_operand_mn(b, "b")
     (K, M), N = a2.shape, b2.shape[1]
+    if b2.shape[0] != K or M % 16 or N % 16:
+        raise ValueError(f"fp8_wgrad needs a [K, M], b [K, N] with M, N % 16 == 0, got {tuple(a.shape)} and {tuple(b.shape)}")
     if not f32 or K * max(a2.stride(0), b2.stride(0)) >= 2 ** 31 or N >= 2 ** 21:
         dw = L.call(fp8_gemm_mn, a, sa, b, sb)
         return dw.float() if f32 else dw
     L.require_gpu(a2, b2, sa, sb)
+    sa, sb = _scale(sa), _scale(sb)
     c = torch.empty(M, N, dtype=torch.float32, device=a.device)
     with L.on_device(a.device):
         nws = L.gemm_workspace_bytes(a.device, M, N, K)
@@ -582,6 +586,8 @@ def _(a, sa, b, sb, f32):
 @L.step_op("gpic::fp8_bias_grad")
 def bias_grad(dy: torch.Tensor, f32: bool) -> torch.Tensor:
     """dy [M, N] bf16 -> dy.sum(0) (fp32 sums, one bf16 rounding), as bf16 or its values in fp32 (fp8_native.py:203)."""
+    if dy.dim() != 2 or dy.dtype != torch.bfloat16:
+        raise ValueError(f"bias_grad takes bf16 dy [M, N], got {dy.dtype} {tuple(dy.shape)}")
     L.require_gpu(dy)
     dt = torch.float32 if f32 else torch.bfloat16
     M, N = dy.shape
@@ -607,6 +613,9 @@ def bf16_wgrad(dy: torch.Tensor, x: torch.Tensor, f32: bool) -> torch.Tensor:
     """(dy [M, N].t() @ x [M, K]) bf16 -> [N, K] bf16, or its values in fp32 (fp8_native.py:202, 225, 264-265): the bf16
     wgrad on the hand-written GEMM, both operands read with the tokens as their rows, the gradient of an fp32 weight
     written as fp32."""
+    if dy.dim() != 2 or x.dim() != 2 or dy.shape[0] != x.shape[0] or dy.dtype != torch.bfloat16 or x.dtype != dy.dtype:
+        raise ValueError(f"bf16_wgrad takes bf16 dy [M, N] and x [M, K], got {dy.dtype} {tuple(dy.shape)} and {x.dtype} "
+                         f"{tuple(x.shape)}")
     L.require_gpu(dy, x)
     (M, N), K = dy.shape, x.shape[1]
     dt = torch.float32 if f32 else torch.bfloat16

@@ -390,3 +390,23 @@ def test_reference_norm_op_schemas():
     assert bwd.startswith("gpic::res_mod_rmsnorm_bwd(Tensor dh, Tensor dxn, Tensor xn, Tensor a, Tensor gate, Tensor w, "
                           "Tensor scale, Tensor rstd, bool has_res, bool has_dxn) -> (Tensor, Tensor, Tensor, Tensor, "
                           "Tensor, Tensor)"), bwd
+
+
+def test_wgrad_operands_are_checked():
+    """The step's own ops refuse operands whose rows, types or shapes do not fit each other before anything is launched."""
+    e = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)
+    q = lambda *s: torch.zeros(*s).to(F.E4)
+    one = torch.ones(1)
+    for dy, x in ((e(32, 16), e(16, 16)), (e(32, 16), torch.zeros(32, 16)), (torch.zeros(32, 16), e(32, 16)),
+                  (e(2, 32, 16), e(32, 16))):
+        with pytest.raises(ValueError, match="bf16_wgrad"):
+            F.bf16_wgrad(dy, x, True)
+    for a, b in ((q(32, 16), q(16, 16)), (q(32, 24), q(32, 16)), (q(32, 16), q(32, 24))):
+        for f32 in (False, True):
+            with pytest.raises(ValueError, match="fp8_wgrad"):
+                F.fp8_wgrad(a, one, b, one, f32)
+    for dy in (torch.zeros(4, 16), e(2, 4, 16)):
+        with pytest.raises(ValueError, match="bias_grad"):
+            F.bias_grad(dy, False)
+    with pytest.raises(ValueError, match="dequant"):
+        F.dequant(torch.zeros(4, dtype=torch.uint8), one)

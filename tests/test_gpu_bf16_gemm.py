@@ -65,3 +65,17 @@ def test_e4m3_wgrad_f32(dev, K, M, N):
     sa, sb = torch.tensor([0.37], device=dev), torch.tensor([1.9], device=dev)
     y = F.fp8_wgrad(a, sa, b, sb, True)
     assert y.dtype == torch.float32 and torch.equal(y, G.fp8_gemm_mn(a, sa, b, sb).float())
+
+
+def test_e4m3_wgrad_f32_scales_and_errors(dev):
+    """The general form (strided operands) takes a scale as any one-element float tensor, as fp8_gemm_mn does, and refuses
+    operands of different row counts."""
+    a, b = (torch.randn(64, n + 16, device=dev).to(G.E4)[:, :n] for n in (32, 48))
+    s = torch.tensor(0.5, dtype=torch.float64, device=dev)
+    assert torch.equal(F.fp8_wgrad(a, s, b, s, True), G.fp8_gemm_mn(a, s, b, s).float())
+    one = torch.ones(1, device=dev)
+    for f32 in (False, True):
+        with pytest.raises(ValueError):
+            F.fp8_wgrad(a, one, b[:48], one, f32)
+    with pytest.raises(ValueError):
+        F.bf16_wgrad(a.to(torch.bfloat16), b[:48].to(torch.bfloat16), True)
