@@ -640,7 +640,7 @@ def _(dy, x, f32):
 
 def _bias_grad(dy, dtype):
     """dy.sum(0).to(dtype)."""
-    return dy.sum(0).to(dtype) if _recorded() else L.call(bias_grad, dy, dtype == torch.float32).to(dtype)
+    return dy.sum(0).to(dtype) if _torch_ops(dy) else L.call(bias_grad, dy, dtype == torch.float32).to(dtype)
 
 
 def _wgrad8(a, sa, b, sb, dtype):
@@ -648,14 +648,17 @@ def _wgrad8(a, sa, b, sb, dtype):
     return L.call(fp8_wgrad, a, sa, b, sb, dtype == torch.float32).to(dtype)
 
 
-def _recorded():
-    """Whether a backward is itself being recorded (create_graph): its operations then have to be differentiable ones."""
-    return torch.is_grad_enabled() and not torch.compiler.is_compiling()
+def _torch_ops(dy):
+    """Whether a bf16 backward has to consist of torch's operations: when it is itself being recorded (create_graph; they
+    then have to be differentiable ones), and when dy is no ordinary tensor with memory of its own (a batch of gradients,
+    is_grads_batched or a vectorized jacobian; a wrapper subclass)."""
+    return not torch.compiler.is_compiling() and (torch.is_grad_enabled() or type(dy) is not torch.Tensor
+                                                  or not torch._C._has_storage(dy))
 
 
 def _wgrad16(dy, x, dtype):
     """(dy.t() @ x).to(dtype)."""
-    if _recorded():
+    if _torch_ops(dy):
         return (dy.t() @ x).to(dtype)
     return L.call(bf16_wgrad, dy, x, dtype == torch.float32).to(dtype)
 
@@ -686,7 +689,7 @@ def _linear_fwd(x2, w, b, kind):
 def _linear_bwd(dy2, xq, sx, wqt, sw, has_b, dtype):
     """The phase-3 backward of a linear: (dx [M, K] = [M, N] . [K, N]^T, dw [N, K] = [M, N]^T . [M, K], db or None)."""
     # (a backward that is itself recorded: the bias gradient is then a differentiable operation)
-    r = None if has_b and _recorded() else L.native("linear_bwd", dy2, dy2, xq, sx, wqt, sw, has_b, dtype == torch.float32)
+    r = None if has_b and _torch_ops(dy2) else L.native("linear_bwd", dy2, dy2, xq, sx, wqt, sw, has_b, dtype == torch.float32)
     if r is not None:
         dx, dw, db = r
         return dx, dw.to(dtype), None if db is None else db.to(dtype)
@@ -784,10 +787,10 @@ class _SwiGLUw3(torch.autograd.Function):
         z, aq, sa, w3 = ctx.saved_tensors
         dy2 = dy.reshape(-1, dy.shape[-1]).to(torch.bfloat16)
         da = dy2 @ w3.to(torch.bfloat16)
-        dw3 = _wgrad16(dy2, L.call(dequant, aq, sa), ctx.wdt)
-        if not _recorded():
-            return L.call(swiglu_dz, z, da).view(ctx.shape), dw3
-        # the same expression as torch operations
+        if not _torch_ops(dy):
+            return L.call(swiglu_dz, z, da).view(ctx.shape), _wgrad16(dy2, L.call(dequant, aq, sa), ctx.wdt)
+        # the same expressions as torch operations
+        dw3 = (dy2.t() @ (aq.to(torch.float32) * sa).to(torch.bfloat16)).to(ctx.wdt)
         z1, z2 = z.chunk(2, dim=-1)
         z1f = z1.float()
         sg = torch.sigmoid(z1f)

@@ -410,3 +410,49 @@ def test_wgrad_operands_are_checked():
             F.bias_grad(dy, False)
     with pytest.raises(ValueError, match="dequant"):
         F.dequant(torch.zeros(4, dtype=torch.uint8), one)
+
+
+def _saving(fn, forward):
+    """An autograd Function with fn's backward, and a forward that saves what fn's would and returns `forward`'s result."""
+    class Saved(torch.autograd.Function):
+        backward = staticmethod(fn.backward)
+
+        @staticmethod
+        def forward(ctx, *ins):
+            saved, attrs, y = forward(*ins)
+            ctx.save_for_backward(*saved)
+            for k, v in attrs.items():
+                setattr(ctx, k, v)
+            return y
+    return Saved
+
+
+def test_batched_gradients_of_the_bf16_backward():
+    """The recipe "native" takes a batch of output gradients (is_grads_batched, a vectorized jacobian): its backward is then
+    torch's operations, one gradient of the batch as it comes alone."""
+    B16 = torch.bfloat16
+    g = torch.Generator().manual_seed(0)
+    r = lambda *s: torch.randn(*s, generator=g)
+    x, w, b = r(6, 32).to(B16).requires_grad_(), r(48, 32).requires_grad_(), r(48).requires_grad_()
+    lin = _saving(F._Fp8Linear, lambda x, w, b: ((x, w), dict(has_b=True, shape=x.shape, wdt=w.dtype),
+                                                 (x.float() @ w.t() + b).to(B16)))
+    y, dy = lin.apply(x, w, b), r(5, 6, 48).to(B16)
+    for got, want in zip(torch.autograd.grad(y, (x, w, b), dy, is_grads_batched=True, retain_graph=True),
+                         ([d @ w.detach().to(B16) for d in dy], [(d.t() @ x.detach()).float() for d in dy],
+                          [d.sum(0).float() for d in dy])):
+        torch.testing.assert_close(got, torch.stack(want), rtol=1e-2, atol=1e-2)
+    z, w3 = r(6, 64).to(B16).requires_grad_(), r(48, 32).requires_grad_()
+    aq, sa = r(6, 32).to(F.E4), torch.tensor([0.5])
+    mlp = _saving(F._SwiGLUw3, lambda z, w3: ((z, aq, sa, w3), dict(shape=z.shape, wdt=w3.dtype),
+                                              (aq.float() @ w3.t()).to(B16)))
+    y = mlp.apply(z, w3)
+    dz, dw3 = torch.autograd.grad(y, (z, w3), dy, is_grads_batched=True, retain_graph=True)
+    a = (aq.float() * sa).to(B16)
+    torch.testing.assert_close(dw3, torch.stack([(d.t() @ a).float() for d in dy]), rtol=1e-2, atol=1e-2)
+    for i, d in enumerate(dy):
+        z1, z2 = (t.float().requires_grad_() for t in z.detach().chunk(2, dim=-1))
+        da = (d @ w3.detach().to(B16)).float()
+        want = torch.cat(torch.autograd.grad(nn.functional.silu(z1) * z2, (z1, z2), da), dim=-1)
+        torch.testing.assert_close(dz[i].float(), want, rtol=2e-2, atol=2e-2)
+    jac = torch.autograd.functional.jacobian(lambda w: lin.apply(x.detach(), w, b.detach()).float(), w.detach(), vectorize=True)
+    assert jac.shape == (6, 48, 48, 32)
