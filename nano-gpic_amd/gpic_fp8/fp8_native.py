@@ -643,8 +643,17 @@ def _bias_grad(dy, dtype):
     return dy.sum(0).to(dtype) if _torch_ops(dy) else L.call(bias_grad, dy, dtype == torch.float32).to(dtype)
 
 
+# The ops that a joint call (cast_group, fp8_wgrad, the host module's whole linears) does the work of: it is made only while
+# each of them is in its place, since a stand-in put there is called as it is.
+_CAST_OPS = (tcast, tcast_t)
+_FWD_OPS = (tcast, tcast_t, cast_group, fp8_gemm)
+_BWD_OPS = (tcast, fp8_gemm, fp8_gemm_mn, fp8_wgrad, bias_grad)
+
+
 def _wgrad8(a, sa, b, sb, dtype):
     """fp8_gemm_mn(a, sa, b, sb).to(dtype)."""
+    if fp8_gemm_mn is not _BWD_OPS[2]:
+        return L.call(fp8_gemm_mn, a, sa, b, sb).to(dtype)
     return L.call(fp8_wgrad, a, sa, b, sb, dtype == torch.float32).to(dtype)
 
 
@@ -672,6 +681,13 @@ def _mm(xq, sx, wq, sw, fast=True):
 
 def _cast_xw(x2, *ws, kind):
     """x2's (q, dequant) and each weight's cast_group triple, cast together."""
+    if (tcast, tcast_t) != _CAST_OPS:
+        def one(w):
+            if kind != FLAT:
+                return tuple(L.call(tcast_t, w, kind == BOTH))
+            q, s = L.call(tcast, w)
+            return q, q.new_empty(0), s
+        return *L.call(tcast, x2), *map(one, ws)
     o = L.call(cast_group, [x2, *ws], [FLAT] + [kind] * len(ws))
     return o[0], o[2], *(tuple(o[3 * i:3 * i + 3]) for i in range(1, len(ws) + 1))
 
@@ -679,9 +695,10 @@ def _cast_xw(x2, *ws, kind):
 def _linear_fwd(x2, w, b, kind):
     """The forward of a linear: (y, xq, sx, wqt, sw), the weight cast with x in one launch (kind BOTH: wqt its transposed
     bytes, FLAT: an empty tensor)."""
-    r = L.native("linear_fwd", x2, x2, w, b, kind == BOTH)
-    if r is not None:
-        return r
+    if (tcast, tcast_t, cast_group, fp8_gemm) == _FWD_OPS:
+        r = L.native("linear_fwd", x2, x2, w, b, kind == BOTH)
+        if r is not None:
+            return r
     xq, sx, (wq, wqt, sw) = _cast_xw(x2, w, kind=kind)
     return L.call(fp8_gemm, xq, sx, wq, sw, b), xq, sx, wqt, sw
 
@@ -689,7 +706,9 @@ def _linear_fwd(x2, w, b, kind):
 def _linear_bwd(dy2, xq, sx, wqt, sw, has_b, dtype):
     """The phase-3 backward of a linear: (dx [M, K] = [M, N] . [K, N]^T, dw [N, K] = [M, N]^T . [M, K], db or None)."""
     # (a backward that is itself recorded: the bias gradient is then a differentiable operation)
-    r = None if has_b and _torch_ops(dy2) else L.native("linear_bwd", dy2, dy2, xq, sx, wqt, sw, has_b, dtype == torch.float32)
+    r = None
+    if (tcast, fp8_gemm, fp8_gemm_mn, fp8_wgrad, bias_grad) == _BWD_OPS and not (has_b and _torch_ops(dy2)):
+        r = L.native("linear_bwd", dy2, dy2, xq, sx, wqt, sw, has_b, dtype == torch.float32)
     if r is not None:
         dx, dw, db = r
         return dx, dw.to(dtype), None if db is None else db.to(dtype)

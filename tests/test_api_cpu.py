@@ -456,3 +456,49 @@ def test_batched_gradients_of_the_bf16_backward():
         torch.testing.assert_close(dz[i].float(), want, rtol=2e-2, atol=2e-2)
     jac = torch.autograd.functional.jacobian(lambda w: lin.apply(x.detach(), w, b.detach()).float(), w.detach(), vectorize=True)
     assert jac.shape == (6, 48, 48, 32)
+
+
+@pytest.mark.parametrize("name", ["tcast", "tcast_t", "cast_group", "fp8_gemm", "fp8_gemm_mn", "fp8_wgrad", "bias_grad"])
+@torch.no_grad()   # (as inside an autograd Function)
+def test_stand_ins_for_ops_are_called(monkeypatch, name):
+    """A stand-in put in an op's place is called for a linear's forward and backward, where the native host module would
+    otherwise take the whole call (here one that answers every call of it)."""
+    from gpic_fp8 import _lib as L
+    T = torch
+    q = lambda t: t.to(F.E4)
+    plain = dict(
+        tcast=lambda x: (q(x), T.ones(1)),
+        tcast_t=lambda x, want_q=True: (q(x) if want_q else q(x[:0, 0]), q(x).view(T.uint8).t().contiguous().view(F.E4), T.ones(1)),
+        cast_group=lambda xs, ks: [t for x, k in zip(xs, ks) for t in (q(x), q(x.t().contiguous()) if k else q(x[:0, 0]), T.ones(1))],
+        fp8_gemm=lambda a, sa, b, sb, bias=None, fast=True: (a.float() @ b.float().t() + (0 if bias is None else bias)).bfloat16(),
+        fp8_gemm_mn=lambda a, sa, b, sb, bias=None: (a.float().t() @ b.float()).bfloat16(),
+        fp8_wgrad=lambda a, sa, b, sb, f32: (a.float().t() @ b.float()).to(T.float32 if f32 else T.bfloat16),
+        bias_grad=lambda dy, f32: dy.float().sum(0))
+    took, called = [], []
+
+    def native(fn, t, *args):
+        took.append(fn)
+        return None
+    monkeypatch.setattr(L, "native", native)
+    own = {getattr(F, n): n for n in plain}
+    monkeypatch.setattr(L, "call", lambda op, *a: plain[own[op]](*a) if op in own else op(*a))
+
+    def stand_in(*a):
+        called.append(name)
+        return plain[name](*a)
+    x, w = torch.ones(8, 16, dtype=torch.bfloat16), torch.ones(32, 16)
+    for kind in (F.FLAT, F.BOTH):
+        F._linear_fwd(x, w, None, kind)
+    y, xq, sx, wqt, sw = F._linear_fwd(x, w, None, F.BOTH)
+    dy = torch.ones(8, 32, dtype=torch.bfloat16)
+    want = F._linear_bwd(dy, xq, sx, wqt, sw, True, torch.float32)
+    assert "linear_fwd" in took and "linear_bwd" in took   # (its own ops in place: the module is asked)
+    took.clear()
+    monkeypatch.setattr(F, name, stand_in)
+    for kind in (F.FLAT, F.BOTH):
+        assert torch.equal(F._linear_fwd(x, w, None, kind)[0], y)
+    got = F._linear_bwd(dy, xq, sx, wqt, sw, True, torch.float32)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert called
+    assert ("linear_fwd" in took) == (name not in ("tcast", "tcast_t", "cast_group", "fp8_gemm"))
+    assert ("linear_bwd" in took) == (name not in ("tcast", "fp8_gemm", "fp8_gemm_mn", "fp8_wgrad", "bias_grad"))
