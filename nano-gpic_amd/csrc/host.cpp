@@ -6,7 +6,8 @@
 // Every function takes tensors of the usual form only (on the current device, contiguous, 16-byte aligned, the types
 // the C ABI takes) and returns None for any other, for which the caller runs its general form. Outputs are ordinary
 // tensors of torch's allocator on the current stream, as the general form's. dev, ws, stream: the current device, its
-// current stream's cast workspace and that stream.
+// current stream's cast workspace (0 for the calls that cast nothing) and that stream. The GIL is released while a call
+// allocates and launches, as ctypes and torch's own operations release it: a launch waits where the queue is full.
 #include <ATen/ATen.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/utils/pybind.h>
@@ -130,8 +131,20 @@ at::Tensor gemm_mn(const at::Tensor &a, const at::Tensor &sa, const at::Tensor &
   return c;
 }
 
+at::Tensor bias_grad(const at::Tensor &dy, bool f32, void *stream) {
+  const int64_t M = dy.size(0), N = dy.size(1);
+  const size_t bytes = gpic_fp8_bias_grad_workspace_bytes(M, N);
+  at::Tensor part = make(dy, {std::max<int64_t>((int64_t)bytes, 16)}, at::kByte);
+  at::Tensor db = make(dy, {N}, f32 ? at::kFloat : at::kBFloat16);
+  check(gpic_fp8_bias_grad(ptr<uint16_t>(dy), N, M, N, db.data_ptr(), f32 ? GPIC_DTYPE_F32 : GPIC_DTYPE_BF16,
+                           part.data_ptr(), bytes, stream),
+        "gpic_fp8_bias_grad");
+  return db;
+}
+
 typedef uintptr_t handle;
 void *vp(handle h) { return reinterpret_cast<void *>(h); }
+typedef py::gil_scoped_release NoGil;
 
 py::object casts(const std::vector<at::Tensor> &xs, const std::vector<int> &kinds, int dev, handle ws, handle stream) {
   const int n = (int)xs.size();
@@ -142,7 +155,10 @@ py::object casts(const std::vector<at::Tensor> &xs, const std::vector<int> &kind
     p[i] = &xs[i];
   }
   Casts o;
-  cast_group(n, p, kinds.data(), vp(ws), vp(stream), o);
+  {
+    NoGil no_gil;
+    cast_group(n, p, kinds.data(), vp(ws), vp(stream), o);
+  }
   py::list out;
   for (int i = 0; i < n; i++) {
     out.append(o.q[i]);
@@ -157,13 +173,23 @@ py::object gemm(const at::Tensor &a, const at::Tensor &sa, const at::Tensor &b, 
   if (!operand(a, sa, dev) || !operand(b, sb, dev) || a.size(1) != b.size(1) || b.size(0) % 16 ||
       !bias_ok(bias, b.size(0), dev))
     return py::none();
-  return py::cast(gemm_tn(a, sa, b, sb, bias, vp(stream)));
+  at::Tensor c;
+  {
+    NoGil no_gil;
+    c = gemm_tn(a, sa, b, sb, bias, vp(stream));
+  }
+  return py::cast(c);
 }
 
 py::object wgrad(const at::Tensor &a, const at::Tensor &sa, const at::Tensor &b, const at::Tensor &sb, bool f32, int dev,
                  handle, handle stream) {
   if (!operand(a, sa, dev) || !operand(b, sb, dev) || !wgrad_ok(a, b)) return py::none();
-  return py::cast(gemm_mn(a, sa, b, sb, f32, vp(stream)));
+  at::Tensor c;
+  {
+    NoGil no_gil;
+    c = gemm_mn(a, sa, b, sb, f32, vp(stream));
+  }
+  return py::cast(c);
 }
 
 // x [M, K] bf16, w [N, K], bias [N] or None -> y [M, N], and x's and w's casts: (y, xq, sx, wqt, sw), w's
@@ -176,8 +202,12 @@ py::object linear_fwd(const at::Tensor &x, const at::Tensor &w, const std::optio
   const at::Tensor *p[2] = {&x, &w};
   const int kinds[2] = {kFlat, both ? kBoth : kFlat};
   Casts o;
-  cast_group(2, p, kinds, vp(ws), vp(stream), o);
-  at::Tensor y = gemm_tn(o.q[0], o.s[0], o.q[1], o.s[1], bias, vp(stream));
+  at::Tensor y;
+  {
+    NoGil no_gil;
+    cast_group(2, p, kinds, vp(ws), vp(stream), o);
+    y = gemm_tn(o.q[0], o.s[0], o.q[1], o.s[1], bias, vp(stream));
+  }
   return py::make_tuple(y, o.q[0], o.s[0], o.qt[1], o.s[1]);
 }
 
@@ -191,19 +221,17 @@ py::object linear_bwd(const at::Tensor &dy, const at::Tensor &xq, const at::Tens
     return py::none();
   const at::Tensor *p[1] = {&dy};
   const int kinds[1] = {kFlat};
-  Casts o;
-  cast_group(1, p, kinds, vp(ws), vp(stream), o);
-  const at::Tensor &dyq = o.q[0], &sdy = o.s[0];
-  at::Tensor dx = gemm_tn(dyq, sdy, wqt, sw, std::nullopt, vp(stream));
-  at::Tensor dw = gemm_mn(dyq, sdy, xq, sx, f32, vp(stream));
+  at::Tensor dx, dw, db;
+  {
+    NoGil no_gil;
+    Casts o;
+    cast_group(1, p, kinds, vp(ws), vp(stream), o);
+    const at::Tensor &dyq = o.q[0], &sdy = o.s[0];
+    dx = gemm_tn(dyq, sdy, wqt, sw, std::nullopt, vp(stream));
+    dw = gemm_mn(dyq, sdy, xq, sx, f32, vp(stream));
+    if (has_bias) db = bias_grad(dy, f32, vp(stream));
+  }
   if (!has_bias) return py::make_tuple(dx, dw, py::none());
-  const int64_t M = dy.size(0), N = dy.size(1);
-  const size_t bytes = gpic_fp8_bias_grad_workspace_bytes(M, N);
-  at::Tensor part = make(dy, {std::max<int64_t>((int64_t)bytes, 16)}, at::kByte);
-  at::Tensor db = make(dy, {N}, f32 ? at::kFloat : at::kBFloat16);
-  check(gpic_fp8_bias_grad(ptr<uint16_t>(dy), N, M, N, db.data_ptr(), f32 ? GPIC_DTYPE_F32 : GPIC_DTYPE_BF16,
-                           part.data_ptr(), bytes, vp(stream)),
-        "gpic_fp8_bias_grad");
   return py::make_tuple(dx, dw, db);
 }
 

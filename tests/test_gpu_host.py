@@ -135,3 +135,45 @@ def test_gemm_first_on_a_capturing_stream(dev, monkeypatch):
     first.replay()
     torch.cuda.synchronize()
     assert torch.equal(got[0], c) and torch.equal(got[1], w)
+
+
+@pytest.mark.parametrize("name", ["casts", "gemm", "wgrad", "linear_fwd", "linear_bwd"])
+def test_other_threads_run_during_a_call(dev, name):
+    """The host module's calls release the GIL: a second Python thread, which with this switch interval never gets it unless
+    the first gives it up, counts while the first does nothing but call the module."""
+    import sys
+    import threading
+    import time
+    index, stream = torch.cuda.current_device(), torch.cuda.current_stream().cuda_stream
+    ws = L.cast_workspace(dev).data_ptr()
+    x, w = torch.randn(64, 64, device=dev).to(B16), torch.randn(64, 64, device=dev)
+    q, s = x.to(G.E4), torch.ones(1, device=dev)
+    f = getattr(L.host(), name)
+    args = {"casts": ([x, w], [F.FLAT, F.BOTH]), "gemm": (q, s, q, s, None), "wgrad": (q, s, q, s, True),
+            "linear_fwd": (x, w, None, True), "linear_bwd": (x, q, s, q, s, True, True)}[name]
+    count, running, stop = [0], threading.Event(), False
+
+    def other():
+        running.set()
+        while not stop:
+            count[0] += 1
+            time.sleep(0)   # gives the GIL up
+    t = threading.Thread(target=other)
+    interval = sys.getswitchinterval()
+    try:
+        t.start()
+        running.wait()
+        sys.setswitchinterval(60.0)
+        end = time.monotonic() + 0.1
+        while time.monotonic() < end:   # (the other thread's wait that began under the old interval ends here)
+            pass
+        n, kept = count[0], []   # (results kept: freeing a tensor may give the GIL up as well)
+        for _ in range(1000):
+            kept.append(f(*args, index, ws, stream))
+        got = count[0] - n
+    finally:
+        sys.setswitchinterval(interval)
+        stop = True
+        t.join()
+    torch.cuda.synchronize()
+    assert all(r is not None for r in kept) and got >= 500   # (several a call; none where the GIL is held)
