@@ -863,6 +863,23 @@ static Plan plan_gemm(int64_t M, int64_t N, int64_t K) {
   return ktiles > 0 && tbest[1] < kNarrowGain * tbest[0] ? best[1] : best[0];
 }
 
+// plan_gemm through the plans of each thread's last shapes (at most 2^kPlanBits of them): the search, up to 128 candidates,
+// takes 0.5 us of host time for a long K, and a call wants it twice, for the workspace's size and for the launch.
+constexpr int kPlanBits = 6;
+static Plan plan_of(int64_t M, int64_t N, int64_t K) {
+  struct Entry {
+    int64_t M, N, K;
+    int cus;   // (0: empty)
+    Plan p;
+  };
+  static thread_local Entry plans[1 << kPlanBits];
+  const int cus = num_cus();
+  constexpr uint64_t kMul = 0x9E3779B97F4A7C15u;   // (2^64 over the golden ratio: spreads a product over its top bits)
+  Entry &e = plans[((((uint64_t)M * kMul + (uint64_t)N) * kMul + (uint64_t)K) * kMul) >> (64 - kPlanBits)];
+  if (e.M != M || e.N != N || e.K != K || e.cus != cus) e = Entry{M, N, K, cus, plan_gemm(M, N, K)};
+  return e.p;
+}
+
 template <int kSM, int kSN, int kSS>
 static void launch_small(const void *A, int64_t lda, const float *sa, const void *B, int64_t ldb, const float *sb,
                          const void *bias, int bias32, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K,
@@ -909,7 +926,7 @@ static int launch_gemm(const void *A, int64_t lda, const float *sa, const void *
   if (K > 0 && (!A || !B)) return GPIC_EINVAL;
   if (!aligned16(A) || !aligned16(B) || !aligned16(C) || (bias && ((uintptr_t)bias & (bias32 ? 15u : 7u)))) return GPIC_EALIGN;
   // (a K tile is 128 bytes of each operand's K: the plan of a byte matrix kEl times as long)
-  Plan p = K > 0 ? plan_gemm(M, N, K * kEl) : Plan{(int)((M + kBM - 1) / kBM), (int)((N + kBN - 1) / kBN), 1, kBK, kBN};
+  Plan p = K > 0 ? plan_of(M, N, K * kEl) : Plan{(int)((M + kBM - 1) / kBM), (int)((N + kBN - 1) / kBN), 1, kBK, kBN};
   const bool far = kMN && std::max(lda, ldb) > kMaxDescLd;   // (K x ld is below 2^31 bytes: one K tile, never split)
   if (far) p = Plan{(int)((M + kBM - 1) / kBM), (int)((N + kBN - 1) / kBN), 1, kBK, kBN};
   float *P = nullptr;
@@ -955,7 +972,7 @@ extern "C" {
 
 size_t gpic_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const Plan p = plan_gemm(M, N, K);
+  const Plan p = plan_of(M, N, K);
   return p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
 }
 

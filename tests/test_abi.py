@@ -203,3 +203,23 @@ def test_only_casting_calls_get_a_cast_workspace(monkeypatch):
         assert L.native(name, t, "a") == ("a", 0, 0, 5) and not made
     for name in ("casts", "linear_fwd", "linear_bwd"):
         assert L.native(name, t, "a") == ("a", 0, 77, 5) and made.pop()
+
+
+def test_gemm_plans_are_kept():
+    """A shape's plan is searched once: its workspace size is the same however many other shapes, and threads, came between,
+    and asking again costs no search (a short K's search is a few candidates, a long K's over a hundred)."""
+    import threading
+    import timeit
+    f = L.lib().gpic_fp8_gemm_workspace_bytes
+    shapes = [(m, n, k) for m in (1, 64, 511, 1024, 8192) for n in (16, 768, 1024, 3072) for k in
+              (16, 128, 1024, 1040, 3072, 4096, 8192, 16384, 32768)]
+    first = {}
+    t = threading.Thread(target=lambda: first.update({s: f(*s) for s in shapes}))   # (its own, empty, plans)
+    t.start()
+    t.join()
+    for order in (shapes, shapes[::-1], shapes[::7] * 3):
+        assert [f(*s) for s in order] == [first[s] for s in order]
+    for m, n, k in shapes:   # whole fp32 partials: splits x M x N
+        assert first[m, n, k] % (4 * m * n) == 0 and first[m, n, k] // (4 * m * n) != 1
+    cost = lambda *s: min(timeit.repeat(lambda: f(*s), number=5000, repeat=9))
+    assert cost(1024, 1024, 32768) < 1.3 * cost(64, 64, 128)
