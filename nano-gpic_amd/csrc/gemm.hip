@@ -885,10 +885,37 @@ static void launch_small(const void *A, int64_t lda, const float *sa, const void
                          const void *bias, int bias32, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K,
                          const Plan &p, hipStream_t st) {
   const int tiles_n = (int)((N + kSN - 1) / kSN), tiles = (int)((M + kSM - 1) / kSM) * tiles_n;
-  auto *kernel = p.splits > 1 ? (K % kBK ? gemm_small_kernel<kSM, kSN, kSS, true, true> : gemm_small_kernel<kSM, kSN, kSS, false, true>)
-                              : (K % kBK ? gemm_small_kernel<kSM, kSN, kSS, true, false> : gemm_small_kernel<kSM, kSN, kSS, false, false>);
+  auto *kernel = K % kBK ? gemm_small_kernel<kSM, kSN, kSS, true, false> : gemm_small_kernel<kSM, kSN, kSS, false, false>;
+  if constexpr (kSM < 128)   // (the largest tile takes no split plan)
+    if (p.splits > 1) kernel = K % kBK ? gemm_small_kernel<kSM, kSN, kSS, true, true> : gemm_small_kernel<kSM, kSN, kSS, false, true>;
   kernel<<<tiles, 256, 0, st>>>(static_cast<const uint8_t *>(A), (int)lda, static_cast<const uint8_t *>(B), (int)ldb, sa,
                                 sb, bias, bias32, C, ldc, (int)M, (int)N, (int)K, tiles_n, p.ksplit / kBK);
+}
+
+// Millions of bytes that the eight XCDs read for t small-class tiles of sm x 64 in xcd_remap's order: each, through its own
+// L2, the columns of B and the rows of A of its contiguous run of tiles.
+static double small_traffic(int64_t sm, int64_t t, int64_t M, int64_t N, int64_t K) {
+  const int64_t run = (t + 7) / 8, n64 = (N + 63) / 64;
+  return 8e-6 * (double)K * (double)(std::min(N, 64 * run) + std::min(M, sm * (1 + (run + n64 - 1) / n64)));
+}
+
+// Whether the small class (t tiles of sm x 64) is expected to beat a plan that splits K by 5% or more. Its chain is one K
+// tile after another and a fold a split, whatever the rows; the plan's is its longest split, the launch and latency of the
+// reduce, which reads a split after another, and the partials' bytes. Both fitted, in us, to 1104 shapes that both can run
+// (1-3000 rows, 16-14336 columns, K 2048-8192; 7% rms), the last term of the 64-row tile then raised from 0.165 so that close
+// calls stay with the plan. Taken wherever its tiles fit, the small class lost more than 3% to the plan on 276 of them:
+// few rows ([16 x 1024 x 8192] 23.5 us against 16.7, [24 x 1536 x 6144] 17.2 / 12.7), and a large B that every XCD streams
+// ([256 x 3072 x 8192] 31.5 / 22.1, [1388 x 1728 x 7056] 54.4 / 38.0; past 128 MB no formula held). Under this rule on 3, by
+// 7% at most, and on the 621 that it takes it is 1.37x as fast ([512 x 768 x 3072] 9.2 us against 17.8, [2048 x 1024 x 4096]
+// 18.0 / 27.6). The fit ends at K = 8192.
+static bool small_beats_split(const Plan &p, int64_t sm, int64_t t, int64_t M, int64_t N, int64_t K) {
+  const double mb = small_traffic(sm, t, M, N, K);
+  if (K > 8192 || mb > 128.0) return false;
+  const double kt = (double)((K + kBK - 1) / kBK), s = p.splits, fill = kt * (double)t / num_cus();
+  const double small = sm == 32 ? 2.2 + 0.21 * kt + 0.19 * s + 0.042 * mb + 0.034 * fill
+                                : 3.7 + 0.06 * kt + 0.25 * s + 0.05 * mb + 0.22 * fill;
+  const double plan = 7.0 + 0.87 * (p.ksplit / kBK) + 0.21 * s + 1.71e-6 * s * (double)M * (double)N;
+  return small < 0.95 * plan;
 }
 
 // The small class where its tiles are few enough for the device (false, nothing launched, otherwise). The limits are
@@ -897,21 +924,27 @@ static void launch_small(const void *A, int64_t lda, const float *sa, const void
 //   [1024 x 3072] 32 x 64 9.7 (6), 64 x 64 7.7 (3), 128 x 64 8.2, 256 x 128 10.7;   [2048 x 1024] 7.6, 5.9 (2), 6.6, 10.2
 //   [4096 x 1024] 64 x 64 9.9 (4), 128 x 64 8.4 (2), 128 x 128 9.2, 256 x 128 11.0
 //   [2048 x 3072] 64 x 64 13.0 (6), 128 x 64 13.0 (3), 256 x 128 11.7: past these the bytes a small tile reads per flop
-//   (through L2) cost more than its latency saves.
-// Plans that split K (their partials and the reduce's launch fall away; 32 x 64 / 64 x 64 / 128 x 64 against the plan):
-//   [512 x 768 x 3072] 9.2 / 11.6 / 16.0 us, 17.8;   [1024 x 1024 x 8192] 24.8 / 27.2 / 36.1, 27.1;
-//   [2048 x 1024 x 4096] 25.9 / 18.0 / 20.7, 27.6;   [4096 x 768 x 6144] 49.7 / 34.8 / 34.4, 39.0;
-//   [1632 x 1280 x 10240] 65.8 / 46.9 / 50.0, 42.7: a long K is worth the splits' CUs, so they end at K = 8192.
+//   (through L2) cost more than its latency saves -- for 64 x 64 tiles above 2 a CU already where the XCDs read more than
+//   110 MB ([512 x 6144 x 2560] 22.2 us against 20.2, [512 x 6144 x 4608] 35.6 / 32.2; [800 x 3072 x 4096], 107 MB, 24.7 / 28.9).
+// Plans that split K take the 32 x 64 or 64 x 64 tile where small_beats_split says so (their partials and the reduce's
+// launch fall away).
 static bool launch_small_class(const void *A, int64_t lda, const float *sa, const void *B, int64_t ldb, const float *sb,
                                const void *bias, int bias32, uint16_t *C, int64_t ldc, int64_t M, int64_t N, int64_t K,
                                const Plan &p, hipStream_t st) {
   const int64_t cus = num_cus(), n64 = (N + 63) / 64, t32 = (M + 31) / 32 * n64, t64 = (M + 63) / 64 * n64,
                 t128 = (M + 127) / 128 * n64;
-  if (p.splits > 1 && K > 8192) return false;
-  if (t32 <= 2 * cus) launch_small<32, 64, 4>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, p, st);
-  else if (t64 <= 3 * cus) launch_small<64, 64, 3>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, p, st);
-  else if (t128 <= 2 * cus) launch_small<128, 64, 3>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, p, st);
-  else return false;
+  const bool split = p.splits > 1;
+  if (t32 <= 2 * cus) {
+    if (split && !small_beats_split(p, 32, t32, M, N, K)) return false;
+    launch_small<32, 64, 4>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, p, st);
+  } else if (t64 <= 3 * cus && (split || t64 <= 2 * cus || small_traffic(64, t64, M, N, K) <= 110.0)) {
+    if (split && !small_beats_split(p, 64, t64, M, N, K)) return false;
+    launch_small<64, 64, 3>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, p, st);
+  } else if (t128 <= 2 * cus && !split) {
+    launch_small<128, 64, 3>(A, lda, sa, B, ldb, sb, bias, bias32, C, ldc, M, N, K, p, st);
+  } else {
+    return false;
+  }
   return true;
 }
 

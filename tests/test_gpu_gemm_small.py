@@ -37,3 +37,34 @@ def test_small_gemm(dev, M, N, K, bias):
     if m16:
         t = lambda u: u.contiguous().view(torch.uint8).t().contiguous().view(G.E4)
         assert torch.equal(y[:m16], G.fp8_gemm_mn(t(a[:m16]), sa, t(b), sb, bi))
+
+
+def _device_us(f):
+    """The device time of f: the median of 9 replays of a graph of 20 launches."""
+    f()
+    torch.cuda.synchronize()
+    graph, times = torch.cuda.CUDAGraph(), []
+    with torch.cuda.graph(graph):
+        for _ in range(20):
+            f()
+    for _ in range(9):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        graph.replay()
+        end.record()
+        torch.cuda.synchronize()
+        times.append(start.elapsed_time(end) * 1e3 / 20)
+    return sorted(times)[4]
+
+
+@pytest.mark.parametrize("M,N,K,most", [(16, 64, 8192, 1.15), (16, 1024, 8192, 1.15), (16, 1536, 6144, 1.15),
+                                        (256, 3072, 8192, 1.15), (512, 6144, 4608, 0.95)])
+def test_small_class_only_where_it_pays(dev, M, N, K, most):
+    """Few rows of a long K, and small tiles that would stream a large B: no slower than the plan, whose time is taken from
+    the MN-major layout's, which never has another class. (Measured ratios: 1.0 for split plans, 0.79 for the last, whose
+    MN-major form is the slower one; with the small class 1.31-1.41, and 1.05.)"""
+    g = torch.Generator(device=dev).manual_seed(K)
+    a, b = (torch.randn(n, K, generator=g, device=dev).to(G.E4) for n in (M, N))
+    at, bt = (t.view(torch.uint8).t().contiguous().view(G.E4) for t in (a, b))
+    s = torch.ones(1, device=dev)
+    assert _device_us(lambda: G.fp8_gemm(a, s, b, s)) < most * _device_us(lambda: G.fp8_gemm_mn(at, s, bt, s))
