@@ -1190,16 +1190,16 @@ __device__ __forceinline__ void cast_once_run(const T *__restrict__ x, int64_t n
   };
   uint32_t m0 = max(words_amax<T, kW>(w), tail_amax());
   if (sgroups > 0) m0 = max(m0, stream_amax(blk));
-  const uint32_t m = block_max_u32(m0);
+  const uint32_t m = block_max_u32<256>(m0);
   uint32_t tk;
-  const uint32_t g = once_fold_range(m, ws, ep, wait_ticks, tk, first, (int)G, [&](int c) {
+  const uint32_t g = once_fold_range<256>(m, ws, ep, wait_ticks, tk, first, (int)G, [&](int c) {
     uint32_t a = tail_amax();
     for (int j = 0; j < wpt; j++) {
       const int64_t i = word(c, j);
       if (i < nw) a = max(a, word_amax_exact<T>(__builtin_nontemporal_load(xv + map(i))));
     }
     if (sgroups > 0) a = max(a, stream_amax(c));
-    return block_max_u32(a);
+    return block_max_u32<256>(a);
   });
   hold(w);
   float scale, deq;
@@ -1289,7 +1289,7 @@ __device__ __forceinline__ void cast_t_once_run(const T *__restrict__ x, int64_t
       m = max(m, words_amax<T, L::kW>(S));
     }
   uint32_t tk;
-  const uint32_t g = once_fold_range(block_max_u32(m), ws, ep, wait_ticks, tk, first, (int)G, [&](int c) {
+  const uint32_t g = once_fold_range<256>(block_max_u32<256>(m), ws, ep, wait_ticks, tk, first, (int)G, [&](int c) {
     uint32_t a = 0;
     for (int64_t t = c; t < tiles; t += G) {
       const int64_t r0 = r0_of(t), c0 = c0_of(t);
@@ -1299,7 +1299,7 @@ __device__ __forceinline__ void cast_t_once_run(const T *__restrict__ x, int64_t
         if (gr < rows && gc < cols) a = max(a, word_amax_exact<T>(*reinterpret_cast<const u32x4 *>(x + gr * ld + gc)));
       }
     }
-    return block_max_u32(a);
+    return block_max_u32<256>(a);
   });
   hold(R);
   float scale, deq;

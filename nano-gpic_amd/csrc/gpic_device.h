@@ -131,10 +131,13 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// kThreads: blockDim.x where it is known: read from the launch's arguments it costs a load, and a loop, on the way to the
+// fold (flat single-pass cast of 15.7M bf16 elements 11.67 -> 10.68 us, of 10.5M fp32 10.81 -> 9.65).
+template <int kThreads = 0>
 __device__ __forceinline__ uint32_t block_max_u32(uint32_t v) {
   __shared__ uint32_t red[16];
   v = wave_max_u32(v);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (kThreads ? kThreads : blockDim.x) >> 6;
   lds_barrier();  // red[] may still be read by a previous call
   if (lane == 0) red[wave] = v;
   lds_barrier();

@@ -60,7 +60,8 @@ __device__ __forceinline__ uint32_t once_epoch(void *ws) {
 // counter is back at zero when the call ends.
 // once_fold_range: the same over the partials of workgroups [first, first + count) only (a launch that casts several
 // tensors, each over its own range of workgroups); share_max then takes the index within the range.
-template <class ShareMax>
+// kThreads: as block_max_u32's.
+template <int kThreads = 0, class ShareMax>
 __device__ __forceinline__ uint32_t once_fold_range(uint32_t m, void *ws, uint32_t epoch, uint32_t wait_ticks,
                                                     uint32_t &ticket, int first, int count, ShareMax share_max) {
   __shared__ int missing[kMaxOnceBlocks];
@@ -86,7 +87,7 @@ __device__ __forceinline__ uint32_t once_fold_range(uint32_t m, void *ws, uint32
   const uint32_t tag = stag;
   uint32_t g = m;
   const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-  for (int i = first + (int)threadIdx.x; i < first + count; i += blockDim.x) {
+  for (int i = first + (int)threadIdx.x; i < first + count; i += kThreads ? kThreads : blockDim.x) {
     uint64_t w = __hip_atomic_load(tagged + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     while ((uint32_t)(w >> 32) != tag && __builtin_amdgcn_s_memrealtime() - t0 < wait_ticks) {
       __builtin_amdgcn_s_sleep(2);
@@ -95,7 +96,7 @@ __device__ __forceinline__ uint32_t once_fold_range(uint32_t m, void *ws, uint32
     if ((uint32_t)(w >> 32) == tag) g = max(g, (uint32_t)w);
     else missing[atomicAdd(&nmissing, 1)] = i;
   }
-  g = block_max_u32(g);   // its barriers also publish `missing`
+  g = block_max_u32<kThreads>(g);   // its barriers also publish `missing`
   const int nm = nmissing;
   if (nm > 0) {
     // Waiters help each other: each starts at a different missing partial, computes it from x and publishes it (the
