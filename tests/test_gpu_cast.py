@@ -422,3 +422,34 @@ def test_tcast_t_hybrid_matches_two_pass(dev, rows, cols, single_pass_default):
     if (rows, cols) == (32768, 3072):
         oq, od, _ = O.tcast(bits(x.cpu()))
         assert s0 == od and np.array_equal(q0.cpu().numpy(), oq)
+
+
+def _device_us(f):
+    """The device time of f: the median of 9 replays of a graph of 20 launches."""
+    f()
+    torch.cuda.synchronize()
+    graph, times = torch.cuda.CUDAGraph(), []
+    with torch.cuda.graph(graph):
+        for _ in range(20):
+            f()
+    for _ in range(9):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        graph.replay()
+        end.record()
+        torch.cuda.synchronize()
+        times.append(start.elapsed_time(end) * 1e3 / 20)
+    return sorted(times)[4]
+
+
+@pytest.mark.parametrize("rows,cols", [(16, 16), (48, 64), (256, 256), (1024, 1024), (8192, 1024)])
+def test_transposing_fp32_single_pass_only_where_it_pays(dev, rows, cols):
+    """The transposing cast of fp32 takes no longer than its two passes, which small parts of one tile are left to."""
+    x = torch.randn(rows, cols, device=dev)
+    once = _device_us(lambda: G.tcast_t(x))
+    L.set_single_pass(False)
+    try:
+        two = _device_us(lambda: G.tcast_t(x))
+    finally:
+        L.set_single_pass(True, -1)
+    assert once < 1.08 * two
