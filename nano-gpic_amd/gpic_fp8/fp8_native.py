@@ -665,9 +665,20 @@ def _torch_ops(dy):
                                                   or not torch._C._has_storage(dy))
 
 
+def _library_wgrad(M, N, K, f32):
+    """Whether the library's dy.t() @ x, with the conversion for an fp32 weight, is the faster wgrad of [M, N] and [M, K]: for
+    few tokens and a small gradient, whose few tiles the kernel has to split over K and reduce. [1200, 1024 x 1024] 15.9 us
+    against the kernel's 20.9 (fp32 18.5 / 20.9), [2048, 1280 x 1280] 20.9 / 25.7, [2048, 1024 x 1024] 17.4 / 25.2 (20.0 / 25.5);
+    past the lines it is the other way: [3000, 1024 x 1024] ratio 0.85, [1200, 2304 x 1152] 0.92, fp32 [400, 1024 x 1024] 0.91.
+    (Gradients with a side below 512: the library's times vary threefold between neighbouring sizes, and 256 to 384 tiles
+    of 256 x 256 over 4096-8192 tokens lose up to 20% or gain up to 33%; no rule on sizes separates those.)"""
+    return M <= 2600 and min(N, K) >= 512 and (M >= 600 and N * K <= 1200000 if f32 else N * K <= 2200000)
+
+
 def _wgrad16(dy, x, dtype):
     """(dy.t() @ x).to(dtype)."""
-    if _torch_ops(dy):
+    if _torch_ops(dy) or (not torch.compiler.is_compiling()
+                          and _library_wgrad(dy.shape[0], dy.shape[1], x.shape[1], dtype == torch.float32)):
         return (dy.t() @ x).to(dtype)
     return L.call(bf16_wgrad, dy, x, dtype == torch.float32).to(dtype)
 

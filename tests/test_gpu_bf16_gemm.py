@@ -79,3 +79,32 @@ def test_e4m3_wgrad_f32_scales_and_errors(dev):
             F.fp8_wgrad(a, one, b[:48], one, f32)
     with pytest.raises(ValueError):
         F.bf16_wgrad(a.to(torch.bfloat16), b[:48].to(torch.bfloat16), True)
+
+
+@pytest.mark.parametrize("M,N,K,dt", [(1200, 1024, 1024, torch.bfloat16), (2048, 1280, 1280, torch.bfloat16),
+                                      (2048, 1024, 1024, torch.float32), (512, 768, 768, torch.bfloat16),
+                                      (4096, 1024, 1024, torch.bfloat16), (13303, 896, 1792, torch.float32)])
+def test_the_faster_wgrad_is_taken(dev, M, N, K, dt):
+    """A weight gradient of the bf16 backward: right either way, and its device time that of the faster of the kernel and
+    the library's product (with its conversion for an fp32 weight)."""
+    dy, x = torch.randn(M, N, device=dev).to(torch.bfloat16), torch.randn(M, K, device=dev).to(torch.bfloat16)
+
+    def us(f):   # the median of 9 replays of a graph of 20 launches
+        f()
+        torch.cuda.synchronize()
+        graph, times = torch.cuda.CUDAGraph(), []
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                f()
+        for _ in range(9):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            graph.replay()
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end) * 1e3 / 20)
+        return sorted(times)[4]
+    with torch.no_grad():
+        _check(F._wgrad16(dy, x, dt).to(torch.bfloat16), dy.t(), x, False)
+        got = us(lambda: F._wgrad16(dy, x, dt))
+        assert got < 1.1 * min(us(lambda: (dy.t() @ x).to(dt)), us(lambda: F.bf16_wgrad(dy, x, dt == torch.float32)))
