@@ -1830,7 +1830,7 @@ __global__ __launch_bounds__(kSwThreads) void cast_wide_kernel(const uint16_t *_
   };
   if (blockIdx.x < sgroups) m = max(m, stream_amax(blockIdx.x));
   uint32_t tk;
-  const uint32_t g = once_fold(block_max_u32(m), ws, ep, wait_ticks, tk, [&](int cb) {
+  const uint32_t g = once_fold_range<kSwThreads>(block_max_u32<kSwThreads>(m), ws, ep, wait_ticks, tk, 0, (int)G, [&](int cb) {
     uint32_t a = tail_amax();
     for (int j = 0; j < wpt; j++) {
       const uint32_t i = hword((uint32_t)cb, j);
@@ -1840,7 +1840,7 @@ __global__ __launch_bounds__(kSwThreads) void cast_wide_kernel(const uint16_t *_
       const uint32_t i = sword(s);
       if (i < nw) a = max(a, word_amax_exact<uint16_t>(__builtin_nontemporal_load(xv + map(i))));
     }
-    return block_max_u32(a);
+    return block_max_u32<kSwThreads>(a);
   });
   hold(w);
   float scale, deq;
