@@ -27,8 +27,8 @@ from typing import Optional
 import torch
 
 from . import _lib as L
-from .fp8_native import (BOTH, E4, Fp8LinearF8, _linear_bwd, _no_autocast, _wgrad8, cast_group, fp8_gemm, fp8_linear_f8,
-                         swiglu_bwd_q, swiglu_tcast, tcast, tcast_t)
+from .fp8_native import (BOTH, E4, Fp8LinearF8, _bias_grad, _linear_bwd, _no_autocast, _wgrad8, cast_group, fp8_gemm,
+                         fp8_gemm_mn, fp8_linear_f8, swiglu_bwd_q, swiglu_tcast, tcast, tcast_t)
 
 
 # The widest rows the backward kernel takes (its per-column sums live in registers); the forward takes any width.
@@ -170,10 +170,40 @@ def _(dh, dxn, xs, a, gate, w, scale, rstd):
             xs.new_empty(C, dtype=torch.float32), xs.new_empty(B, C), xs.new_empty(B, C))
 
 
+# The ops that a joint call (cast_group, the fp32 weight gradients, a whole linear's backward, the bf16 sums) does the work of:
+# it is made only while each of them is in its place here, since a stand-in put there is called as it is.
+_NORM_BWD = res_mod_rmsnorm_bwd_k
+_OWN = (tcast, tcast_t, fp8_gemm, fp8_gemm_mn)
+
+
+def _linear_backward(dy2, xq, sx, wqt, sw, has_b, dtype):
+    """fp8_native's _linear_bwd through this module's ops."""
+    if (tcast, tcast_t, fp8_gemm, fp8_gemm_mn) == _OWN:
+        return _linear_bwd(dy2, xq, sx, wqt, sw, has_b, dtype)
+    dyq, sdy = L.call(tcast, dy2)
+    dx = L.call(fp8_gemm, dyq, sdy, wqt, sw, None, False)
+    return dx, _weight_grad(dyq, sdy, xq, sx, dtype), _bias_grad(dy2, dtype) if has_b else None
+
+
+def _weight_grad(a, sa, b, sb, dtype):
+    """fp8_gemm_mn(a, sa, b, sb).to(dtype)."""
+    if fp8_gemm_mn is _OWN[3]:
+        return _wgrad8(a, sa, b, sb, dtype)
+    return L.call(fp8_gemm_mn, a, sa, b, sb).to(dtype)
+
+
+def _weight_casts(*ws):
+    """Each weight's tcast_t, all in one launch."""
+    if tcast_t is not _OWN[1]:
+        return [t for w in ws for t in L.call(tcast_t, w)]
+    return L.call(cast_group, list(ws), [BOTH] * len(ws))
+
+
 def _norm_backward(dh, dxn, xs, a, gate, w, shift, scale, rstd):
     """The norm site's backward: (dx, da or None, d_gate or None, d_w, d_shift, d_scale), the column sums fp32, or bf16
     (but d_w) where the whole modulation is bf16."""
-    bf16 = all(t is None or t.dtype == torch.bfloat16 for t in (gate, shift, scale))
+    bf16 = (res_mod_rmsnorm_bwd_k is _NORM_BWD
+            and all(t is None or t.dtype == torch.bfloat16 for t in (gate, shift, scale)))
     dx, da, dg, dw, dsh, dsc = L.call(res_mod_rmsnorm_bwd16 if bf16 else res_mod_rmsnorm_bwd_k, dh,
                                       dxn if a is not None else None, xs, a, gate, w, scale, rstd)
     if a is None:
@@ -312,7 +342,7 @@ class _Fp8ModRMSNormLinear(torch.autograd.Function):
         x, w_norm, shift, scale, rstd, hq2, sh, wqt, sw = ctx.saved_tensors
         B, N, C = x.shape
         dy2 = dy.reshape(B * N, -1).to(torch.bfloat16)
-        dh, dweight, db = _linear_bwd(dy2, hq2, sh, wqt, sw, ctx.has_b, ctx.wdt)
+        dh, dweight, db = _linear_backward(dy2, hq2, sh, wqt, sw, ctx.has_b, ctx.wdt)
         dx, _, _, dw, dsh, dsc = _norm_backward(dh.view(B, N, C), None, x, None, None, w_norm, shift, scale, rstd)
         _, dw, dshift, dscale = _param_grads(B, C, None, dw, dsh, dsc, None, w_norm, shift, scale)
         return dx, dw, dshift, dscale, None, dweight, db
@@ -328,7 +358,7 @@ class _Fp8ResModRMSNormMLP(torch.autograd.Function):
         _check_bwd_width(C, ctx)
         xn, _, hq, sh, rstd = L.call(res_mod_rmsnorm_q, x, a, gate, w_norm, shift, scale, eps, True, False)
         hq2 = hq.view(B * N, C)
-        w12q, w12qt, s12, w3q, w3qt, s3 = L.call(cast_group, [w12, w3], [BOTH, BOTH])
+        w12q, w12qt, s12, w3q, w3qt, s3 = _weight_casts(w12, w3)
         z = L.call(fp8_gemm, hq2, sh, w12q, s12)
         aq, sa = L.call(swiglu_tcast, z)
         y = L.call(fp8_gemm, aq, sa, w3q, s3)
@@ -343,10 +373,10 @@ class _Fp8ResModRMSNormMLP(torch.autograd.Function):
         dy2 = dy.reshape(B * N, -1).to(torch.bfloat16)
         dyq, sdy = L.call(tcast, dy2)
         da_ = L.call(fp8_gemm, dyq, sdy, w3qt, s3, None, False)
-        dw3 = _wgrad8(dyq, sdy, aq, sa, ctx.dt[1])
+        dw3 = _weight_grad(dyq, sdy, aq, sa, ctx.dt[1])
         dzq, sdz = L.call(swiglu_bwd_q, z, da_)
         dh = L.call(fp8_gemm, dzq, sdz, w12qt, s12, None, False).view(B, N, C)
-        dw12 = _wgrad8(dzq, sdz, hq2, sh, ctx.dt[0])
+        dw12 = _weight_grad(dzq, sdz, hq2, sh, ctx.dt[0])
         dx, da, dg, dw, dsh, dsc = _norm_backward(dh, dxn, xn, a, gate, w_norm, shift, scale, rstd)
         dgate, dw, dshift, dscale = _param_grads(B, C, dg, dw, dsh, dsc, gate, w_norm, shift, scale)
         return dx, da, dgate, dw, dshift, dscale, None, dw12, dw3

@@ -502,3 +502,60 @@ def test_stand_ins_for_ops_are_called(monkeypatch, name):
     assert called
     assert ("linear_fwd" in took) == (name not in ("tcast", "tcast_t", "cast_group", "fp8_gemm"))
     assert ("linear_bwd" in took) == (name not in ("tcast", "fp8_gemm", "fp8_gemm_mn", "fp8_wgrad", "bias_grad"))
+
+
+@pytest.mark.parametrize("name", ["tcast", "tcast_t", "fp8_gemm", "fp8_gemm_mn", "res_mod_rmsnorm_bwd_k"])
+@torch.no_grad()
+def test_stand_ins_for_the_norm_sites_ops_are_called(monkeypatch, name):
+    """The same for the linear and the MLP behind a norm site, whose module has the ops under its own names."""
+    from types import SimpleNamespace
+    from gpic_fp8 import _lib as L
+    from gpic_fp8 import norm as NM
+    T, B16 = torch, torch.bfloat16
+    q, qt = (lambda t: t.to(F.E4)), (lambda t: t.to(F.E4).view(T.uint8).t().contiguous().view(F.E4))
+    mm = lambda a, b: (a.float() @ b.float()).to(B16)
+    B, N, C, H = 2, 4, 16, 32
+
+    def bwd(vdt):
+        def f(dh, dxn, xs, a, gate, w, scale, rstd):
+            v = dh.float().sum(1).to(vdt)
+            return dh, dh, v, dh.float().sum((0, 1)), v, v
+        return f
+    plain = dict(
+        tcast=lambda x: (q(x), T.ones(1)),
+        tcast_t=lambda x, want_q=True: (q(x), qt(x), T.ones(1)),
+        cast_group=lambda xs, ks: [t for x in xs for t in (q(x), qt(x), T.ones(1))],
+        fp8_gemm=lambda a, sa, b, sb, bias=None, fast=True: mm(a, b.float().t()),
+        fp8_gemm_mn=lambda a, sa, b, sb, bias=None: mm(a.float().t(), b),
+        swiglu_tcast=lambda z: (q(z[:, :H]), T.ones(1)),
+        swiglu_bwd_q=lambda z, da: (q(T.cat([da, da], 1)), T.ones(1)),
+        res_mod_rmsnorm_q=lambda x, a, gate, w, sh, sc, eps, res, h: (x, x, q(x), T.ones(1), T.ones(B * N)),
+        res_mod_rmsnorm_bwd_k=bwd(T.float32), res_mod_rmsnorm_bwd16=bwd(B16))
+    monkeypatch.setattr(L, "native", lambda *a: None)
+    own = {getattr(NM, n): n for n in plain}
+    own[F.fp8_wgrad], plain["fp8_wgrad"] = "fp8_wgrad", lambda a, sa, b, sb, f32: mm(a.float().t(), b).to(T.float32 if f32 else B16)
+    own[F.bias_grad], plain["bias_grad"] = "bias_grad", lambda dy, f32: dy.float().sum(0)
+    monkeypatch.setattr(L, "call", lambda op, *a: plain[own[op]](*a) if op in own else op(*a))
+    g = T.Generator().manual_seed(1)
+    r = lambda *s: T.randint(-2, 3, s, generator=g).to(B16)
+    x, a, dy, mod = r(B, N, C), r(B, N, C), r(B, N, C), [r(B, 1, C) for _ in range(3)]
+    w, w12, w3 = r(H, C).float(), r(2 * H, C).float(), r(C, H).float()
+
+    def run():
+        ctx = SimpleNamespace(needs_input_grad=[True] * 9)
+        ctx.save_for_backward = lambda *t: setattr(ctx, "saved_tensors", t)
+        ctx.mark_non_differentiable = lambda *t: None
+        y = NM._Fp8ModRMSNormLinear.forward(ctx, x, w[0, :C], mod[0], mod[1], 1e-6, w, w[:, 0])
+        out = [y, *NM._Fp8ModRMSNormLinear.backward(ctx, r(B, N, H) * 0 + 1)]
+        out += NM._Fp8ResModRMSNormMLP.forward(ctx, x, a, mod[2], w[0, :C], mod[0], mod[1], 1e-6, w12, w3)
+        return out + list(NM._Fp8ResModRMSNormMLP.backward(ctx, dy, dy))
+    want, called = run(), []
+
+    def stand_in(*a):
+        called.append(name)
+        return plain[name](*a)
+    monkeypatch.setattr(NM, name, stand_in)
+    for got, ref in zip(run(), want):
+        assert got is ref is None or T.equal(got.to(B16), ref.to(B16))
+    # (the linear's weight is cast alone; both weights of the MLP; a dgrad or forward for each GEMM; one wgrad per weight)
+    assert len(called) == {"tcast": 2, "tcast_t": 3, "fp8_gemm": 6, "fp8_gemm_mn": 3, "res_mod_rmsnorm_bwd_k": 2}[name]
