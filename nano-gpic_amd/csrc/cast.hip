@@ -2018,10 +2018,15 @@ static bool launch_swiglu_bwd_once(const uint16_t *z, const uint16_t *da, int64_
   return true;
 }
 
-// The single-pass transposing cast when it fits (false, nothing launched, otherwise). A small part of one fp32 tile is left to
-// the two passes, which touch only what is there: [16 x 16] 5.3 us against 6.5, [48 x 64] 5.6 / 6.5, [100 x 128] 6.8 / 6.75,
-// [256 x 256] 7.4 / 7.1.
-constexpr int64_t kMinOnceT32 = 8192;   // fp32 elements
+// The single-pass transposing cast when it fits (false, nothing launched, otherwise). Small parts of fp32 tiles are left to the
+// two passes, which touch only what is there, where the single pass loads, casts and writes whole tiles: few elements, and the
+// more so the fewer of a tile's 128 rows they fill. One pass against two, us: [16 x 16] 6.9 / 5.3, [128 x 64] 6.7 / 6.5, [160 x
+// 64] 6.7 / 7.0; [64 x 256] 6.8 / 6.7, [64 x 512] 6.9 / 7.2; [32 x 256] 6.8 / 6.4, [32 x 1024] 7.2 / 7.1; [8 x 1024] 7.2 / 6.2,
+// [8 x 8192] 7.3 / 7.0, [16 x 8192] 7.2 / 7.3; [256 x 256] 7.0 / 7.5.
+constexpr int64_t kTwoPassT32 = 65536, kTwoPassRowsT32 = 1600000;   // fp32 elements; rows x elements
+static bool two_pass_t32(int64_t rows, int64_t cols) {
+  return rows * cols <= kTwoPassT32 && rows * rows * cols <= kTwoPassRowsT32;
+}
 template <typename T>
 static bool launch_tcast_t_once(const T *x, int64_t rows, int64_t cols, uint8_t *q, uint8_t *qt, int64_t ldt,
                                 float *dequant, void *ws, hipStream_t st) {
@@ -2029,7 +2034,7 @@ static bool launch_tcast_t_once(const T *x, int64_t rows, int64_t cols, uint8_t 
   const int64_t tiles = ((cols + kTT - 1) / kTT) * ((ldt + kTT - 1) / kTT);
   if (!once_enabled() || cap <= 0 || tiles <= 0 || tiles > (int64_t)(sizeof(T) == 2 ? kHybridTiles : 1) * cap)
     return false;
-  if (sizeof(T) == 4 && rows * cols < kMinOnceT32) return false;
+  if (sizeof(T) == 4 && two_pass_t32(rows, cols)) return false;
   const int grid = (int)std::min<int64_t>(tiles, cap);
   cast_t_once_kernel<T><<<grid, 256, 0, st>>>(x, cols, rows, cols, q, cols, qt, ldt, dequant, ws, once_wait_ticks());
   return true;
@@ -2218,7 +2223,8 @@ int gpic_fp8_tcast_t_group(int count, const void *const *x, int dtype, const int
     dt[i] = dtype;
     rows_ok = qt[i] != nullptr && rows[i] > 0 && cols[i] > 0;
   }
-  if (rows_ok && launch_cast_group(count, x, dt, rows, cols, q, qt, ldt, dequant, ws, (hipStream_t)stream))
+  // (one tensor: the per-tensor call, which also knows where fp32 is better off with two passes)
+  if (rows_ok && count > 1 && launch_cast_group(count, x, dt, rows, cols, q, qt, ldt, dequant, ws, (hipStream_t)stream))
     return (int)hipGetLastError();
   for (int i = 0; i < count; i++) {   // otherwise one call per tensor, in order
     const int rc = gpic_fp8_tcast_t(x[i], dtype, rows[i], cols[i], q[i], qt[i], ldt[i], dequant[i], ws, stream);

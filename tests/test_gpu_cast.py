@@ -442,11 +442,13 @@ def _device_us(f):
     return sorted(times)[4]
 
 
-@pytest.mark.parametrize("rows,cols", [(16, 16), (48, 64), (256, 256), (1024, 1024), (8192, 1024)])
+@pytest.mark.parametrize("rows,cols", [(1, 4096), (2, 1488), (8, 1024), (16, 16), (34, 352), (48, 64), (128, 64),
+                                       (256, 256), (1024, 1024), (8192, 1024)])
 def test_transposing_fp32_single_pass_only_where_it_pays(dev, rows, cols):
-    """The transposing cast of fp32 takes no longer than its two passes, which small parts of one tile are left to."""
+    """The transposing cast of fp32, alone or as a group of one, takes no longer than its two passes, which small parts of tiles
+    are left to."""
     x = torch.randn(rows, cols, device=dev)
-    once = _device_us(lambda: G.tcast_t(x))
+    once = max(_device_us(lambda: G.tcast_t(x)), _device_us(lambda: G.tcast_t_group([x])))
     L.set_single_pass(False)
     try:
         two = _device_us(lambda: G.tcast_t(x))
