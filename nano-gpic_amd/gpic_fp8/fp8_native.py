@@ -675,12 +675,25 @@ def _library_wgrad(M, N, K, f32):
     return M <= 2600 and min(N, K) >= 512 and (M >= 600 and N * K <= 1200000 if f32 else N * K <= 2200000)
 
 
+@L.step_op("gpic::fp8_wgrad16")
+def wgrad16(dy: torch.Tensor, x: torch.Tensor, f32: bool) -> torch.Tensor:
+    """bf16_wgrad(dy, x, f32), or the library's product where that is the faster one. (Chosen here, when the op runs, so that a
+    compiled graph takes the same one, whatever its sizes were when it was traced.)"""
+    if _library_wgrad(dy.shape[0], dy.shape[1], x.shape[1], f32):
+        return (dy.t() @ x).to(torch.float32 if f32 else torch.bfloat16)
+    return L.call(bf16_wgrad, dy, x, f32)
+
+
+@wgrad16.register_fake
+def _(dy, x, f32):
+    return dy.new_empty(dy.shape[1], x.shape[1], dtype=torch.float32 if f32 else torch.bfloat16)
+
+
 def _wgrad16(dy, x, dtype):
     """(dy.t() @ x).to(dtype)."""
-    if _torch_ops(dy) or (not torch.compiler.is_compiling()
-                          and _library_wgrad(dy.shape[0], dy.shape[1], x.shape[1], dtype == torch.float32)):
+    if _torch_ops(dy):
         return (dy.t() @ x).to(dtype)
-    return L.call(bf16_wgrad, dy, x, dtype == torch.float32).to(dtype)
+    return L.call(wgrad16, dy, x, dtype == torch.float32).to(dtype)
 
 
 def _mm(xq, sx, wq, sw, fast=True):

@@ -559,3 +559,13 @@ def test_stand_ins_for_the_norm_sites_ops_are_called(monkeypatch, name):
         assert got is ref is None or T.equal(got.to(B16), ref.to(B16))
     # (the linear's weight is cast alone; both weights of the MLP; a dgrad or forward for each GEMM; one wgrad per weight)
     assert len(called) == {"tcast": 2, "tcast_t": 3, "fp8_gemm": 6, "fp8_gemm_mn": 3, "res_mod_rmsnorm_bwd_k": 2}[name]
+
+
+@torch.no_grad()   # (as inside an autograd Function)
+def test_the_wgrad_is_chosen_when_a_compiled_graph_runs(monkeypatch):
+    """Under torch.compile a bf16 weight gradient of few tokens is the library's product too: the traced op chooses when it runs."""
+    monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
+    dy, x = torch.ones(600, 512, dtype=torch.bfloat16), torch.ones(600, 512, dtype=torch.bfloat16)
+    for dt in (torch.bfloat16, torch.float32):
+        dw = F._wgrad16(dy, x, dt)
+        assert dw.dtype == dt and (dw == 600).all()
