@@ -569,3 +569,21 @@ def test_the_wgrad_is_chosen_when_a_compiled_graph_runs(monkeypatch):
     for dt in (torch.bfloat16, torch.float32):
         dw = F._wgrad16(dy, x, dt)
         assert dw.dtype == dt and (dw == 600).all()
+
+
+@torch.no_grad()   # (as inside an autograd Function)
+def test_compiled_graphs_keep_the_fusable_expressions(monkeypatch):
+    """Under torch.compile the bias gradient and the dequantization are torch's expressions, for it to fuse, not opaque ops."""
+    from gpic_fp8 import _lib as L
+
+    def call(op, *a):
+        raise AssertionError(op)
+    monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
+    monkeypatch.setattr(L, "call", call)
+    g = torch.Generator().manual_seed(3)
+    dy, s = torch.randn(40, 48, generator=g).to(torch.bfloat16), torch.tensor([0.37])
+    for dt in (torch.bfloat16, torch.float32):
+        db = F._bias_grad(dy, dt)
+        assert db.dtype == dt and torch.equal(db, dy.sum(0).to(dt))
+    q = dy.to(F.E4)
+    assert torch.equal(F._dequant(q, s), (q.float() * s).to(torch.bfloat16))
