@@ -53,8 +53,9 @@ const char *gpic_fp8_status_string(int status);
 size_t gpic_fp8_cast_workspace_bytes(void);
 
 /* Tuning and test knob (process-wide; a call made on another thread at the same time sees the old or the new
- * setting; no counterpart in the reference, whose casts are always two Triton launches). gpic_fp8_tcast and gpic_fp8_tcast_t cast a bf16 or fp32 tensor
- * that fits in the chip's registers in one launch (x read once) and larger ones in two (amax pass, then cast pass).
+ * setting; no counterpart in the reference, whose casts are always two Triton launches). gpic_fp8_tcast and
+ * gpic_fp8_tcast_t cast a bf16 or fp32 tensor that fits in the chip's registers in one launch (x read once) and larger
+ * ones, and small parts of fp32 tiles of gpic_fp8_tcast_t, in two (amax pass, then cast pass).
  * enabled = 0 forces the two-pass path; wait_us bounds how long a workgroup of the single pass waits for another's
  * partial maximum before computing it from x itself (< 0: the default, 200 us; 0 makes every missing partial a direct
  * computation, which tests use to exercise that path). The results are the same bytes either way. */

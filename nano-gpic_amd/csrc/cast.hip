@@ -3,13 +3,14 @@
 //
 // Two designs, chosen per call by size:
 //  * Single pass (flat bf16 tensors of at most 100 MiB, fp32 of 48 MiB, transposing casts of 64 MiB; but for fp32 transposing
-//    casts hybrids up to 8x that; the SwiGLU casts, whose limits are stated with their kernels): ONE launch. Each workgroup holds its
-//    share of x on chip, publishes a partial maximum tagged with the call's number, folds every workgroup's partial and
+//    casts hybrids up to 8x that; the SwiGLU casts, whose limits are stated with their kernels): ONE launch. Each workgroup
+//    holds its share of x on chip, publishes a partial maximum tagged with the call's number, folds every workgroup's partial and
 //    casts from what it holds (3 B/elem moved for bf16). The call number lives in the
 //    workspace (an epoch word the last workgroup of each call advances), so the workspace carries state from call to
 //    call: it is zeroed once when created, and calls that may run at the same time (different streams) need
 //    different workspaces. Graph capture is fine: a replayed launch reads the epoch the previous call left.
-//  * Two passes (larger tensors, the SwiGLU kernels past their single passes): two stream-ordered launches,
+//  * Two passes (larger tensors, the SwiGLU kernels past their single passes, transposing casts of small parts of fp32 tiles):
+//    two stream-ordered launches,
 //      1. an amax pass: each workgroup reduces its share to one partial maximum (|x| bit patterns, NaN ignored) and
 //         writes it to partial[blockIdx.x] -- no atomics, so nothing has to be zeroed beforehand;
 //      2. a cast pass: each workgroup folds all partials (<= kMaxParts words, served from L2), derives the scale with
@@ -1141,8 +1142,8 @@ __device__ __forceinline__ uint32_t words_amax(const u32x4 (&w)[W]) {
   return m;
 }
 
-// Flat single-pass cast, run by the G workgroups [first, first + G) of a launch. x as nw 16-byte words (8 bf16 or 4 fp32 elements) plus `tail` (< 8 or < 4) elements;
-// workgroup b holds words [b P, (b + 1) P), P = 256 wpt, thread t words b P + 256 j + t, j < wpt <= kOnceWords<T>.
+// Flat single-pass cast, run by the G workgroups [first, first + G) of a launch. x as nw 16-byte words (8 bf16 or 4 fp32
+// elements) plus `tail` (< 8 or < 4) elements; workgroup b holds words [b P, (b + 1) P), P = 256 wpt, thread t words b P + 256 j + t, j < wpt <= kOnceWords<T>.
 // Hybrid (sgroups > 0, x larger than the grid holds): the 256-word groups past the held words, G P + 256 s + t, are
 // streamed by workgroup s % G twice -- for the maximum, then (last first, for MALL hits) for the cast -- so only
 // what does not fit is read twice. Map: the source word of each output word (the tail is read flat: HeadMap sources

@@ -178,8 +178,8 @@ __device__ __forceinline__ int xcd_remap(int bid, int G) {
 // flops of the e4m3 instruction in the same cycles. lda and ldb are in bytes. No scales. Against the library's bf16
 // GEMM (dy^T @ x): [32768 tokens, 6144 x 768] 288-312 us against 418-428, [32768, 768 x 3072] 144 / 300, [32768,
 // 3072 x 1024] 176 / 303, [13303, 7168 x 896] 183-190 / 200, [13303, 896 x 3584] 101 / 138, [6592, 8192 x 1024] 102 / 102;
-// the caller leaves few tokens with a small gradient to the library ([2048, 1024 x 1024] 25.2 us against 17.4). (A bf16 dgrad with this kernel, its B read
-// MN-major, was not kept: 6-20% faster on some shapes, 14-25% slower on others, with no rule on sizes between them.)
+// the caller leaves few tokens with a small gradient to the library ([2048, 1024 x 1024] 25.2 us against 17.4). (A bf16 dgrad
+// with this kernel, its B read MN-major, was not kept: 6-20% faster on some shapes, 14-25% slower on others, with no rule on sizes between them.)
 // kC32: C is fp32 and holds the bf16-rounded results: the gradient of an fp32 weight, without a separate conversion.
 template <bool kTail, bool kMN, int kBNt, int kEl = 1, bool kC32 = false, typename CT = std::conditional_t<kC32, float, uint16_t>>
 __global__ __launch_bounds__(kThreads) void gemm_tn_kernel(const uint8_t *__restrict__ A, int lda,
