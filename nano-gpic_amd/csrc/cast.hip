@@ -1967,8 +1967,9 @@ static bool launch_tcast_once(const T *x, int64_t n, uint8_t *q, float *dequant,
     return true;
   }
   const int64_t groups = std::max<int64_t>(1, (nw + 255) / 256);   // 256-word groups
-  const int grid = (int)std::min<int64_t>((groups + kFlatWords - 1) / kFlatWords, cap);
-  const int wpt = (int)((groups + grid - 1) / grid);
+  const int64_t most = std::min<int64_t>((groups + kFlatWords - 1) / kFlatWords, cap);
+  const int wpt = (int)((groups + most - 1) / most);
+  const int grid = (int)((groups + wpt - 1) / wpt);   // (no workgroup without words: it would poll while the others read)
   cast_once_kernel<T, Map><<<grid, 256, 0, st>>>(x, n, wpt, 0, q, dequant, ws, once_wait_ticks(), map);
   return true;
 }
@@ -2075,6 +2076,7 @@ static bool launch_cast_group(int count, const void *const *x, const int *dtype,
         const int64_t groups = std::max<int64_t>(1, (rows[i] * cols[i] / (f32 ? 4 : 8) + 255) / 256);   // of 256 words
         wgs = (groups + words - 1) / words;
         wpt = (int)((groups + wgs - 1) / wgs);
+        wgs = (groups + wpt - 1) / wpt;
       }
       total += wgs;
       if (total > cap) break;

@@ -455,3 +455,25 @@ def test_transposing_fp32_single_pass_only_where_it_pays(dev, rows, cols):
     finally:
         L.set_single_pass(True, -1)
     assert once < 1.08 * two
+
+
+@pytest.mark.parametrize("n,full,dt", [(21500000, 23000000, torch.bfloat16), (10500000, 11500000, torch.float32)])
+def test_flat_single_pass_leaves_no_workgroup_idle(dev, n, full, dt):
+    """A flat tensor that does not fill every workgroup's last words is cast by as many workgroups as hold some: no slower than a
+    larger one that fills them (7%: a full turn of words more or less), and to the two passes' bytes."""
+    def us(n):
+        xs, k = [torch.randn(n, device=dev).to(dt) for _ in range(3)], [0]
+
+        def f():
+            k[0] += 1
+            return G.tcast(xs[k[0] % 3])
+        return xs[0], min(_device_us(f) for _ in range(3))
+    x, t = us(n)
+    q, s = G.tcast(x)
+    L.set_single_pass(False)
+    try:
+        q2, s2 = G.tcast(x)
+    finally:
+        L.set_single_pass(True, -1)
+    assert torch.equal(q.view(torch.uint8), q2.view(torch.uint8)) and torch.equal(s, s2)
+    assert t < 1.07 * us(full)[1]
