@@ -35,6 +35,7 @@
 //  * Split-K (for the small-output wgrad shapes): each split writes fp32 partials; a second kernel sums them in
 //    split order (deterministic) and applies scale, bias and the bf16 rounding.
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 #include "gpic_device.h"
@@ -863,21 +864,34 @@ static Plan plan_gemm(int64_t M, int64_t N, int64_t K) {
   return ktiles > 0 && tbest[1] < kNarrowGain * tbest[0] ? best[1] : best[0];
 }
 
-// plan_gemm through the plans of each thread's last shapes (at most 2^kPlanBits of them): the search, up to 128 candidates,
-// takes 0.5 us of host time for a long K, and a call wants it twice, for the workspace's size and for the launch.
+// plan_gemm through the plans of the last shapes (at most 2^kPlanBits of them): the search, up to 128 candidates, takes 0.5 us of
+// host time for a long K, and a call wants it twice, for the workspace's size and for the launch. One table for all threads, an
+// entry held by one of them at a time (another searches for itself meanwhile), and not one a thread: while a thread has not
+// touched the thread-local storage of the last library loaded, glibc's lookups take the slow way in all of its others, torch's
+// among them (a tcast's host time 15.5 us against 13.9).
 constexpr int kPlanBits = 6;
 static Plan plan_of(int64_t M, int64_t N, int64_t K) {
   struct Entry {
+    std::atomic<bool> held;
     int64_t M, N, K;
     int cus;   // (0: empty)
     Plan p;
   };
-  static thread_local Entry plans[1 << kPlanBits];
+  static Entry plans[1 << kPlanBits];
   const int cus = num_cus();
   constexpr uint64_t kMul = 0x9E3779B97F4A7C15u;   // (2^64 over the golden ratio: spreads a product over its top bits)
   Entry &e = plans[((((uint64_t)M * kMul + (uint64_t)N) * kMul + (uint64_t)K) * kMul) >> (64 - kPlanBits)];
-  if (e.M != M || e.N != N || e.K != K || e.cus != cus) e = Entry{M, N, K, cus, plan_gemm(M, N, K)};
-  return e.p;
+  if (e.held.exchange(true, std::memory_order_acquire)) return plan_gemm(M, N, K);
+  if (e.M != M || e.N != N || e.K != K || e.cus != cus) {
+    e.p = plan_gemm(M, N, K);
+    e.M = M;
+    e.N = N;
+    e.K = K;
+    e.cus = cus;
+  }
+  const Plan p = e.p;
+  e.held.store(false, std::memory_order_release);
+  return p;
 }
 
 template <int kSM, int kSN, int kSS>
