@@ -31,9 +31,7 @@ def _host_command(out):
     import torch
     from torch.utils import cpp_extension
     inc = [f for p in cpp_extension.include_paths() + [sysconfig.get_paths()["include"]] for f in ("-isystem", p)]
-    # (NDEBUG: pybind11's debug counter is thread-local, which slows torch's own thread-local lookups)
-    return [CXX, "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-Wall",
-            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+    return [CXX, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
             *inc, "-o", out, os.path.join(CSRC, "host.cpp"), *[f"-L{p}" for p in cpp_extension.library_paths()],
             "-lc10", "-ltorch_cpu", "-ltorch_python", f"-L{HERE}", "-l:libgpic_fp8.so", "-Wl,-rpath,$ORIGIN"]
 
